@@ -104,7 +104,7 @@ int tdhf_rk4_step(tdhf_ctx* ctx, double* u, double Aave, double A);
  * A(it-1) = 2*Aave - A, Aave, Aave, A; the four stage launches are enqueued on
  * stream (a hipStream_t; NULL = the context's stream) and the call returns
  * without waiting.  The stage buffers live in a fixed device array of the
- * library (6 MiB per GPU, held until the process ends): NG*NB*NK must not
+ * library (16 MiB per GPU, held until the process ends): NG*NB*NK must not
  * exceed 131072 (TDHF_EINVAL otherwise).  The call allocates nothing; the
  * context (tables) must have been created before.  All calls on one GPU share
  * that array, so calls whose launches overlap on one GPU (other streams,
@@ -248,6 +248,12 @@ int tdhf_bwd(tdhf_ctx* ctx, double* dLdA, double* dLdu0);
  * partial sums outside the budget, ntraj * NK*NB * ceil(NK*NB/32) * NG * 16
  * bytes (2.1 GB for 32 trajectories at NK = 128, NB = 8); without that
  * memory it evaluates them row-wise (the same results to rounding).
+ * Where the exchange runs through the density matrices of the k-points (large
+ * cells or many trajectories; NK <= 128), their matrices are allocated outside
+ * the budget too, 32 * NG * (NG+1) * N bytes per trajectory with N = NK rounded
+ * up to 16, 32, 64 or 128, and the states are held with NK padded to N; if the
+ * padded states exceed a given budget, or without that memory, the run is
+ * row-wise (the same results to rounding).
  *   u      : ntraj states concatenated (NG*NB*NK complex each), in: initial,
  *            out: final
  *   A      : ntraj*nt, trajectory t at A + nt*t
@@ -303,9 +309,10 @@ int tdhf_batch_propagate(tdhf_batch* b, int nt, const double* A, const double* A
 int tdhf_batch_run(const tdhf_params* p, int ntraj, const int* nk, const double* vion,
                    double* u, int nt, const double* A, const double* Aave, double* etot,
                    double* nele, double* jtot, double* init3);
-/* Launch shape: waves per workgroup of the fused kernel, or with pair tiles of
- * the per-row epilogue launch (1, 2, 4 or 8, at least NG/64; default the
- * smallest).
+/* Launch shape: waves per workgroup of the fused kernel, with pair tiles of
+ * the per-row epilogue launch, with density matrices of their product with the
+ * orbitals (1, 2, 4 or 8, at least NG/64; default the smallest, with density
+ * matrices 4 or 8).
  * tdhf_batch_autotune times nt_trial steps for each candidate on a copy of the
  * state (the batch state is unchanged), keeps the fastest and remembers it for
  * batches of the same shape created later in the process; best_nw receives
@@ -317,22 +324,27 @@ int tdhf_batch_autotune(tdhf_batch* b, int nt_trial, const double* A, const doub
 /* Row schedule of the batched launch (which workgroup runs which trajectory's
  * row, and so on which XCD): 0 = trajectories bin-packed over the XCDs (a
  * trajectory's rows on one XCD, contiguous; the default), 1 = the same with
- * the rows of an XCD's trajectories interleaved, 2 = no XCD pinning.  The
+ * the rows of an XCD's trajectories interleaved, 2 = no XCD pinning (the
+ * default for fewer than 8 trajectories with density matrices).  The
  * results do not depend on it.  tdhf_batch_autotune times every (exchange
  * evaluation, schedule, waves per workgroup) combination and keeps the
  * fastest. */
 int tdhf_batch_set_schedule(tdhf_batch* b, int sched);
 int tdhf_batch_get_schedule(const tdhf_batch* b);
-/* Exchange evaluation of the batched stages: 0 = row-wise (every ordered pair
- * of rows (k,i), (q,j) transformed by the fused kernel of row (k,i), as
- * ubkwbk_vFwbk, src/Functions.f90:247-257), 1, 2, 3 = pair tiles of 64, 32
+/* Exchange evaluation of the batched stages: 0 = direct: row-wise (every
+ * ordered pair of rows (k,i), (q,j) transformed by the fused kernel of row
+ * (k,i), as ubkwbk_vFwbk, src/Functions.f90:247-257) or, where the batch is
+ * large enough for it to be faster, through the density matrices of the
+ * k-points, 1, 2, 3 = pair tiles of 64, 32
  * or 16 rows: since the stage acts on its own state, the convolutions of
  * (k,i),(q,j) and (q,j),(k,i) are conjugates up to the Nyquist component, so
  * one transform pair per unordered pair feeds both rows (needs NG = 64,
  * NB == NBocc and fewer than 2^22 rows per trajectory; TDHF_EINVAL
  * otherwise); a second launch per stage adds each row's partial sums and
  * applies the rest of H and the stage update.  Smaller tiles make more
- * workgroups and more partial sums per row.  Results agree to rounding.  tdhf_batch_autotune includes all four. */
+ * workgroups and more partial sums per row.  Results agree to rounding.
+ * tdhf_batch_autotune includes all four, or mode 0 only where that runs through
+ * the density matrices. */
 int tdhf_batch_set_exchange(tdhf_batch* b, int mode);
 int tdhf_batch_get_exchange(const tdhf_batch* b);
 int tdhf_batch_set_kernel_timing(tdhf_batch* b, int enable);

@@ -27,6 +27,8 @@
 #include "tdhf_adjoint.h"
 #include "tdhf_adjtile.h"
 #include "tdhf_post.h"
+#include "tdhf_kspace.h"
+#include "tdhf_kadjoint.h"
 
 using tdhf::zd;
 
@@ -34,15 +36,17 @@ namespace {
 
 thread_local std::string g_err = "no error";
 
-// Stage buffers of the allocation-free RK4 step (tdhf_rk4_step_noalloc):
-// ksum | sa | sb, each of at most kNoAllocMaxState complex elements
-// (NG*NB*NK <= 131072, e.g. NG=128, NB=8, NK=128), 6 MiB in all.  A
+// Buffers of the allocation-free RK4 step (tdhf_rk4_step_noalloc):
+// ksum | sa | sb | u0, each of at most kNoAllocSlot complex elements, 16 MiB
+// in all: states of NG*NB*NK <= kNoAllocMaxState = 131072 (e.g. NG=128, NB=8,
+// NK=128), twice that with the k-points padded (tdhf_kspace.h).  A
 // file-scope device array: every GPU the library runs on holds its own copy
 // until the process ends.  Host code never names the array in a kernel
 // argument or a copy; it uses the device address taken with
 // hipGetSymbolAddress for each device (noalloc_scratch).
 constexpr size_t kNoAllocMaxState = (size_t)1 << 17;
-__device__ __align__(256) double scratch[6 * kNoAllocMaxState];
+constexpr size_t kNoAllocSlot = 2 * kNoAllocMaxState;
+__device__ __align__(256) double scratch[8 * kNoAllocSlot];
 
 std::mutex g_scratch_mu;
 std::vector<double*> g_scratch_ptr;  // per device id
@@ -65,7 +69,14 @@ struct tdhf_ctx {
   double* d_kc = nullptr;  // circulant kernels K_H, K_2, K_1 of the apply kernel
   double* d_vhg = nullptr; // vCG/NG in the transforms' G layout (pair-tile epilogue)
   zd* d_tw = nullptr;
-  // orbital buffers (NG*NB*NK complex each)
+  // density-matrix path (tdhf_kspace.h): used by this context, k transform
+  // length, spectra, twiddles, twist factors; u0_padded: d_u0 is in its layout
+  bool kpath = false, u0_padded = false;
+  int kn = 0;
+  zd *d_ktab = nullptr, *d_ktw = nullptr, *d_om = nullptr;
+  zd* d_hm = nullptr;      // matrices of a stage
+  double* d_nx = nullptr;  // density and partial observables of a stage
+  // orbital buffers (NG*NB*NK complex each, NK padded to kn with kpath)
   zd *d_u0 = nullptr, *d_ksum = nullptr, *d_sa = nullptr, *d_sb = nullptr;
   zd *d_w = nullptr, *d_out = nullptr;
   // observables
@@ -337,7 +348,8 @@ tdhf::ApplyArgs base_args(const tdhf_ctx* c) {
 int ensure_obs(tdhf_ctx* c, long slots) {
   if (slots > c->obs_slots) {
     dfree(c->d_obs);
-    CHKRET(dalloc(c, &c->d_obs, (size_t)slots * c->obs_stride));
+    const int stride = std::max(c->obs_stride, tdhf::kspace_obs_stride(c->ng));
+    CHKRET(dalloc(c, &c->d_obs, (size_t)slots * stride));
     c->obs_slots = slots;
   }
   if (slots > c->res_slots) {
@@ -373,9 +385,10 @@ void destroy_graph(tdhf_ctx* c) {
   c->graphs_ready = false;
 }
 
+int launch_stage(tdhf_ctx* c, const tdhf::ApplyArgs& a);
+
 // Enqueues steps [*d_step + j0, *d_step + j0 + n) of the RK4 loop.
 int enqueue_steps(tdhf_ctx* c, int j0, int n) {
-  const int rows = c->nb * c->nk;
   tdhf::ApplyArgs a = base_args(c);
   a.Aarr = c->d_A;
   a.Aavearr = c->d_Aave;
@@ -389,19 +402,19 @@ int enqueue_steps(tdhf_ctx* c, int j0, int n) {
     a.mode = tdhf::M_S1;
     a.u = a.w = c->d_u0;
     a.unext = c->d_sa;
-    CHKRET(launch_apply(c, a, rows));
+    CHKRET(launch_stage(c, a));
     a.mode = tdhf::M_S2;
     a.u = a.w = c->d_sa;
     a.unext = c->d_sb;
-    CHKRET(launch_apply(c, a, rows));
+    CHKRET(launch_stage(c, a));
     a.mode = tdhf::M_S3;
     a.u = a.w = c->d_sb;
     a.unext = c->d_sa;
-    CHKRET(launch_apply(c, a, rows));
+    CHKRET(launch_stage(c, a));
     a.mode = tdhf::M_S4;
     a.u = a.w = c->d_sa;
     a.unext = nullptr;
-    CHKRET(launch_apply(c, a, rows));
+    CHKRET(launch_stage(c, a));
   }
   return 0;
 }
@@ -656,6 +669,7 @@ void release(tdhf_ctx* c) {
   dfree(c->d_vq); dfree(c->d_vtl); dfree(c->d_tw); dfree(c->d_kc); dfree(c->d_vhg);
   dfree(c->d_u0); dfree(c->d_ksum); dfree(c->d_sa); dfree(c->d_sb);
   dfree(c->d_w); dfree(c->d_out);
+  dfree(c->d_ktab); dfree(c->d_ktw); dfree(c->d_om); dfree(c->d_hm); dfree(c->d_nx);
   dfree(c->d_obs); dfree(c->d_res); dfree(c->d_A); dfree(c->d_Aave); dfree(c->d_step);
   tdhf::gs_free(c->gs);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -685,6 +699,7 @@ int ctx_fail(tdhf_ctx* c, int code, const char* msg) { return fail(c, code, "%s"
 
 }  // namespace tdhf
 
+#include "tdhf_kspace_impl.h"
 #include "tdhf_gs_impl.h"
 #include "tdhf_adjoint_impl.h"
 
@@ -735,20 +750,26 @@ int tdhf_create(const tdhf_params* p, const double* vion, const double* vcg, con
     fail(c, TDHF_EDEVICE, "hipStreamCreate failed");
     return bail(TDHF_EDEVICE);
   }
-  const size_t n = nstate(c);
-  if ((rc = dalloc(c, &c->d_kx, c->nk)) || (rc = dalloc(c, &c->d_vion, c->ng)) ||
+  c->kn = tdhf::kspace_len(c->nk);
+  c->kpath = kspace_pays(c->ng, c->nk, c->nb, c->nbocc, 1);
+  const size_t n = path_count(c);
+  // kx with zeros up to the padded number of k-points
+  std::vector<double> kxp(std::max(c->nk, c->kn), 0.0);
+  std::copy(c->kx.begin(), c->kx.end(), kxp.begin());
+  if ((rc = dalloc(c, &c->d_kx, kxp.size())) || (rc = dalloc(c, &c->d_vion, c->ng)) ||
       (rc = dalloc(c, &c->d_u0, n)) || (rc = dalloc(c, &c->d_ksum, n)) ||
       (rc = dalloc(c, &c->d_sa, n)) || (rc = dalloc(c, &c->d_sb, n)) ||
       (rc = dalloc(c, &c->d_w, n)) || (rc = dalloc(c, &c->d_out, n)) ||
       (rc = dalloc(c, &c->d_step, 1)))
     return bail(rc);
-  if (hipMemcpy(c->d_kx, c->kx.data(), c->nk * sizeof(double), hipMemcpyHostToDevice) !=
+  if (hipMemcpy(c->d_kx, kxp.data(), kxp.size() * sizeof(double), hipMemcpyHostToDevice) !=
           hipSuccess ||
       hipMemcpy(c->d_vion, vion, c->ng * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
     fail(c, TDHF_EDEVICE, "table upload failed");
     return bail(TDHF_EDEVICE);
   }
   if ((rc = build_tables(c, vcg, vcgkk))) return bail(rc);
+  if (c->kn && (rc = kspace_tables(c))) return bail(rc);
   {
     const hipError_t e = set_apply_lds_limit(c->ng);
     if (e != hipSuccess && c->lds > 64 * 1024) {
@@ -813,10 +834,10 @@ int tdhf_get_tables(tdhf_ctx* c, double* vcg, double* vq) {
 int tdhf_hpsi(tdhf_ctx* c, const double* u, const double* w, double A, double* hw) {
   if (!c) return fail(nullptr, TDHF_EINVAL, "ctx is NULL");
   if (!u || !w || !hw) return fail(c, TDHF_EINVAL, "NULL array");
-  CHKRET(upload(c, c->d_sa, u));
-  CHKRET(upload(c, c->d_w, w));
-  CHKRET(tdhf::ctx_apply(c, c->d_sa, c->d_w, c->nb, A, c->d_out));
-  CHKRET(download(c, hw, c->d_out));
+  CHKRET(upload_state(c, c->d_sa, u));
+  CHKRET(upload_state(c, c->d_w, w));
+  CHKRET(path_hpsi(c, c->d_sa, c->d_w, A, c->d_out));
+  CHKRET(download_state(c, hw, c->d_out));
   return sync(c);
 }
 
@@ -824,9 +845,9 @@ int tdhf_observables(tdhf_ctx* c, const double* u, double A, double* etot, doubl
                      double* nele, double* je) {
   if (!c) return fail(nullptr, TDHF_EINVAL, "ctx is NULL");
   if (!u) return fail(c, TDHF_EINVAL, "NULL array");
-  CHKRET(upload(c, c->d_sa, u));
+  CHKRET(upload_state(c, c->d_sa, u));
   double r[7];
-  CHKRET(observables_of(c, c->d_sa, A, r));
+  CHKRET(path_observables_of(c, c->d_sa, A, r));
   if (etot) *etot = r[0];
   if (nele) *nele = r[1];
   if (je) *je = r[2];
@@ -841,13 +862,14 @@ int tdhf_observables(tdhf_ctx* c, const double* u, double A, double* etot, doubl
 
 int tdhf_state_upload(tdhf_ctx* c, const double* u) {
   if (!c || !u) return fail(c, TDHF_EINVAL, "NULL argument");
-  CHKRET(upload(c, c->d_u0, u));
+  CHKRET(upload_state(c, c->d_u0, u));
+  c->u0_padded = c->kpath;
   return sync(c);
 }
 
 int tdhf_state_download(tdhf_ctx* c, double* u) {
   if (!c || !u) return fail(c, TDHF_EINVAL, "NULL argument");
-  return download(c, u, c->d_u0);
+  return c->u0_padded ? download_state(c, u, c->d_u0) : download(c, u, c->d_u0);
 }
 
 int tdhf_rt_begin(tdhf_ctx* c, int nt, const double* A, const double* Aave) {
@@ -863,6 +885,7 @@ int tdhf_rt_begin(tdhf_ctx* c, int nt, const double* A, const double* Aave) {
   }
   const int zero = 0;
   HIPCHK(c, hipMemcpyAsync(c->d_step, &zero, sizeof zero, hipMemcpyHostToDevice, c->stream));
+  CHKRET(resident_to_path(c));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->rt_open = true;
   c->rt_nt = nt;
@@ -876,6 +899,7 @@ int tdhf_rt_advance(tdhf_ctx* c, int n) {
   if (n < 0 || c->rt_done + n > c->rt_nt)
     return fail(c, TDHF_EINVAL, "advance by %d steps: %ld of %ld steps done", n, c->rt_done,
                 c->rt_nt);
+  CHKRET(resident_to_path(c));
   CHKRET(run_steps(c, n));
   CHKRET(sync(c));
   c->rt_done += n;
@@ -887,9 +911,10 @@ int tdhf_rt_end(tdhf_ctx* c, double* etot, double* nele, double* jtot, double* i
   if (!c->rt_open) return fail(c, TDHF_EINVAL, "tdhf_rt_end without tdhf_rt_begin");
   c->rt_open = false;
   const long done = c->rt_done;
+  CHKRET(resident_to_path(c));
   if (done == 0) {
     double r[7];
-    CHKRET(observables_of(c, c->d_u0, 0.0, r));
+    CHKRET(path_observables_of(c, c->d_u0, 0.0, r));
     if (init3) { init3[0] = r[0]; init3[1] = r[1]; init3[2] = r[2]; }
     return 0;
   }
@@ -904,11 +929,16 @@ int tdhf_rt_end(tdhf_ctx* c, double* etot, double* nele, double* jtot, double* i
   a.step_base = c->d_step;
   a.jstep = -1;
   a.obs = c->d_obs;
-  CHKRET(launch_apply(c, a, rows));
+  CHKRET(launch_stage(c, a));
   const long ns = done + 1;
-  hipLaunchKernelGGL(tdhf::obs_reduce_kernel, dim3((unsigned)((ns + 63) / 64)), dim3(64), 0,
-                     c->stream, c->d_obs, c->obs_stride, rows, (int)ns, c->dv, c->vcell, c->d_res);
-  HIPCHK(c, hipGetLastError());
+  if (c->kpath) {
+    CHKRET(launch_obs_reduce(c, c->d_obs, ns, 1, 0, c->d_res));
+  } else {
+    hipLaunchKernelGGL(tdhf::obs_reduce_kernel, dim3((unsigned)((ns + 63) / 64)), dim3(64), 0,
+                       c->stream, c->d_obs, c->obs_stride, rows, (int)ns, c->dv, c->vcell,
+                       c->d_res);
+    HIPCHK(c, hipGetLastError());
+  }
   std::vector<double> res((size_t)7 * ns);
   HIPCHK(c, hipMemcpyAsync(res.data(), c->d_res, res.size() * sizeof(double),
                            hipMemcpyDeviceToHost, c->stream));
@@ -967,10 +997,17 @@ int tdhf_rk4_step_noalloc(tdhf_ctx* c, double* u, double Aave, double A, void* s
   double* sc = noalloc_scratch(c);
   if (!sc) return fail(c, TDHF_EDEVICE, "step scratch not set up on device %d", c->device);
   zd* ksum = reinterpret_cast<zd*>(sc);
-  zd* sa = ksum + kNoAllocMaxState;
-  zd* sb = sa + kNoAllocMaxState;
+  zd* sa = ksum + kNoAllocSlot;
+  zd* sb = sa + kNoAllocSlot;
   zd* u0 = reinterpret_cast<zd*>(u);
   hipStream_t st = stream ? static_cast<hipStream_t>(stream) : c->stream;
+  // padded k-points: the step runs on a copy in that layout (row-wise if the
+  // padding does not fit the array)
+  const bool kp = c->kpath && kcount(c) <= kNoAllocSlot;
+  if (kp) {
+    u0 = sb + kNoAllocSlot;
+    CHKRET(kspace_layout(c, reinterpret_cast<zd*>(u), u0, true, 1, st));
+  }
   // the four stages of RT_RK4_ubk with the fields as kernel arguments
   // (no step counter, no field arrays, no observables)
   tdhf::ApplyArgs a = base_args(c);
@@ -986,6 +1023,10 @@ int tdhf_rk4_step_noalloc(tdhf_ctx* c, double* u, double Aave, double A, void* s
     a.A = a.Aobs = fields[s];
     a.u = a.w = ins[s];
     a.unext = nexts[s];
+    if (kp) {
+      CHKRET(launch_kspace(c, a, 1, st));
+      continue;
+    }
     switch (c->ng) {
       case 16: launch_apply_t<16>(a, rows, 1, c->nw, c->lds, st); break;
       case 32: launch_apply_t<32>(a, rows, 1, c->nw, c->lds, st); break;
@@ -994,6 +1035,7 @@ int tdhf_rk4_step_noalloc(tdhf_ctx* c, double* u, double Aave, double A, void* s
     }
     HIPCHK(c, hipGetLastError());
   }
+  if (kp) CHKRET(kspace_layout(c, u0, reinterpret_cast<zd*>(u), false, 1, st));
   return 0;
 }
 

@@ -47,6 +47,11 @@ struct AdjState {
   int4* tiles = nullptr;
   double* zrow = nullptr;
   int ntiles = 0, nblk = 0;
+  // density-matrix path (tdhf_kspace.h, tdhf_kadjoint.h): states padded, the
+  // two matrices and the density scratch of every trajectory
+  bool kp = false;
+  zd* hm = nullptr;
+  double* nx = nullptr;
   // captured step blocks, keyed by the buffers they use
   std::vector<std::pair<std::vector<const void*>, hipGraphExec_t>> graphs;
 };
@@ -91,6 +96,8 @@ void adj_free(AdjState& s) {
   dfree(s.dpart);
   dfree(s.tiles);
   dfree(s.zrow);
+  dfree(s.hm);
+  dfree(s.nx);
   for (auto& g : s.graphs) (void)hipGraphExecDestroy(g.second);
   s = AdjState();
 }
@@ -297,6 +304,64 @@ int adj_tiles_setup(tdhf_ctx* c, AdjState& s) {
   return 0;
 }
 
+// Elements of one trajectory's state in the record's layout.
+size_t adj_count(const tdhf_ctx* c, const AdjState& s) { return s.kp ? kcount(c) : nstate(c); }
+// Per-row (row-wise) or per-point field derivatives of a stage.
+int adj_nabar(const tdhf_ctx* c, const AdjState& s) { return s.kp ? c->ng : c->nb * c->nk; }
+
+KScratch adj_scratch(const tdhf_ctx* c, const AdjState& s) {
+  const int gpw = kspace_gpw(c->kn);
+  return {s.hm, s.nx, 2 * tdhf::kmat_elems(c->ng, c->kn),
+          std::max(tdhf::kmat_extra(c->ng, gpw), tdhf::kadj_extra(c->ng, gpw))};
+}
+
+int adj_obs_stride(const tdhf_ctx* c, const AdjState& s) {
+  return s.kp ? tdhf::kspace_obs_stride(c->ng) : c->obs_stride;
+}
+
+// One forward stage of the record's trajectories.
+int adj_stage(tdhf_ctx* c, const AdjState& s, const tdhf::ApplyArgs& a) {
+  if (!s.kp) return launch_apply(c, a, c->nb * c->nk, s.ntraj);
+  const KScratch k = adj_scratch(c, s);
+  return launch_kspace(c, a, s.ntraj, nullptr, &k);
+}
+
+// One reverse stage (or the start, A_EGRAD) through the density matrices.
+int launch_kadj(tdhf_ctx* c, const AdjState& s, const tdhf::AdjArgs& a) {
+  const KScratch sc = adj_scratch(c, s);
+  tdhf::KAdjArgs k{};
+  k.a = a;
+  k.ng = c->ng;
+  k.n = c->kn;
+  k.nchunk = kspace_chunks(c->nb);
+  k.ktab = c->d_ktab;
+  k.tw = c->d_ktw;
+  k.om = c->d_om;
+  k.hm = sc.hm;
+  k.qoff = sc.hstride / 2;
+  k.hstride = sc.hstride;
+  k.nx = sc.nx;
+  k.nstride = sc.nstride;
+  k.J = s.objective == TDHF_OBJ_JSQ ? s.dJ : nullptr;
+  k.vcell = c->vcell;
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  if (c->timing) {
+    CHKRET(take_events(c, &e0, &e1));
+    HIPCHK(c, hipEventRecord(e0, c->stream));
+  }
+  void* args[] = {&k};
+  const int wa = kmat_waves(2L * tdhf::kmat_tasks(c->ng, kspace_gpw(c->kn)) * s.ntraj);
+  HIPCHK(c, hipLaunchKernel(kadj_mat_fn(c->kn), dim3(kmat_groups(c->kn, c->ng, wa), s.ntraj, 2),
+                            dim3(64 * wa), args, kmat_lds_for(c->kn, wa, c->ng), c->stream));
+  const int wb = kapply_waves(c->kn, c->ng), nbt = kspace_nbt(c->nb);
+  const int xt = kapply_points((long)kapply_groups(c->kn, c->ng, c->nb, 1) * s.ntraj);
+  HIPCHK(c, hipLaunchKernel(kadj_apply_fn(nbt, xt),
+                            dim3(kapply_groups(c->kn, c->ng, c->nb, xt), s.ntraj), dim3(64 * wb),
+                            args, tdhf::kadj_apply_lds(wb, nbt, xt, c->ng), c->stream));
+  if (c->timing) HIPCHK(c, hipEventRecord(e1, c->stream));
+  return 0;
+}
+
 int launch_jgrad(tdhf_ctx* c, const AdjState& s, int step, const zd* y, zd* ua, zd* gb,
                  int init, int jstep = -1) {
   tdhf::JgradArgs j{};
@@ -315,7 +380,7 @@ int launch_jgrad(tdhf_ctx* c, const AdjState& s, int step, const zd* y, zd* ua, 
   j.ua = ua;
   j.gb = gb;
   j.init = init;
-  j.tstride = nstate(c);
+  j.tstride = adj_count(c, s);
   j.fstride = s.nt;
   if (jstep >= 0) {  // step and state from the device counter and the tape
     j.step_base = c->d_step;
@@ -323,6 +388,12 @@ int launch_jgrad(tdhf_ctx* c, const AdjState& s, int step, const zd* y, zd* ua, 
     j.tape = s.tape;
     j.tape_seg = s.seg;
     j.blk = (size_t)s.ntraj * nstate(c);
+  }
+  if (s.kp) {  // the start; the steps' terms are part of launch_kadj's stage 1
+    hipLaunchKernelGGL(tdhf::kadj_jinit_kernel, dim3(c->ng, s.ntraj), dim3(256), 0, c->stream, j,
+                       c->ng, c->kn);
+    HIPCHK(c, hipGetLastError());
+    return 0;
   }
   const dim3 grid(c->nb * c->nk, s.ntraj);
   switch (c->ng) {
@@ -351,7 +422,7 @@ tdhf::AdjArgs adj_base(const tdhf_ctx* c, const AdjState& s) {
   a.tw = c->d_tw;
   a.Aarr = s.dA;
   a.Aavearr = s.dAave;
-  a.tstride = nstate(c);
+  a.tstride = adj_count(c, s);
   a.fstride = s.nt;
   return a;
 }
@@ -361,8 +432,7 @@ tdhf::AdjArgs adj_base(const tdhf_ctx* c, const AdjState& s) {
 // tape == nullptr, untaped.  Observables of step it go to slot it.  Blocks of
 // kAdjGraphSteps steps are replayed from a captured graph.
 int adj_forward_steps(tdhf_ctx* c, AdjState& s, int s0, int n, zd* tape) {
-  const int rows = c->nb * c->nk;
-  const size_t ns = nstate(c), blk = (size_t)s.ntraj * ns;
+  const size_t ns = adj_count(c, s), blk = (size_t)s.ntraj * ns;
   zd *u0 = s.st, *ks = s.st + blk, *sa = s.st + 2 * blk, *sb = s.st + 3 * blk;
   tdhf::ApplyArgs a = base_args(c);
   a.Aarr = s.dA;
@@ -376,18 +446,18 @@ int adj_forward_steps(tdhf_ctx* c, AdjState& s, int s0, int n, zd* tape) {
   a.nstate = blk;
   a.tstride = ns;
   a.fstride = s.nt;
-  a.ostride = (size_t)(s.nt + 1) * c->obs_stride;
+  a.ostride = (size_t)(s.nt + 1) * adj_obs_stride(c, s);
   auto enq = [&](int m) -> int {
     for (int j = 0; j < m; ++j) {
       a.jstep = j;
       a.mode = tdhf::M_S1; a.u = a.w = u0; a.unext = sa;
-      CHKRET(launch_apply(c, a, rows, s.ntraj));
+      CHKRET(adj_stage(c, s, a));
       a.mode = tdhf::M_S2; a.u = a.w = sa; a.unext = sb;
-      CHKRET(launch_apply(c, a, rows, s.ntraj));
+      CHKRET(adj_stage(c, s, a));
       a.mode = tdhf::M_S3; a.u = a.w = sb; a.unext = sa;
-      CHKRET(launch_apply(c, a, rows, s.ntraj));
+      CHKRET(adj_stage(c, s, a));
       a.mode = tdhf::M_S4; a.u = a.w = sa; a.unext = nullptr;
-      CHKRET(launch_apply(c, a, rows, s.ntraj));
+      CHKRET(adj_stage(c, s, a));
     }
     hipLaunchKernelGGL(tdhf::step_advance_kernel, dim3(1), dim3(1), 0, c->stream, c->d_step, m);
     HIPCHK(c, hipGetLastError());
@@ -414,8 +484,8 @@ int adj_forward_steps(tdhf_ctx* c, AdjState& s, int s0, int n, zd* tape) {
 // replayed from a captured graph (their buffer rotation returns to the start).
 int adj_backward_steps(tdhf_ctx* c, AdjState& s, int s0, int n, zd** ub, zd** ua, zd** ga,
                        zd** gb) {
-  const size_t ns = nstate(c), blk = (size_t)s.ntraj * ns;
-  const int rows = c->nb * c->nk;
+  const size_t ns = adj_count(c, s), blk = (size_t)s.ntraj * ns;
+  const int rows = adj_nabar(c, s);
   tdhf::AdjArgs a = adj_base(c, s);
   a.abar_tstride = (size_t)s.seg * 4 * rows;
   a.step_base = c->d_step;
@@ -433,11 +503,12 @@ int adj_backward_steps(tdhf_ctx* c, AdjState& s, int s0, int n, zd** ub, zd** ua
         a.mode = st;
         a.gb = *pga;
         a.gout = *pgb;
-        CHKRET(launch_adj(c, a, s.ntraj, &s));
+        CHKRET(s.kp ? launch_kadj(c, s, a) : launch_adj(c, a, s.ntraj, &s));
         std::swap(*pga, *pgb);
       }
       // current-squared objective: J after step it-1 is evaluated on y1 of step it
-      if (s.objective == TDHF_OBJ_JSQ) CHKRET(launch_jgrad(c, s, 0, nullptr, *pua, *pga, 0, j));
+      if (s.objective == TDHF_OBJ_JSQ && !s.kp)
+        CHKRET(launch_jgrad(c, s, 0, nullptr, *pua, *pga, 0, j));
       std::swap(*pub, *pua);  // the accumulated cotangent becomes ubar of the step before
     }
     hipLaunchKernelGGL(tdhf::step_advance_kernel, dim3(1), dim3(1), 0, c->stream, c->d_step, -m);
@@ -508,21 +579,20 @@ extern "C" int tdhf_fwd_batch(tdhf_ctx* c, int ntraj, double* u, int nt, const d
       const double* At = A + (size_t)t * nt;
       s.Aave[(size_t)t * nt + it] = 0.5 * (At[it] + (it > 0 ? At[it - 1] : 0.0));
     }
-  const size_t ns = nstate(c), blk = (size_t)ntraj * ns, bb = blk * sizeof(zd);
-  const int rows = c->nb * c->nk;
+  const double bb = (double)ntraj * nstate(c) * sizeof(zd);  // a state of every trajectory
   double budget = mem_budget;
   if (!(budget > 0.0)) {
     size_t fr = 0, tot = 0;
     HIPCHK(c, hipMemGetInfo(&fr, &tot));
     budget = 0.25 * (double)fr;
   }
-  if (4.0 * nt * (double)bb <= budget) {
+  if (4.0 * nt * bb <= budget) {
     s.full = true;
     s.seg = nt;
   } else {
     // sqrt(nt) spacing; if that does not fit, the spacing of least memory,
     // ceil(nt/S) + 4 S states with S ~ sqrt(nt/4)
-    auto need = [&](int S) { return ((double)((nt + S - 1) / S) + 4.0 * S) * (double)bb; };
+    auto need = [&](int S) { return ((double)((nt + S - 1) / S) + 4.0 * S) * bb; };
     int S = (int)std::ceil(std::sqrt((double)nt));
     if (need(S) > budget) S = std::max(1, (int)std::ceil(std::sqrt(nt / 4.0)));
     if (need(S) > budget)
@@ -531,11 +601,30 @@ extern "C" int tdhf_fwd_batch(tdhf_ctx* c, int ntraj, double* u, int nt, const d
     s.full = false;
     s.seg = S;
   }
+  // The density-matrix path pads the k-points: a caller's budget has to hold
+  // the same plan with the padded states, else the run stays row-wise.
+  if (kspace_pays(c->ng, c->nk, c->nb, c->nbocc, ntraj)) {
+    const double kb = (double)ntraj * kcount(c) * sizeof(zd);
+    const double plan = s.full ? 4.0 * nt : (double)((nt + s.seg - 1) / s.seg) + 4.0 * s.seg;
+    s.kp = !(mem_budget > 0.0) || plan * kb <= budget;
+    if (s.kp) {
+      const KScratch k = adj_scratch(c, s);
+      if (hipMalloc((void**)&s.hm, (size_t)ntraj * k.hstride * sizeof(zd)) != hipSuccess ||
+          hipMalloc((void**)&s.nx, (size_t)ntraj * k.nstride * sizeof(double)) != hipSuccess) {
+        (void)hipGetLastError();  // without that memory: row-wise
+        dfree(s.hm);
+        dfree(s.nx);
+        s.kp = false;
+      }
+    }
+  }
+  const size_t ns = adj_count(c, s), blk = (size_t)ntraj * ns;
   int rc = 0;
   const long nsl = (long)nt + 1;
+  const int ostride = adj_obs_stride(c, s);
   if ((rc = dalloc(c, &s.dA, s.A.size())) || (rc = dalloc(c, &s.dAave, s.A.size())) ||
       (rc = dalloc(c, &s.st, 4 * blk)) || (rc = dalloc(c, &s.tape, (size_t)4 * s.seg * blk)) ||
-      (rc = dalloc(c, &s.obs, (size_t)ntraj * nsl * c->obs_stride)) ||
+      (rc = dalloc(c, &s.obs, (size_t)ntraj * nsl * ostride)) ||
       (rc = dalloc(c, &s.res, (size_t)ntraj * nsl * 7)))
     return adj_fail_free(s, rc);
   if (!s.full && (rc = dalloc(c, &s.ckpt, (size_t)((nt + s.seg - 1) / s.seg) * blk)))
@@ -544,14 +633,17 @@ extern "C" int tdhf_fwd_batch(tdhf_ctx* c, int ntraj, double* u, int nt, const d
                            c->stream));
   HIPCHK(c, hipMemcpyAsync(s.dAave, s.Aave.data(), s.Aave.size() * sizeof(double),
                            hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipMemcpyAsync(s.st, u, bb, hipMemcpyHostToDevice, c->stream));
+  const size_t ub = (size_t)ntraj * nstate(c) * sizeof(zd);
+  zd* ref = s.kp ? s.st + blk : s.st;  // the host's layout (through ksum's place)
+  HIPCHK(c, hipMemcpyAsync(ref, u, ub, hipMemcpyHostToDevice, c->stream));
+  if (s.kp) CHKRET(kspace_layout(c, ref, s.st, true, ntraj));
   CHKRET(adj_prepare(c));
   if (s.full) {
     CHKRET(adj_forward_steps(c, s, 0, nt, s.tape));
   } else {
     const long nseg = (nt + s.seg - 1) / s.seg;
     for (int s0 = 0; s0 < nt; s0 += s.seg) {
-      HIPCHK(c, hipMemcpyAsync(s.ckpt + (size_t)(s0 / s.seg) * blk, s.st, bb,
+      HIPCHK(c, hipMemcpyAsync(s.ckpt + (size_t)(s0 / s.seg) * blk, s.st, blk * sizeof(zd),
                                hipMemcpyDeviceToDevice, c->stream));
       CHKRET(adj_forward_steps(c, s, s0, std::min(s.seg, nt - s0), nullptr));
       CHKRET(adj_report(c, 0, s0 / s.seg + 1, nseg));
@@ -570,18 +662,21 @@ extern "C" int tdhf_fwd_batch(tdhf_ctx* c, int ntraj, double* u, int nt, const d
   a.obs = s.obs;
   a.tstride = ns;
   a.fstride = nt;
-  a.ostride = (size_t)nsl * c->obs_stride;
-  CHKRET(launch_apply(c, a, rows, ntraj));
-  for (int t = 0; t < ntraj; ++t) {
+  a.ostride = (size_t)nsl * ostride;
+  CHKRET(adj_stage(c, s, a));
+  if (s.kp) CHKRET(launch_obs_reduce(c, s.obs, nsl, ntraj, a.ostride, s.res));
+  for (int t = 0; t < ntraj && !s.kp; ++t) {
     hipLaunchKernelGGL(tdhf::obs_reduce_kernel, dim3((unsigned)((nsl + 63) / 64)), dim3(64), 0,
-                       c->stream, s.obs + (size_t)t * nsl * c->obs_stride, c->obs_stride, rows,
+                       c->stream, s.obs + (size_t)t * nsl * c->obs_stride, c->obs_stride,
+                       c->nb * c->nk,
                        (int)nsl, c->dv, c->vcell, s.res + (size_t)t * nsl * 7);
     HIPCHK(c, hipGetLastError());
   }
   std::vector<double> res((size_t)ntraj * nsl * 7);
   HIPCHK(c, hipMemcpyAsync(res.data(), s.res, res.size() * sizeof(double), hipMemcpyDeviceToHost,
                            c->stream));
-  HIPCHK(c, hipMemcpyAsync(u, s.st, bb, hipMemcpyDeviceToHost, c->stream));
+  if (s.kp) CHKRET(kspace_layout(c, s.st, ref, false, ntraj));
+  HIPCHK(c, hipMemcpyAsync(u, ref, ub, hipMemcpyDeviceToHost, c->stream));
   CHKRET(sync(c));
   s.jt.resize((size_t)ntraj * nt);
   s.nel.resize((size_t)ntraj * nt);
@@ -626,13 +721,13 @@ extern "C" int tdhf_bwd_batch(tdhf_ctx* c, double* dLdA, double* dLdu0) {
   if (!dLdA) return fail(c, TDHF_EINVAL, "dLdA is NULL");
   if (!s.full && !s.ckpt)
     return fail(c, TDHF_EINVAL, "the checkpointed forward state was consumed by an earlier backward call");
-  const size_t ns = nstate(c), blk = (size_t)s.ntraj * ns;
-  const int rows = c->nb * c->nk;
+  const size_t ns = adj_count(c, s), blk = (size_t)s.ntraj * ns;
+  const int rows = adj_nabar(c, s);
   const int nt = s.nt;
   if (!s.buf) CHKRET(dalloc(c, &s.buf, 4 * blk));
   if (!s.abar) CHKRET(dalloc(c, &s.abar, (size_t)s.ntraj * s.seg * 4 * rows));
   if (!s.stsum) CHKRET(dalloc(c, &s.stsum, (size_t)s.ntraj * nt * 4));
-  CHKRET(adj_tiles_setup(c, s));
+  if (!s.kp) CHKRET(adj_tiles_setup(c, s));
   zd *ua = s.buf, *ub = s.buf + blk, *ga = s.buf + 2 * blk, *gb = s.buf + 3 * blk;
   // cotangent of the final state (s.st holds it after the forward run)
   if (s.objective == TDHF_OBJ_ENERGY) {
@@ -642,7 +737,7 @@ extern "C" int tdhf_bwd_batch(tdhf_ctx* c, double* dLdA, double* dLdu0) {
     e.y = s.st;
     e.cout = ub;
     e.gout = ga;
-    CHKRET(launch_adj(c, e, s.ntraj));
+    CHKRET(s.kp ? launch_kadj(c, s, e) : launch_adj(c, e, s.ntraj));
   } else {
     CHKRET(launch_jgrad(c, s, nt - 1, s.st, ub, ga, 1));
   }
@@ -666,8 +761,15 @@ extern "C" int tdhf_bwd_batch(tdhf_ctx* c, double* dLdA, double* dLdu0) {
   std::vector<double> sts((size_t)s.ntraj * nt * 4);
   HIPCHK(c, hipMemcpyAsync(sts.data(), s.stsum, sts.size() * sizeof(double), hipMemcpyDeviceToHost,
                            c->stream));
-  if (dLdu0)
-    HIPCHK(c, hipMemcpyAsync(dLdu0, ub, blk * sizeof(zd), hipMemcpyDeviceToHost, c->stream));
+  if (dLdu0) {
+    zd* src = ub;
+    if (s.kp) {  // to the host's layout, in a buffer the finished sweep leaves free
+      CHKRET(kspace_layout(c, ub, ga, false, s.ntraj));
+      src = ga;
+    }
+    HIPCHK(c, hipMemcpyAsync(dLdu0, src, (size_t)s.ntraj * nstate(c) * sizeof(zd),
+                             hipMemcpyDeviceToHost, c->stream));
+  }
   CHKRET(sync(c));
   for (int t = 0; t < s.ntraj; ++t) {
     double* g = dLdA + (size_t)t * nt;

@@ -31,8 +31,21 @@ struct tdhf_batch {
   std::vector<int> tab_of;
   std::vector<size_t> off;      // state offset (complex elements) per trajectory
   size_t total = 0;             // complex elements of all trajectories
+  // density-matrix path (tdhf_kspace.h): whether mode 0 takes it, the padded
+  // state offsets, the layout d_state's first region is in, matrices and
+  // density scratch per trajectory, the two launches' work lists
+  bool kuse = false, padded = false;
+  std::vector<size_t> koff;
+  size_t region = 0;            // elements of one of the four state regions
+  size_t *d_roff = nullptr, *d_koff = nullptr;
+  int kn = 0, kmax = 0;         // common transform length (0: several) and the longest
+  zd* d_hm = nullptr;
+  double* d_nx = nullptr;
+  std::vector<size_t> hoff, noff;
+  int2 *d_amap = nullptr, *d_bmap = nullptr;
+  int na = 0, nbm = 0, map_nw = 0, map_sched = -1;
   double* d_vion = nullptr;
-  zd* d_state = nullptr;        // 4 * total: u0 | ksum | sa | sb
+  zd* d_state = nullptr;        // 4 * region: u0 | ksum | sa | sb
   tdhf::TrajDesc* d_td = nullptr;
   std::vector<tdhf::TrajDesc> h_td;
   int2* d_rowmap = nullptr;
@@ -104,6 +117,9 @@ int balloc(tdhf_batch* b, T** p, size_t n) {
   }
   return 0;
 }
+
+// Whether the batch's stages run through the density matrices now.
+bool batch_kspace(const tdhf_batch* b) { return b->kuse && b->xmode == 0; }
 
 size_t bstate(const tdhf_batch* b, int t) { return (size_t)b->p.ng * b->p.nb * b->nk[t]; }
 
@@ -350,10 +366,15 @@ int batch_update_desc(tdhf_batch* b) {
     d.vion = b->d_vion + (size_t)b->p.ng * t;
     d.vtl = c->d_vtl;
     d.kc = c->d_kc;
-    d.u0 = b->d_state + b->off[t];
-    d.ksum = b->d_state + b->total + b->off[t];
-    d.sa = b->d_state + 2 * b->total + b->off[t];
-    d.sb = b->d_state + 3 * b->total + b->off[t];
+    const size_t so = batch_kspace(b) ? b->koff[t] : b->off[t];
+    d.u0 = b->d_state + so;
+    d.ksum = b->d_state + b->region + so;
+    d.sa = b->d_state + 2 * b->region + so;
+    d.sb = b->d_state + 3 * b->region + so;
+    d.n = b->kuse ? c->kn : 0;
+    d.ktab = c->d_ktab;
+    d.hm = b->kuse ? b->d_hm + b->hoff[t] : nullptr;
+    d.nx = b->kuse ? b->d_nx + b->noff[t] : nullptr;
     d.A = b->d_A ? b->d_A + (size_t)b->A_cap * t : nullptr;
     d.Aave = b->d_Aave ? b->d_Aave + (size_t)b->A_cap * t : nullptr;
     d.obs = b->d_obs ? b->d_obs + b->obs_off[t] * (size_t)b->obs_cap : nullptr;
@@ -366,6 +387,138 @@ int batch_update_desc(tdhf_batch* b) {
   BHIP(b, hipMemcpyAsync(b->d_td, b->h_td.data(), b->h_td.size() * sizeof(tdhf::TrajDesc),
                          hipMemcpyHostToDevice, b->stream));
   BHIP(b, hipStreamSynchronize(b->stream));
+  return 0;
+}
+
+// Waves of the product launch: as asked for, as far as the grid has x' for
+// them (every trajectory of the batch).
+int batch_apply_waves(const tdhf_batch* b, int nw) {
+  int w = nw;
+  for (size_t i = 0; i < b->tabs.size(); ++i)
+    w = std::min(w, kapply_waves(b->tabs[i]->kn, b->p.ng));
+  return w;
+}
+
+long batch_tasks(const tdhf_batch* b) {
+  long tasks = 0;
+  for (int t = 0; t < b->ntraj; ++t)
+    tasks += tdhf::kmat_tasks(b->p.ng, kspace_gpw(b->tabs[b->tab_of[t]]->kn));
+  return tasks;
+}
+
+int batch_points(const tdhf_batch* b) {
+  long groups = 0;
+  for (int t = 0; t < b->ntraj; ++t)
+    groups += kapply_groups(b->tabs[b->tab_of[t]]->kn, b->p.ng, b->p.nb, 1);
+  return kapply_points(groups);
+}
+
+// Work lists of the two launches for the current row schedule: per trajectory
+// its groups of (x, block) tasks and its (x tile, bands, k block) items, the
+// trajectories pinned to XCDs (schedules 0 and 1; 1 interleaves those of an
+// XCD) or spread (2), the costliest first.
+int batch_kspace_maps(tdhf_batch* b) {
+  if (b->map_sched == b->sched) return 0;
+  const int wa = kmat_waves(batch_tasks(b));
+  std::vector<int2> am, bm;
+  auto build = [&](std::vector<int2>& map, auto count) {
+    constexpr int kXcd = 8;
+    std::vector<int> order(b->ntraj);
+    std::iota(order.begin(), order.end(), 0);
+    auto cost = [&](int t) { return (double)count(t) * b->tabs[b->tab_of[t]]->kn; };
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cost(x) > cost(y); });
+    map.clear();
+    if (b->sched == 2) {
+      for (int t : order)
+        for (int i = 0; i < count(t); ++i) map.push_back(make_int2(t, i));
+      return;
+    }
+    std::vector<double> load(kXcd, 0.0);
+    std::vector<std::vector<int>> bins(kXcd);
+    for (int t : order) {
+      const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+      load[x] += cost(t);
+      bins[x].push_back(t);
+    }
+    std::vector<std::vector<int2>> q(kXcd);
+    size_t longest = 0;
+    for (int x = 0; x < kXcd; ++x) {
+      int most = 0;
+      for (int t : bins[x]) most = std::max(most, count(t));
+      if (b->sched == 1) {
+        for (int i = 0; i < most; ++i)
+          for (int t : bins[x])
+            if (i < count(t)) q[x].push_back(make_int2(t, i));
+      } else {
+        for (int t : bins[x])
+          for (int i = 0; i < count(t); ++i) q[x].push_back(make_int2(t, i));
+      }
+      longest = std::max(longest, q[x].size());
+    }
+    for (size_t i = 0; i < longest; ++i)
+      for (int x = 0; x < kXcd; ++x) map.push_back(i < q[x].size() ? q[x][i] : make_int2(-1, 0));
+    while (!map.empty() && map.back().x < 0) map.pop_back();
+  };
+  build(am, [&](int t) { return kmat_groups(b->tabs[b->tab_of[t]]->kn, b->p.ng, wa); });
+  const int xt = batch_points(b);
+  build(bm, [&](int t) { return kapply_groups(b->tabs[b->tab_of[t]]->kn, b->p.ng, b->p.nb, xt); });
+  BHIP(b, hipStreamSynchronize(b->stream));
+  dfree(b->d_amap);
+  dfree(b->d_bmap);
+  CHKRET(balloc(b, &b->d_amap, am.size()));
+  CHKRET(balloc(b, &b->d_bmap, bm.size()));
+  BHIP(b, hipMemcpy(b->d_amap, am.data(), am.size() * sizeof(int2), hipMemcpyHostToDevice));
+  BHIP(b, hipMemcpy(b->d_bmap, bm.data(), bm.size() * sizeof(int2), hipMemcpyHostToDevice));
+  b->na = (int)am.size();
+  b->nbm = (int)bm.size();
+  b->map_sched = b->sched;
+  return 0;
+}
+
+int batch_kspace_launch(tdhf_batch* b, const tdhf::ApplyArgs& a, int nw) {
+  tdhf::KArgs k{};
+  k.a = a;
+  k.ng = b->p.ng;
+  k.nchunk = kspace_chunks(b->p.nb);
+  for (auto c : b->tabs) {
+    k.tw[kspace_class(c->kn)] = c->d_ktw;
+    k.om[kspace_class(c->kn)] = c->d_om;
+  }
+  k.amap = b->d_amap;
+  k.bmap = b->d_bmap;
+  void* args[] = {&k};
+  const bool obs = a.mode == tdhf::M_S1 || a.mode == tdhf::M_OBS;
+  const long tasks = batch_tasks(b);
+  const int wa = kmat_waves(tasks), wb = batch_apply_waves(b, nw), nbt = kspace_nbt(b->p.nb);
+  const int xt = batch_points(b);
+  BHIP(b, hipLaunchKernel(kmat_fn_for(b->kn, obs, kmat_deep(tasks)), dim3(b->na), dim3(64 * wa),
+                          args, kmat_lds_for(b->kn, wa, b->p.ng), b->stream));
+  BHIP(b, hipLaunchKernel(kapply_fn(nbt, xt), dim3(b->nbm), dim3(64 * wb), args,
+                          tdhf::kapply_lds(wb, nbt, xt), b->stream));
+  return 0;
+}
+
+// The resident states into the padded layout or back (through the region of
+// the second stage state, which holds nothing between steps).
+int batch_layout(tdhf_batch* b, bool padded) {
+  if (b->padded == padded) return 0;
+  zd* tmp = b->d_state + 2 * b->region;
+  tdhf::KLayoutArgs l{};
+  l.src = b->d_state;
+  l.dst = tmp;
+  l.ng = b->p.ng;
+  l.nb = b->p.nb;
+  l.td = b->d_td;
+  l.roff = b->d_roff;
+  l.koff = b->d_koff;
+  l.to_k = padded;
+  hipLaunchKernelGGL(tdhf::kspace_layout_kernel,
+                     dim3(b->p.ng / 16, b->kmax / 16, b->p.nb * b->ntraj), dim3(256), 0, b->stream,
+                     l);
+  BHIP(b, hipGetLastError());
+  BHIP(b, hipMemcpyAsync(b->d_state, tmp, b->region * sizeof(zd), hipMemcpyDeviceToDevice,
+                         b->stream));
+  b->padded = padded;
   return 0;
 }
 
@@ -407,7 +560,9 @@ int batch_launch(tdhf_batch* b, const tdhf::ApplyArgs& a, int nw) {
     }
     BHIP(b, hipGetLastError());
   }
-  if (b->xmode) {  // pair tiles: NG = 64 (batch_pairtile_ok); 8 rows per wave
+  if (batch_kspace(b)) {
+    CHKRET(batch_kspace_launch(b, a, nw));
+  } else if (b->xmode) {  // pair tiles: NG = 64 (batch_pairtile_ok); 8 rows per wave
     const int rpb = 8 * nw;
     hipLaunchKernelGGL(tdhf::pair_epilogue_kernel, dim3((b->nerows + rpb - 1) / rpb),
                        dim3(64 * nw), tdhf::pair_epilogue_lds_bytes(nw), b->stream, a, b->d_erows,
@@ -509,6 +664,11 @@ int batch_run_steps(tdhf_batch* b, int nt) {
   return 0;
 }
 
+// Doubles of trajectory t's observables slot (the larger of the two paths').
+size_t batch_slot(const tdhf_batch* b, int t) {
+  return std::max((size_t)3 * b->p.nb * b->nk[t] + 3, (size_t)tdhf::kspace_obs_stride(b->p.ng));
+}
+
 int batch_ensure(tdhf_batch* b, long nt) {
   if (nt > b->A_cap || nt + 1 > b->obs_cap) {
     if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
@@ -521,7 +681,7 @@ int batch_ensure(tdhf_batch* b, long nt) {
     CHKRET(balloc(b, &b->d_A, (size_t)cap * b->ntraj));
     CHKRET(balloc(b, &b->d_Aave, (size_t)cap * b->ntraj));
     size_t per_slot = 0;
-    for (int t = 0; t < b->ntraj; ++t) per_slot += 3 * (size_t)b->p.nb * b->nk[t] + 3;
+    for (int t = 0; t < b->ntraj; ++t) per_slot += batch_slot(b, t);
     CHKRET(balloc(b, &b->d_obs, per_slot * (size_t)(cap + 1)));
     CHKRET(balloc(b, &b->d_res, (size_t)7 * b->ntraj * (cap + 1)));
     b->A_cap = cap;
@@ -540,10 +700,54 @@ void batch_release(tdhf_batch* b) {
   dfree(b->d_vion); dfree(b->d_state); dfree(b->d_td); dfree(b->d_rowmap); dfree(b->d_erows);
   dfree(b->d_A); dfree(b->d_Aave); dfree(b->d_obs); dfree(b->d_res); dfree(b->d_step);
   dfree(b->d_xpart); dfree(b->d_dpart); dfree(b->d_tiles);
+  dfree(b->d_roff); dfree(b->d_koff); dfree(b->d_hm); dfree(b->d_nx);
+  dfree(b->d_amap); dfree(b->d_bmap);
   for (auto c : b->tabs) tdhf_destroy(c);
   b->tabs.clear();
   if (b->stream) (void)hipStreamDestroy(b->stream);
   b->stream = nullptr;
+}
+
+// Sets the batch up for the density-matrix path where it serves every
+// trajectory and is the faster one (KspaceCost); without memory for the
+// matrices mode 0 stays row-wise.
+int batch_kspace_setup(tdhf_batch* b) {
+  for (auto c : b->tabs)
+    if (!c->kn) return 0;
+  KspaceCost cost;
+  for (int k : b->nk) cost.add(b->p.ng, k, b->p.nb, b->p.nbocc);
+  if (!cost.pays()) return 0;
+  const int ng = b->p.ng;
+  size_t ks = 0, hs = 0, xs = 0;
+  b->koff.resize(b->ntraj);
+  b->hoff.resize(b->ntraj);
+  b->noff.resize(b->ntraj);
+  for (int t = 0; t < b->ntraj; ++t) {
+    const int n = b->tabs[b->tab_of[t]]->kn;
+    b->koff[t] = ks;
+    b->hoff[t] = hs;
+    b->noff[t] = xs;
+    ks += (size_t)ng * b->p.nb * n;
+    hs += tdhf::kmat_elems(ng, n);
+    xs += tdhf::kmat_extra(ng, kspace_gpw(n));
+    b->kmax = std::max(b->kmax, n);
+    b->kn = t == 0 || b->kn == n ? n : 0;
+  }
+  if (hipMalloc((void**)&b->d_hm, hs * sizeof(zd)) != hipSuccess) {
+    (void)hipGetLastError();
+    b->d_hm = nullptr;
+    return 0;
+  }
+  CHKRET(balloc(b, &b->d_nx, xs));
+  CHKRET(balloc(b, &b->d_roff, (size_t)b->ntraj));
+  CHKRET(balloc(b, &b->d_koff, (size_t)b->ntraj));
+  BHIP(b, hipMemcpy(b->d_roff, b->off.data(), b->ntraj * sizeof(size_t), hipMemcpyHostToDevice));
+  BHIP(b, hipMemcpy(b->d_koff, b->koff.data(), b->ntraj * sizeof(size_t), hipMemcpyHostToDevice));
+  const hipError_t e = kmat_lds_limits(b->kn, b->p.nb);
+  if (e != hipSuccess) return bfail(b, TDHF_EDEVICE, "LDS limit: %s", hipGetErrorString(e));
+  b->region = std::max(b->total, ks);
+  b->kuse = true;
+  return 0;
 }
 
 // autotuner cache: shape -> (waves per workgroup, row schedule, exchange
@@ -632,11 +836,14 @@ int tdhf_batch_create(const tdhf_params* p, int ntraj, const int* nk, const doub
     b->off[t] = acc;
     acc += bstate(b, t);
     b->obs_off[t] = oacc;
-    oacc += 3 * (size_t)p->nb * nk[t] + 3;
+    oacc += batch_slot(b, t);
   }
   b->total = acc;
+  b->region = acc;
   int rc;
-  if ((rc = balloc(b, &b->d_vion, (size_t)p->ng * ntraj)) || (rc = balloc(b, &b->d_state, 4 * acc)) ||
+  if ((rc = batch_kspace_setup(b))) return bail(rc);
+  if ((rc = balloc(b, &b->d_vion, (size_t)p->ng * ntraj)) ||
+      (rc = balloc(b, &b->d_state, 4 * b->region)) ||
       (rc = balloc(b, &b->d_td, (size_t)ntraj)) || (rc = balloc(b, &b->d_step, 1)))
     return bail(rc);
   if (hipMemcpy(b->d_vion, vion, sizeof(double) * p->ng * ntraj, hipMemcpyHostToDevice) != hipSuccess) {
@@ -649,9 +856,13 @@ int tdhf_batch_create(const tdhf_params* p, int ntraj, const int* nk, const doub
   // workgroups share a CU) and the XCD-pinned schedule
   std::array<int, 3> ct{};
   const bool cached = tune_lookup(tune_key(b), &ct);
-  b->nw = cached ? ct[0] : (p->ng + 63) / 64;
+  // (density matrices: 8 waves for the product launch, 4 where it has
+  // workgroups enough; fewer trajectories than XCDs are not pinned to them,
+  // NG=128, NK=128, NB=8: 4 trajectories 166 us per stage pinned, 101 not)
+  b->nw = cached ? ct[0] : !b->kuse ? (p->ng + 63) / 64 : batch_points(b) > 1 ? 4 : 8;
   b->ngrid = 0;
-  if ((rc = batch_set_schedule(b, cached ? ct[1] : 0))) return bail(rc);
+  if ((rc = batch_set_schedule(b, cached ? ct[1] : b->kuse && ntraj < 8 ? 2 : 0)))
+    return bail(rc);
   b->h_td.resize(ntraj);
   if ((rc = batch_update_desc(b))) return bail(rc);
   if (cached && ct[2] && (rc = batch_set_xmode(b, ct[2]))) return bail(rc);
@@ -670,17 +881,21 @@ int tdhf_batch_destroy(tdhf_batch* b) {
 
 int tdhf_batch_upload(tdhf_batch* b, int traj, const double* u) {
   if (!b || !u || traj >= b->ntraj) return bfail(b, TDHF_EINVAL, "invalid upload arguments");
-  if (traj < 0)
+  if (traj < 0) {
+    b->padded = false;
     BHIP(b, hipMemcpyAsync(b->d_state, u, b->total * sizeof(zd), hipMemcpyHostToDevice, b->stream));
-  else
+  } else {
+    CHKRET(batch_layout(b, false));
     BHIP(b, hipMemcpyAsync(b->d_state + b->off[traj], u, bstate(b, traj) * sizeof(zd),
                            hipMemcpyHostToDevice, b->stream));
+  }
   BHIP(b, hipStreamSynchronize(b->stream));
   return 0;
 }
 
 int tdhf_batch_download(tdhf_batch* b, int traj, double* u) {
   if (!b || !u || traj >= b->ntraj) return bfail(b, TDHF_EINVAL, "invalid download arguments");
+  CHKRET(batch_layout(b, false));
   if (traj < 0)
     BHIP(b, hipMemcpyAsync(u, b->d_state, b->total * sizeof(zd), hipMemcpyDeviceToHost, b->stream));
   else
@@ -695,6 +910,8 @@ int tdhf_batch_propagate(tdhf_batch* b, int nt, const double* A, const double* A
   if (!b) return bfail(nullptr, TDHF_EINVAL, "batch is NULL");
   if (nt < 1 || !A || !Aave) return bfail(b, TDHF_EINVAL, "invalid field arrays");
   CHKRET(batch_ensure(b, nt));
+  CHKRET(batch_layout(b, batch_kspace(b)));
+  if (batch_kspace(b)) CHKRET(batch_kspace_maps(b));
   for (int t = 0; t < b->ntraj; ++t) {
     BHIP(b, hipMemcpyAsync(b->d_A + (size_t)b->A_cap * t, A + (size_t)nt * t, nt * sizeof(double),
                            hipMemcpyHostToDevice, b->stream));
@@ -712,9 +929,14 @@ int tdhf_batch_propagate(tdhf_batch* b, int nt, const double* A, const double* A
   CHKRET(batch_launch(b, a, b->nw));
   const int ns = nt + 1;
   const int n = b->ntraj * ns;
-  hipLaunchKernelGGL(tdhf::obs_reduce_batch_kernel, dim3((n + 63) / 64), dim3(64), 0, b->stream,
-                     b->d_td, b->ntraj, b->p.nb, ns, std::fabs(b->p.acell) / (double)b->p.ng,
-                     std::fabs(b->p.acell), b->d_res);
+  const double vcell = std::fabs(b->p.acell), dv = vcell / (double)b->p.ng;
+  if (batch_kspace(b))
+    hipLaunchKernelGGL(tdhf::kspace_obs_reduce_kernel, dim3((n + 3) / 4), dim3(256), 0, b->stream,
+                       (const double*)nullptr, b->d_td, b->p.ng, ns, n, dv, vcell, (size_t)0,
+                       b->d_res);
+  else
+    hipLaunchKernelGGL(tdhf::obs_reduce_batch_kernel, dim3((n + 63) / 64), dim3(64), 0, b->stream,
+                       b->d_td, b->ntraj, b->p.nb, ns, dv, vcell, b->d_res);
   BHIP(b, hipGetLastError());
   std::vector<double> res((size_t)7 * n);
   BHIP(b, hipMemcpyAsync(res.data(), b->d_res, res.size() * sizeof(double), hipMemcpyDeviceToHost,
@@ -778,6 +1000,7 @@ int tdhf_batch_autotune(tdhf_batch* b, int nt_trial, const double* A, const doub
   if (!b || nt_trial < 1 || !A || !Aave) return bfail(b, TDHF_EINVAL, "invalid autotune arguments");
   // keep the state: the trial steps run on a copy, freed on every return
   zd* save = nullptr;
+  CHKRET(batch_layout(b, false));
   CHKRET(balloc(b, &save, b->total));
   struct FreeOnReturn {
     zd*& p;
@@ -787,7 +1010,9 @@ int tdhf_batch_autotune(tdhf_batch* b, int nt_trial, const double* A, const doub
   int best = b->nw, best_s = b->sched, best_x = b->xmode;
   double best_t = 1e300;
   const int cand[4] = {1, 2, 4, 8};
-  for (int xm = 0; xm <= (batch_pairtile_ok(b) ? 3 : 0); ++xm)
+  // the pair tiles are candidates where mode 0 is row-wise (the density-matrix
+  // path is only taken where it is faster than either, KspaceCost)
+  for (int xm = 0; xm <= (batch_pairtile_ok(b) && !b->kuse ? 3 : 0); ++xm)
   for (int sc = 0; sc < kNumSchedules; ++sc) {
     CHKRET(batch_set_xmode(b, xm));
     CHKRET(batch_set_schedule(b, sc));
@@ -799,8 +1024,10 @@ int tdhf_batch_autotune(tdhf_batch* b, int nt_trial, const double* A, const doub
       // the first repetition warms up (graph capture); the faster of the
       // next two counts
       for (int rep = 0; rep < 3 && !rc; ++rep) {
+        b->padded = false;
         BHIP(b, hipMemcpyAsync(b->d_state, save, b->total * sizeof(zd), hipMemcpyDeviceToDevice,
                                b->stream));
+        CHKRET(batch_layout(b, batch_kspace(b)));
         BHIP(b, hipStreamSynchronize(b->stream));
         auto t0 = std::chrono::steady_clock::now();
         rc = tdhf_batch_propagate(b, nt_trial, A, Aave, nullptr, nullptr, nullptr, nullptr);
@@ -816,6 +1043,7 @@ int tdhf_batch_autotune(tdhf_batch* b, int nt_trial, const double* A, const doub
       }
     }
   }
+  b->padded = false;
   BHIP(b, hipMemcpyAsync(b->d_state, save, b->total * sizeof(zd), hipMemcpyDeviceToDevice, b->stream));
   BHIP(b, hipStreamSynchronize(b->stream));
   b->nw = best;

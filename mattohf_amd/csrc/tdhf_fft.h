@@ -55,6 +55,12 @@ __device__ __forceinline__ zd gload(const zd* p) {
 __device__ __forceinline__ double gload(const double* p) {
   return *(const TDHF_GLOBAL double*)(p);
 }
+// The same from a wave-uniform base and a 32-bit byte offset of the lane: the
+// base stays in scalar registers.
+__device__ __forceinline__ zd gload_at(const zd* base, unsigned off) {
+  const gd2 v = *(const TDHF_GLOBAL gd2*)((const TDHF_GLOBAL char*)base + off);
+  return mk(v.x, v.y);
+}
 __device__ __forceinline__ void gstore(zd* p, zd v) {
   gd2 t;
   t.x = v.x;

@@ -107,6 +107,7 @@ extern "C" int tdhf_gs_run(tdhf_ctx* c, double* u, int nscf, int ncg, double tol
   CHKRET(gs_alloc(c, ncg));
   CHKRET(gs_flag_clear(c));
   CHKRET(upload(c, c->d_u0, u));
+  c->u0_padded = false;
   double r[7];
   CHKRET(observables_of(c, c->d_u0, 0.0, r));
   double eprev = r[0];

@@ -65,6 +65,12 @@ struct TrajDesc {
   double* dpart;
   int nblk;
   const double* vhg;  // vCG(G)/NG in the G layout of GroupFFT<NG> (pair-tile epilogue)
+  // density-matrix path (tdhf_kspace.h): length of the k transforms (the
+  // padded number of k-points) and the Coulomb spectra
+  int n;
+  const zd* ktab;
+  zd* hm;
+  double* nx;
 };
 
 // Offsets inside one observables slot: rows*3 partials then (N, Eion, EH).

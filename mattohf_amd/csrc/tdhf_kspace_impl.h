@@ -1,0 +1,316 @@
+// tdhf_kspace_impl.h -- host side of the density-matrix path (included by
+// tdhf.hip after the row-wise launch helpers): when it is used, its tables,
+// launches, layout conversions and observables.
+#pragma once
+
+namespace {
+
+// Whether the density-matrix path pays for nk k-points of ntraj trajectories:
+// its cost against that of the row-wise exchange, in microseconds per stage as
+// measured over NG = 16..128, NK = 4..128, NB = 1..8 and 1..64 trajectories.
+// Row-wise: 5.5 + 0.42 per 10^6 grid points in the pair transforms, weighted by
+// log2 NG.  Density matrices: 13 (two launches, each with its own memory round
+// trips) + 12 per 10^6 matrix elements.  Near the line: NG=64, NK=64, NB=4
+// (one trajectory) 15.5 against 16.0 stays row-wise; NG=128, NK=64, NB=4 32.5
+// against 27.8 does not.
+struct KspaceCost {
+  double rows = 0.0, mat = 0.0;
+  void add(int ng, int nk, int nb, int nbocc, int ntraj = 1) {
+    int lg = 0;
+    while ((1 << lg) < ng) ++lg;
+    rows += 1e-6 * ntraj * nk * nk * nb * nbocc * (double)ng * lg;
+    mat += 1e-6 * ntraj * (double)ng * ng * tdhf::kspace_len(nk);
+  }
+  bool pays() const { return 5.5 + 0.42 * rows > 13.0 + 12.0 * mat; }
+};
+
+bool kspace_pays(int ng, int nk, int nb, int nbocc, int ntraj) {
+  if (!tdhf::kspace_len(nk)) return false;
+  KspaceCost c;
+  c.add(ng, nk, nb, nbocc, ntraj);
+  return c.pays();
+}
+
+// x' values per wave (transform groups).
+int kspace_gpw(int n) { return n == 128 ? 4 : n == 64 ? 8 : 16; }
+
+// Bands per workgroup: 2, 4 or 8 accumulators per lane and k (a variant of
+// the kernel each); more bands go to further workgroups.
+int kspace_nbt(int nbw) { return nbw <= 2 ? 2 : nbw <= 4 ? 4 : 8; }
+int kspace_chunks(int nbw) { return (nbw + kspace_nbt(nbw) - 1) / kspace_nbt(nbw); }
+
+template <int N>
+const void* kmat_fn(bool obs, bool deep) {
+  if (deep)
+    return obs ? (const void*)tdhf::kmat_kernel<N, true, true>
+               : (const void*)tdhf::kmat_kernel<N, false, true>;
+  return obs ? (const void*)tdhf::kmat_kernel<N, true, false>
+             : (const void*)tdhf::kmat_kernel<N, false, false>;
+}
+const void* kmat_fn_for(int n, bool obs, bool deep) {
+  switch (n) {
+    case 16: return kmat_fn<16>(obs, deep);
+    case 32: return kmat_fn<32>(obs, deep);
+    case 64: return kmat_fn<64>(obs, deep);
+    case 128: return kmat_fn<128>(obs, deep);
+  }
+  return kmat_fn<0>(obs, deep);
+}
+template <int XT>
+const void* kapply_fn(int nbt) {
+  return nbt == 2   ? (const void*)tdhf::kapply_kernel<2, XT>
+         : nbt == 4 ? (const void*)tdhf::kapply_kernel<4, XT>
+                    : (const void*)tdhf::kapply_kernel<8, XT>;
+}
+const void* kapply_fn(int nbt, int xt) { return xt == 1 ? kapply_fn<1>(nbt) : kapply_fn<2>(nbt); }
+const void* kadj_mat_fn(int n) {
+  switch (n) {
+    case 16: return (const void*)tdhf::kadj_mat_kernel<16>;
+    case 32: return (const void*)tdhf::kadj_mat_kernel<32>;
+    case 64: return (const void*)tdhf::kadj_mat_kernel<64>;
+  }
+  return (const void*)tdhf::kadj_mat_kernel<128>;
+}
+template <int XT>
+const void* kadj_apply_fn(int nbt) {
+  return nbt == 2   ? (const void*)tdhf::kadj_apply_kernel<2, XT>
+         : nbt == 4 ? (const void*)tdhf::kadj_apply_kernel<4, XT>
+                    : (const void*)tdhf::kadj_apply_kernel<8, XT>;
+}
+const void* kadj_apply_fn(int nbt, int xt) {
+  return xt == 1 ? kadj_apply_fn<1>(nbt) : kadj_apply_fn<2>(nbt);
+}
+size_t kmat_lds_for(int n, int nw, int ng) {
+  switch (n) {
+    case 16: return tdhf::kmat_lds<16>(nw, ng);
+    case 32: return tdhf::kmat_lds<32>(nw, ng);
+    case 64: return tdhf::kmat_lds<64>(nw, ng);
+    case 128: return tdhf::kmat_lds<128>(nw, ng);
+  }
+  return std::max(tdhf::kmat_lds<64>(nw, ng), tdhf::kmat_lds<128>(nw, ng));
+}
+// Two waves per SIMD hold all tasks at once: the deep variant.
+bool kmat_deep(long tasks) { return tasks <= 8L * device_cus(); }
+hipError_t kmat_lds_limits(int n, int nbw) {
+  hipError_t e = hipSuccess;
+  for (int v = 0; v < 4 && e == hipSuccess; ++v)
+    e = hipFuncSetAttribute(kmat_fn_for(n, v & 1, v & 2),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  const int nbt = kspace_nbt(nbw);
+  const void* more[] = {kapply_fn(nbt, 1), kapply_fn(nbt, 2), kadj_mat_fn(n), kadj_apply_fn(nbt, 1),
+                        kadj_apply_fn(nbt, 2)};
+  for (auto f : more)
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  return e;
+}
+// Workgroups of the two launches for one trajectory (nw waves each).
+int kmat_groups(int n, int ng, int nw) {
+  return (tdhf::kmat_tasks(ng, kspace_gpw(n)) + nw - 1) / nw;
+}
+int kapply_groups(int n, int ng, int nbw, int xt) {
+  return ng / xt * kspace_chunks(nbw) * (n > 64 ? n / 64 : 1);
+}
+int kmat_waves(long tasks) { return tasks >= 4096 ? 4 : tasks >= 1024 ? 2 : 1; }
+// Grid points per workgroup of the product launch: two share the columns they
+// read where one each would already fill the CUs.
+int kapply_points(long groups1) { return groups1 >= 512 ? 2 : 1; }
+int kapply_waves(int n, int ng) {
+  const int xs = n < 64 ? 64 / n : 1;
+  int nw = 8;
+  while (nw > 1 && nw * xs > ng) nw /= 2;
+  return nw;
+}
+
+size_t kcount(const tdhf_ctx* c) { return (size_t)c->ng * c->nb * c->kn; }
+
+// complex elements of a state in the path's layout
+size_t path_count(const tdhf_ctx* c) { return c->kpath ? kcount(c) : nstate(c); }
+
+// Spectra, twiddles of the k transforms and the twist factors of a context.
+int kspace_tables(tdhf_ctx* c) {
+  const int NG = c->ng, NK = c->nk, ND = 2 * NK - 1, N = c->kn;
+  zd* tsp = nullptr;
+  CHKRET(dalloc(c, &c->d_ktab, (size_t)NG * 2 * N));
+  CHKRET(dalloc(c, &c->d_ktw, 2 * N));
+  CHKRET(dalloc(c, &c->d_om, N));
+  if (c->kpath) {
+    CHKRET(dalloc(c, &c->d_hm, tdhf::kmat_elems(NG, N)));
+    CHKRET(dalloc(c, &c->d_nx, tdhf::kmat_extra(NG, kspace_gpw(N))));
+  }
+  CHKRET(dalloc(c, &tsp, (size_t)ND * NG));
+  hipStream_t s = c->stream;
+  hipLaunchKernelGGL(tdhf::kspace_space_kernel, dim3((ND * NG + 255) / 256), dim3(256), 0, s,
+                     c->d_vq, ND, NG, -1.0 / ((double)NG * (double)NK), tsp);
+  const dim3 g((NG * 2 * N + 255) / 256), b(256), g1(1);
+  switch (N) {
+    case 16:
+      hipLaunchKernelGGL(tdhf::kspace_spectrum_kernel<16>, g, b, 0, s, tsp, NK, NG, c->d_ktab);
+      hipLaunchKernelGGL(tdhf::twiddle_kernel<16>, g1, b, 0, s, c->d_ktw);
+      break;
+    case 32:
+      hipLaunchKernelGGL(tdhf::kspace_spectrum_kernel<32>, g, b, 0, s, tsp, NK, NG, c->d_ktab);
+      hipLaunchKernelGGL(tdhf::twiddle_kernel<32>, g1, b, 0, s, c->d_ktw);
+      break;
+    case 64:
+      hipLaunchKernelGGL(tdhf::kspace_spectrum_kernel<64>, g, b, 0, s, tsp, NK, NG, c->d_ktab);
+      hipLaunchKernelGGL(tdhf::twiddle_kernel<64>, g1, b, 0, s, c->d_ktw);
+      break;
+    default:
+      hipLaunchKernelGGL(tdhf::kspace_spectrum_kernel<128>, g, b, 0, s, tsp, NK, NG, c->d_ktab);
+      hipLaunchKernelGGL(tdhf::twiddle_kernel<128>, g1, b, 0, s, c->d_ktw);
+      break;
+  }
+  hipLaunchKernelGGL(tdhf::kspace_om_kernel, g1, dim3(128), 0, s, c->d_om, N);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  dfree(tsp);
+  if (e == hipSuccess) e = kmat_lds_limits(N, c->nb);
+  if (e != hipSuccess) return fail(c, TDHF_EDEVICE, "k-space tables: %s", hipGetErrorString(e));
+  return 0;
+}
+
+int kspace_class(int n) { return n == 16 ? 0 : n == 32 ? 1 : n == 64 ? 2 : 3; }
+
+// Arguments of a launch on the context's own tables (states in the padded
+// k-fastest layout); a as for launch_apply.
+tdhf::KArgs kspace_args(const tdhf_ctx* c, const tdhf::ApplyArgs& a) {
+  tdhf::KArgs k{};
+  k.a = a;
+  k.ng = c->ng;
+  k.n = c->kn;
+  k.nchunk = kspace_chunks(a.nbw);
+  k.ktab = c->d_ktab;
+  k.tw[kspace_class(c->kn)] = c->d_ktw;
+  k.om[kspace_class(c->kn)] = c->d_om;
+  return k;
+}
+
+// Matrices and density scratch of ntraj trajectories.
+struct KScratch {
+  zd* hm;
+  double* nx;
+  size_t hstride, nstride;
+};
+
+int launch_kspace(tdhf_ctx* c, const tdhf::ApplyArgs& a, int ntraj = 1,
+                  hipStream_t st = nullptr, const KScratch* sc = nullptr) {
+  tdhf::KArgs k = kspace_args(c, a);
+  k.hm = sc ? sc->hm : c->d_hm;
+  k.nx = sc ? sc->nx : c->d_nx;
+  k.hstride = sc ? sc->hstride : 0;
+  k.nstride = sc ? sc->nstride : 0;
+  const bool timed = c->timing && !st;
+  hipStream_t s = st ? st : c->stream;
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  if (timed) {
+    CHKRET(take_events(c, &e0, &e1));
+    HIPCHK(c, hipEventRecord(e0, c->stream));
+  }
+  const bool obs = a.mode == tdhf::M_S1 || a.mode == tdhf::M_OBS;
+  void* args[] = {&k};
+  const long tasks = (long)tdhf::kmat_tasks(c->ng, kspace_gpw(c->kn)) * ntraj;
+  const int wa = kmat_waves(tasks);
+  HIPCHK(c, hipLaunchKernel(kmat_fn_for(c->kn, obs, kmat_deep(tasks)),
+                            dim3(kmat_groups(c->kn, c->ng, wa), ntraj), dim3(64 * wa), args,
+                            kmat_lds_for(c->kn, wa, c->ng), s));
+  const int wb = kapply_waves(c->kn, c->ng), nbt = kspace_nbt(a.nbw);
+  const int xt = kapply_points((long)kapply_groups(c->kn, c->ng, a.nbw, 1) * ntraj);
+  HIPCHK(c, hipLaunchKernel(kapply_fn(nbt, xt),
+                            dim3(kapply_groups(c->kn, c->ng, a.nbw, xt), ntraj), dim3(64 * wb),
+                            args, tdhf::kapply_lds(wb, nbt, xt), s));
+  if (timed) HIPCHK(c, hipEventRecord(e1, c->stream));
+  return 0;
+}
+
+// One stage launch of the context's path, states in that path's layout.
+int launch_stage(tdhf_ctx* c, const tdhf::ApplyArgs& a) {
+  return c->kpath ? launch_kspace(c, a) : launch_apply(c, a, c->nb * c->nk);
+}
+
+// dst = src in the other layout, for ntraj states back to back.
+int kspace_layout(tdhf_ctx* c, const zd* src, zd* dst, bool to_k, int ntraj = 1,
+                  hipStream_t st = nullptr) {
+  tdhf::KLayoutArgs l{};
+  l.src = src;
+  l.dst = dst;
+  l.ng = c->ng;
+  l.nb = c->nb;
+  l.nk = c->nk;
+  l.n = c->kn;
+  l.sstride = to_k ? nstate(c) : kcount(c);
+  l.dstride = to_k ? kcount(c) : nstate(c);
+  l.to_k = to_k;
+  hipLaunchKernelGGL(tdhf::kspace_layout_kernel, dim3(c->ng / 16, c->kn / 16, c->nb * ntraj),
+                     dim3(256), 0, st ? st : c->stream, l);
+  HIPCHK(c, hipGetLastError());
+  return 0;
+}
+
+// Host state to dst in the path's layout (through d_ksum, which holds nothing
+// between steps), and back.
+int upload_state(tdhf_ctx* c, zd* dst, const double* src) {
+  if (!c->kpath) return upload(c, dst, src);
+  CHKRET(upload(c, c->d_ksum, src));
+  return kspace_layout(c, c->d_ksum, dst, true);
+}
+
+int download_state(tdhf_ctx* c, double* dst, const zd* src) {
+  if (!c->kpath) return download(c, dst, src);
+  CHKRET(kspace_layout(c, src, c->d_ksum, false));
+  return download(c, dst, c->d_ksum);
+}
+
+// The resident state in the path's layout (the ground state leaves it in the
+// host's).
+int resident_to_path(tdhf_ctx* c) {
+  if (!c->kpath || c->u0_padded) return 0;
+  CHKRET(kspace_layout(c, c->d_u0, c->d_ksum, true));
+  HIPCHK(c, hipMemcpyAsync(c->d_u0, c->d_ksum, kcount(c) * sizeof(zd), hipMemcpyDeviceToDevice,
+                           c->stream));
+  c->u0_padded = true;
+  return 0;
+}
+
+// Observables of nslots slots reduced into out (7 values each), ntraj
+// trajectories ostride doubles apart.
+int launch_obs_reduce(tdhf_ctx* c, const double* obs, long nslots, int ntraj, size_t ostride,
+                      double* out) {
+  const long nw = nslots * ntraj;
+  hipLaunchKernelGGL(tdhf::kspace_obs_reduce_kernel, dim3((unsigned)((nw + 3) / 4)), dim3(256), 0,
+                     c->stream, obs, (const tdhf::TrajDesc*)nullptr, c->ng, (int)nslots, (int)nw,
+                     c->dv, c->vcell, ostride, out);
+  HIPCHK(c, hipGetLastError());
+  return 0;
+}
+
+// Observables of the state u (in the path's layout) at field A.
+int path_observables_of(tdhf_ctx* c, const zd* u, double A, double* res7) {
+  if (!c->kpath) return observables_of(c, u, A, res7);
+  CHKRET(ensure_obs(c, 1));
+  tdhf::ApplyArgs a = base_args(c);
+  a.mode = tdhf::M_OBS;
+  a.u = a.w = u;
+  a.A = A;
+  a.Aobs = A;
+  a.obs = c->d_obs;
+  a.obs_slot = 0;
+  CHKRET(launch_kspace(c, a));
+  CHKRET(launch_obs_reduce(c, c->d_obs, 1, 1, 0, c->d_res));
+  HIPCHK(c, hipMemcpyAsync(res7, c->d_res, 7 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  return sync(c);
+}
+
+// out = H[u] w on the path's layout.
+int path_hpsi(tdhf_ctx* c, const zd* u, const zd* w, double A, zd* out) {
+  tdhf::ApplyArgs a = base_args(c);
+  a.mode = tdhf::M_HPSI;
+  a.u = u;
+  a.w = w;
+  a.A = A;
+  a.Aobs = A;
+  a.out = out;
+  return launch_stage(c, a);
+}
+
+}  // namespace

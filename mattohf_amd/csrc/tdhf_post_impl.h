@@ -5,7 +5,7 @@
 namespace {
 
 int te_launch_update(tdhf_ctx* c, const zd* h, const zd* h2, double f, zd* w, zd* y) {
-  const size_t n = nstate(c);
+  const size_t n = path_count(c);
   hipLaunchKernelGGL(tdhf::te_update_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
                      c->stream, n, h, h2, f, w, y);
   HIPCHK(c, hipGetLastError());
@@ -15,11 +15,11 @@ int te_launch_update(tdhf_ctx* c, const zd* h, const zd* h2, double f, zd* w, zd
 // y += sum_{k=1..4} w_k, w_0 = x, w_k = -i dt H w_{k-1} / k with H = H[ua]
 // (or (H[ua] + H[ub])/2), as the order loops of src/RT_calculation.f90:71-151.
 int te_series(tdhf_ctx* c, const zd* ua, const zd* ub, const zd* x, double Aave, zd* y) {
-  const size_t bytes = nstate(c) * sizeof(zd);
+  const size_t bytes = path_count(c) * sizeof(zd);
   HIPCHK(c, hipMemcpyAsync(c->d_w, x, bytes, hipMemcpyDeviceToDevice, c->stream));
   for (int k = 1; k <= 4; ++k) {
-    CHKRET(tdhf::ctx_apply(c, ua, c->d_w, c->nb, Aave, c->d_out));
-    if (ub) CHKRET(tdhf::ctx_apply(c, ub, c->d_w, c->nb, Aave, c->d_ksum));
+    CHKRET(path_hpsi(c, ua, c->d_w, Aave, c->d_out));
+    if (ub) CHKRET(path_hpsi(c, ub, c->d_w, Aave, c->d_ksum));
     CHKRET(te_launch_update(c, c->d_out, ub ? c->d_ksum : nullptr, c->dt / (double)k, c->d_w, y));
   }
   return 0;
@@ -36,8 +36,9 @@ extern "C" int tdhf_te_step(tdhf_ctx* c, double* u, double Aave, int variant) {
   if (!c) return fail(nullptr, TDHF_EINVAL, "ctx is NULL");
   if (!u) return fail(c, TDHF_EINVAL, "NULL array");
   if (variant < 0 || variant > 2) return fail(c, TDHF_EINVAL, "unknown Taylor variant %d", variant);
-  const size_t bytes = nstate(c) * sizeof(zd);
-  CHKRET(upload(c, c->d_u0, u));
+  const size_t bytes = path_count(c) * sizeof(zd);
+  CHKRET(upload_state(c, c->d_u0, u));
+  c->u0_padded = c->kpath;
   // ubk0 in sa; the state accumulates in u0
   HIPCHK(c, hipMemcpyAsync(c->d_sa, c->d_u0, bytes, hipMemcpyDeviceToDevice, c->stream));
   if (variant == 0) {
@@ -49,14 +50,14 @@ extern "C" int tdhf_te_step(tdhf_ctx* c, double* u, double Aave, int variant) {
     if (variant == 1) {
       CHKRET(te_series(c, c->d_sa, c->d_sb, c->d_sa, Aave, c->d_u0));
     } else {
-      const size_t n = nstate(c);
+      const size_t n = path_count(c);
       hipLaunchKernelGGL(tdhf::te_mid_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
                          c->stream, n, c->d_sb, c->d_sa);
       HIPCHK(c, hipGetLastError());
       CHKRET(te_series(c, c->d_sb, nullptr, c->d_sa, Aave, c->d_u0));
     }
   }
-  return download(c, u, c->d_u0);
+  return download_state(c, u, c->d_u0);
 }
 
 extern "C" int tdhf_gs_run_diag(tdhf_ctx* c, double* u, int nscf, int ncg, double* etot_hist,
@@ -93,6 +94,7 @@ extern "C" int tdhf_gs_run_diag(tdhf_ctx* c, double* u, int nscf, int ncg, doubl
     return 0;
   };
   if ((rc = gs_flag_clear(c)) || (rc = upload(c, c->d_u0, u))) return done(rc);
+  c->u0_padded = false;
   double r[7];
   if ((rc = observables_of(c, c->d_u0, 0.0, r))) return done(rc);
   if (etot_hist) etot_hist[0] = r[0];

@@ -557,7 +557,8 @@ class Batch:
         return load().tdhf_batch_get_schedule(self.h)
 
     def set_exchange(self, mode):
-        """0: row-wise exchange; 1, 2, 3: pair tiles of 64, 32, 16 rows (NG=64,
+        """0: direct (row-wise exchange, or the density matrices of the k-points
+        for large batches); 1, 2, 3: pair tiles of 64, 32, 16 rows (NG=64,
         NB == NBocc)."""
         _bchk(load().tdhf_batch_set_exchange(self.h, int(mode)), self.h)
 
@@ -566,7 +567,7 @@ class Batch:
 
     @staticmethod
     def exchange_name(mode):
-        return "row-wise" if mode == 0 else f"pair tiles of {128 >> mode} rows"
+        return "direct" if mode == 0 else f"pair tiles of {128 >> mode} rows"
 
     def autotune(self, A, Aave):
         A = np.ascontiguousarray(A, dtype=np.float64)
