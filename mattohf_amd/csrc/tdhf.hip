@@ -520,7 +520,7 @@ int observables_of(tdhf_ctx* c, const zd* u, double A, double* res7) {
   a.obs = c->d_obs;
   a.obs_slot = 0;
   CHKRET(launch_apply(c, a, c->nb * c->nk));
-  hipLaunchKernelGGL(tdhf::obs_reduce_kernel, dim3(1), dim3(64), 0, c->stream, c->d_obs,
+  hipLaunchKernelGGL(tdhf::obs_reduce_kernel, dim3(1), dim3(256), 0, c->stream, c->d_obs,
                      c->obs_stride, c->nb * c->nk, 1, c->dv, c->vcell, c->d_res);
   HIPCHK(c, hipGetLastError());
   HIPCHK(c, hipMemcpyAsync(res7, c->d_res, 7 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -682,18 +682,6 @@ void release(tdhf_ctx* c) {
 // ground-state helpers shared with tdhf_gs.h
 // ---------------------------------------------------------------------------
 namespace tdhf {
-
-int ctx_apply(tdhf_ctx* c, const zd* u, const zd* w, int nbw, double A, zd* out) {
-  ApplyArgs a = base_args(c);
-  a.mode = M_HPSI;
-  a.u = u;
-  a.w = w;
-  a.nbw = nbw;
-  a.A = A;
-  a.Aobs = A;
-  a.out = out;
-  return launch_apply(c, a, nbw * c->nk);
-}
 
 int ctx_fail(tdhf_ctx* c, int code, const char* msg) { return fail(c, code, "%s", msg); }
 
@@ -934,7 +922,7 @@ int tdhf_rt_end(tdhf_ctx* c, double* etot, double* nele, double* jtot, double* i
   if (c->kpath) {
     CHKRET(launch_obs_reduce(c, c->d_obs, ns, 1, 0, c->d_res));
   } else {
-    hipLaunchKernelGGL(tdhf::obs_reduce_kernel, dim3((unsigned)((ns + 63) / 64)), dim3(64), 0,
+    hipLaunchKernelGGL(tdhf::obs_reduce_kernel, dim3((unsigned)((ns + 3) / 4)), dim3(256), 0,
                        c->stream, c->d_obs, c->obs_stride, rows, (int)ns, c->dv, c->vcell,
                        c->d_res);
     HIPCHK(c, hipGetLastError());
@@ -1043,9 +1031,7 @@ int tdhf_gram_schmidt(tdhf_ctx* c, double* u) {
   if (!c) return fail(nullptr, TDHF_EINVAL, "ctx is NULL");
   if (!u) return fail(c, TDHF_EINVAL, "NULL array");
   CHKRET(upload(c, c->d_sa, u));
-  hipLaunchKernelGGL(tdhf::gram_schmidt_kernel, dim3(c->nk), dim3(c->ng), 0, c->stream, c->d_sa,
-                     c->ng, c->nb, c->vcell);
-  HIPCHK(c, hipGetLastError());
+  CHKRET(launch_orth(c, c->d_sa, c->nb, 1, nullptr, 0));
   return download(c, u, c->d_sa);
 }
 

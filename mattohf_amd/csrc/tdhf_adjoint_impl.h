@@ -666,7 +666,7 @@ extern "C" int tdhf_fwd_batch(tdhf_ctx* c, int ntraj, double* u, int nt, const d
   CHKRET(adj_stage(c, s, a));
   if (s.kp) CHKRET(launch_obs_reduce(c, s.obs, nsl, ntraj, a.ostride, s.res));
   for (int t = 0; t < ntraj && !s.kp; ++t) {
-    hipLaunchKernelGGL(tdhf::obs_reduce_kernel, dim3((unsigned)((nsl + 63) / 64)), dim3(64), 0,
+    hipLaunchKernelGGL(tdhf::obs_reduce_kernel, dim3((unsigned)((nsl + 3) / 4)), dim3(256), 0,
                        c->stream, s.obs + (size_t)t * nsl * c->obs_stride, c->obs_stride,
                        c->nb * c->nk,
                        (int)nsl, c->dv, c->vcell, s.res + (size_t)t * nsl * 7);

@@ -935,7 +935,7 @@ int tdhf_batch_propagate(tdhf_batch* b, int nt, const double* A, const double* A
                        (const double*)nullptr, b->d_td, b->p.ng, ns, n, dv, vcell, (size_t)0,
                        b->d_res);
   else
-    hipLaunchKernelGGL(tdhf::obs_reduce_batch_kernel, dim3((n + 63) / 64), dim3(64), 0, b->stream,
+    hipLaunchKernelGGL(tdhf::obs_reduce_batch_kernel, dim3((n + 3) / 4), dim3(256), 0, b->stream,
                        b->d_td, b->ntraj, b->p.nb, ns, dv, vcell, b->d_res);
   BHIP(b, hipGetLastError());
   std::vector<double> res((size_t)7 * n);

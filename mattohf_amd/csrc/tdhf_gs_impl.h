@@ -9,9 +9,11 @@ namespace tdhf {
 void gs_free(GsWork& g) {
   if (g.W) (void)hipFree(g.W);
   if (g.HW) (void)hipFree(g.HW);
+  if (g.KW) (void)hipFree(g.KW);
+  if (g.KH) (void)hipFree(g.KH);
   if (g.eps) (void)hipFree(g.eps);
   if (g.nonconv) (void)hipFree(g.nonconv);
-  g.W = g.HW = nullptr;
+  g.W = g.HW = g.KW = g.KH = nullptr;
   g.eps = nullptr;
   g.nonconv = nullptr;
   g.ncg = 0;
@@ -27,6 +29,10 @@ int gs_alloc(tdhf_ctx* c, int ncg) {
   const size_t n = nstate(c) * (size_t)ncg;
   CHKRET(dalloc(c, &c->gs.W, n));
   CHKRET(dalloc(c, &c->gs.HW, n));
+  if (c->kpath) {
+    CHKRET(dalloc(c, &c->gs.KW, kcount(c) * (size_t)ncg));
+    CHKRET(dalloc(c, &c->gs.KH, kcount(c) * (size_t)ncg));
+  }
   CHKRET(dalloc(c, &c->gs.eps, (size_t)c->nb * c->nk * 2));
   CHKRET(dalloc(c, &c->gs.nonconv, 1));
   c->gs.ncg = ncg;
@@ -51,48 +57,131 @@ int gs_flag_check(tdhf_ctx* c) {
   return 0;
 }
 
-int launch_gs_orth(tdhf_ctx* c, zd* u) {
-  hipLaunchKernelGGL(tdhf::gram_schmidt_kernel, dim3(c->nk), dim3(c->ng), 0, c->stream, u, c->ng,
-                     c->nb, c->vcell);
+// Gram-Schmidt of m columns per k-point, npass passes, in place and to copy
+// (ldc columns per k-point).  One wave per column, up to sixteen.
+int launch_orth(tdhf_ctx* c, zd* w, int m, int npass, zd* copy, int ldc) {
+  const size_t lds = tdhf::orth_lds(c->ng, m);
+  if (lds > 160 * 1024) {  // more bands than LDS holds (one pass only)
+    if (npass != 1 || copy) return fail(c, TDHF_EINVAL, "%d columns do not fit LDS", m);
+    hipLaunchKernelGGL(tdhf::gram_schmidt_kernel, dim3(c->nk), dim3(c->ng), 0, c->stream, w, c->ng,
+                       m, c->vcell);
+    HIPCHK(c, hipGetLastError());
+    return 0;
+  }
+  if (lds > 64 * 1024)
+    HIPCHK(c, hipFuncSetAttribute((const void*)tdhf::orth_kernel,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+  hipLaunchKernelGGL(tdhf::orth_kernel, dim3(c->nk), dim3(64 * std::min(m, 16)), lds, c->stream, w,
+                     c->ng, m, c->dv, npass, copy, ldc);
   HIPCHK(c, hipGetLastError());
   return 0;
 }
 
-int launch_rr(tdhf_ctx* c, const zd* W, const zd* HW, size_t blk, int m, zd* uout) {
-  const size_t lds = (size_t)2 * m * m * sizeof(zd) + (size_t)m * sizeof(int) + 16;
-  if (lds > 48 * 1024)
-    HIPCHK(c, hipFuncSetAttribute((const void*)tdhf::rr_kernel,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL(tdhf::rr_kernel, dim3(c->nk), dim3(256), lds, c->stream, W, HW, blk, c->ng,
-                     c->nb, m, c->dv, uout, (double*)nullptr, c->gs.nonconv);
+int launch_rr(tdhf_ctx* c, const zd* W, const zd* HW, int m, zd* uout) {
+  const bool wl = tdhf::rr_lds(c->ng, m, true) <= 160 * 1024;
+  const size_t lds = tdhf::rr_lds(c->ng, m, wl);
+  const void* fn =
+      wl ? (const void*)tdhf::rr_kernel<true> : (const void*)tdhf::rr_kernel<false>;
+  if (lds > 64 * 1024)
+    HIPCHK(c, hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+  if (wl)
+    hipLaunchKernelGGL(tdhf::rr_kernel<true>, dim3(c->nk), dim3(256), lds, c->stream, W, HW, c->ng,
+                       c->nb, m, c->dv, uout, c->gs.nonconv);
+  else
+    hipLaunchKernelGGL(tdhf::rr_kernel<false>, dim3(c->nk), dim3(256), lds, c->stream, W, HW,
+                       c->ng, c->nb, m, c->dv, uout, c->gs.nonconv);
   HIPCHK(c, hipGetLastError());
   return 0;
 }
 
-// KS_ubk2_SVD (src/GS_calculation.f90:124-194) on the state in d_u0.
+// H of the orbitals u (NG,NB,NK) at A = 0, for the gs_product calls after it:
+// on the density-matrix path its matrices are made once.
+int gs_hamiltonian(tdhf_ctx* c, const zd* u) {
+  if (!c->kpath) return 0;
+  CHKRET(kspace_layout(c, u, c->d_sa, true));
+  tdhf::ApplyArgs a = base_args(c);
+  a.mode = tdhf::M_HPSI;
+  a.u = a.w = c->d_sa;
+  tdhf::KArgs k = kspace_args(c, a);
+  return launch_kmat(c, k, 1, c->stream);
+}
+
+// out = H[u] w for nbw columns per k-point, w and out held in ld columns per
+// k-point; u is that of the gs_hamiltonian call before.
+int gs_product(tdhf_ctx* c, const zd* u, const zd* w, int nbw, int ld, zd* out) {
+  tdhf::ApplyArgs a = base_args(c);
+  a.mode = tdhf::M_HPSI;
+  a.nbw = nbw;
+  if (!c->kpath) {
+    a.wld = ld;
+    a.u = u;
+    a.w = w;
+    a.out = out;
+    return launch_apply(c, a, nbw * c->nk);
+  }
+  CHKRET(kspace_layout(c, w, c->gs.KW, true, 1, nullptr, nbw, ld));
+  a.u = c->d_sa;
+  a.w = c->gs.KW;
+  a.out = c->gs.KH;
+  tdhf::KArgs k = kspace_args(c, a);
+  CHKRET(launch_kapply(c, k, 1, c->stream));
+  return kspace_layout(c, c->gs.KH, out, false, 1, nullptr, nbw, ld);
+}
+
+// KS_ubk2_SVD (src/GS_calculation.f90:124-194) on the state in d_u0, which is
+// orthonormalised first (Gram_Schmidt).
 int gs_krylov(tdhf_ctx* c, int ncg) {
-  const size_t blk = nstate(c);
-  zd* W = c->gs.W;
-  zd* HW = c->gs.HW;
-  HIPCHK(c, hipMemcpyAsync(W, c->d_u0, blk * sizeof(zd), hipMemcpyDeviceToDevice, c->stream));
-  for (int icg = 1; icg < ncg; ++icg)
-    CHKRET(tdhf::ctx_apply(c, c->d_u0, W + (icg - 1) * blk, c->nb, 0.0, W + icg * blk));
   const int m = c->nb * ncg;
-  hipLaunchKernelGGL(tdhf::orth_kernel, dim3(c->nk), dim3(c->ng), 0, c->stream, W, blk, c->ng,
-                     c->nb, m, c->dv);
-  HIPCHK(c, hipGetLastError());
-  for (int icg = 0; icg < ncg; ++icg)
-    CHKRET(tdhf::ctx_apply(c, c->d_u0, W + icg * blk, c->nb, 0.0, HW + icg * blk));
-  return launch_rr(c, W, HW, blk, m, c->d_u0);
+  const size_t blk = (size_t)c->ng * c->nb;  // columns of a Krylov block start here at each k
+  zd* W = c->gs.W;
+  CHKRET(launch_orth(c, c->d_u0, c->nb, 1, W, m));
+  CHKRET(gs_hamiltonian(c, c->d_u0));
+  for (int icg = 1; icg < ncg; ++icg)
+    CHKRET(gs_product(c, c->d_u0, W + (icg - 1) * blk, c->nb, m, W + icg * blk));
+  CHKRET(launch_orth(c, W, m, 2, nullptr, 0));
+  CHKRET(gs_product(c, c->d_u0, W, m, m, c->gs.HW));
+  return launch_rr(c, W, c->gs.HW, m, c->d_u0);
 }
 
-// Subspace_diag (src/GS_calculation.f90:197-237) on the state in d_u0.
+// Gram_Schmidt and Subspace_diag (src/GS_calculation.f90:197-237) on the state
+// in d_u0.
 int gs_subspace(tdhf_ctx* c) {
-  const size_t blk = nstate(c);
-  CHKRET(tdhf::ctx_apply(c, c->d_u0, c->d_u0, c->nb, 0.0, c->gs.HW));
-  HIPCHK(c, hipMemcpyAsync(c->gs.W, c->d_u0, blk * sizeof(zd), hipMemcpyDeviceToDevice,
+  CHKRET(launch_orth(c, c->d_u0, c->nb, 1, c->gs.W, c->nb));
+  CHKRET(gs_hamiltonian(c, c->d_u0));
+  CHKRET(gs_product(c, c->d_u0, c->d_u0, c->nb, c->nb, c->gs.HW));
+  return launch_rr(c, c->gs.W, c->gs.HW, c->nb, c->d_u0);
+}
+
+// Observables at A = 0 of the state in d_u0 (host layout) into slot 'slot'.
+int gs_observe(tdhf_ctx* c, long slot) {
+  tdhf::ApplyArgs a = base_args(c);
+  a.mode = tdhf::M_OBS;
+  a.u = a.w = c->d_u0;
+  a.obs = c->d_obs;
+  a.obs_slot = (int)slot;
+  if (!c->kpath) return launch_apply(c, a, c->nb * c->nk);
+  CHKRET(kspace_layout(c, c->d_u0, c->d_sa, true));
+  a.u = a.w = c->d_sa;
+  return launch_kspace(c, a);
+}
+
+// Energies of slots s0 .. s0 + n - 1.
+int gs_energies(tdhf_ctx* c, long s0, long n, double* e) {
+  const size_t stride = c->kpath ? tdhf::kspace_obs_stride(c->ng) : c->obs_stride;
+  if (c->kpath) {
+    CHKRET(launch_obs_reduce(c, c->d_obs + stride * s0, n, 1, 0, c->d_res));
+  } else {
+    hipLaunchKernelGGL(tdhf::obs_reduce_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0,
+                       c->stream, c->d_obs + stride * s0, c->obs_stride, c->nb * c->nk, (int)n,
+                       c->dv, c->vcell, c->d_res);
+    HIPCHK(c, hipGetLastError());
+  }
+  std::vector<double> r((size_t)7 * n);
+  HIPCHK(c, hipMemcpyAsync(r.data(), c->d_res, r.size() * sizeof(double), hipMemcpyDeviceToHost,
                            c->stream));
-  return launch_rr(c, c->gs.W, c->gs.HW, blk, c->nb, c->d_u0);
+  CHKRET(sync(c));
+  for (long i = 0; i < n; ++i) e[i] = r[(size_t)7 * i];
+  return 0;
 }
 
 }  // namespace
@@ -108,27 +197,35 @@ extern "C" int tdhf_gs_run(tdhf_ctx* c, double* u, int nscf, int ncg, double tol
   CHKRET(gs_flag_clear(c));
   CHKRET(upload(c, c->d_u0, u));
   c->u0_padded = false;
-  double r[7];
-  CHKRET(observables_of(c, c->d_u0, 0.0, r));
-  double eprev = r[0];
-  if (etot_hist) etot_hist[0] = eprev;
-  int it = 0;
+  // the energies are read as they come where the loop may end on them, else
+  // after it
+  const bool each = tol > 0.0;
+  const long slots = each ? 2 : (long)nscf + 1;
+  std::vector<double> eh((size_t)nscf + 1);
+  CHKRET(ensure_obs(c, slots));
+  CHKRET(gs_observe(c, 0));
+  if (each) CHKRET(gs_energies(c, 0, 1, &eh[0]));
+  int it = 0, last = nscf;
   for (it = 1; it <= nscf; ++it) {
-    CHKRET(launch_gs_orth(c, c->d_u0));
     CHKRET(gs_krylov(c, ncg));
-    CHKRET(launch_gs_orth(c, c->d_u0));
     CHKRET(gs_subspace(c));
-    CHKRET(observables_of(c, c->d_u0, 0.0, r));
-    if (etot_hist) etot_hist[it] = r[0];
-    if (!std::isfinite(r[0])) return fail(c, TDHF_ENUMERIC, "GS energy is not finite at iteration %d", it);
-    const bool conv = tol > 0.0 && std::fabs(r[0] - eprev) < tol;
-    eprev = r[0];
-    if (conv) break;
+    CHKRET(gs_observe(c, each ? 0 : it));
+    if (!each) continue;
+    CHKRET(gs_energies(c, 0, 1, &eh[it]));
+    last = it;
+    if (!std::isfinite(eh[it]) || std::fabs(eh[it] - eh[it - 1]) < tol) break;
+  }
+  if (!each) CHKRET(gs_energies(c, 0, slots, eh.data()));
+  for (int i = 0; i <= last; ++i) {
+    if (etot_hist) etot_hist[i] = eh[i];
+    if (i > 0 && !std::isfinite(eh[i]))
+      return fail(c, TDHF_ENUMERIC, "GS energy is not finite at iteration %d", i);
   }
   CHKRET(gs_flag_check(c));
   if (niter) *niter = it > nscf ? nscf : it;
   if (epsbk || epserr) {
-    CHKRET(tdhf::ctx_apply(c, c->d_u0, c->d_u0, c->nb, 0.0, c->gs.HW));
+    CHKRET(gs_hamiltonian(c, c->d_u0));
+    CHKRET(gs_product(c, c->d_u0, c->d_u0, c->nb, c->nb, c->gs.HW));
     const int rows = c->nb * c->nk;
     hipLaunchKernelGGL(tdhf::epsbk_kernel, dim3(rows), dim3(c->ng), 0, c->stream, c->d_u0,
                        c->gs.HW, c->ng, c->dv, c->gs.eps, c->gs.eps + rows);

@@ -76,6 +76,7 @@ struct TrajDesc {
 // Offsets inside one observables slot: rows*3 partials then (N, Eion, EH).
 struct ApplyArgs {
   int nk, nb, nbocc, nbw;  // nbw = columns of w / out per k-point
+  int wld;                  // columns per k-point w and out are held in (0: nbw)
   double bx, dv, occ, dt;
   double A, Aobs;           // used when Aarr == nullptr
   const double* Aarr;       // per-step A(it), or nullptr
@@ -334,7 +335,7 @@ __global__ void __launch_bounds__(512) apply_kernel(ApplyArgs a) {
   // first wait, so the loop starts after one memory round trip: the lane
   // twiddles, the first u(q,j), then w of this row and the kinetic kernels,
   // which go to LDS ----
-  const size_t o = (size_t)NG * row + (tid < NG ? tid : 0);
+  const size_t o = (size_t)NG * (a.wld ? ib + a.wld * ik : row) + (tid < NG ? tid : 0);
   F fft;
   fft.init(a.tw, l);
 
@@ -719,16 +720,40 @@ struct CompSum {
   __device__ __forceinline__ double value() const { return s + c; }
 };
 
+// Adds the sums of the 64 lanes of a wave, compensated and in a fixed order;
+// the same in every lane.
+__device__ __forceinline__ void comp_wave_sum(CompSum& c) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const double os = __shfl_xor(c.s, off), oc = __shfl_xor(c.c, off);
+    // the same pair of operands in both lanes of the exchange
+    const double lo = (lane & off) ? os : c.s, hi = (lane & off) ? c.s : os;
+    CompSum r;
+    r.add(lo);
+    r.add(hi);
+    r.c += c.c + oc;
+    c = r;
+  }
+}
+
 // Sums the per-row partials of one observables slot p (rows rows) into
-// (Etot, N, J, Ekin, Eion, EH, Ex), src/Functions.f90:74-91 and :289-318.
+// (Etot, N, J, Ekin, Eion, EH, Ex), src/Functions.f90:74-91 and :289-318; one
+// wave per slot, rows lane, lane + 64, ... of a lane first (one thread per slot
+// took 78 us for 256 rows, one wave 5 us).
 __device__ __forceinline__ void obs_reduce_slot(const double* p, int rows, double dv, double vcell,
                                                 double* o) {
+  const int lane = threadIdx.x & 63;
   CompSum ek, jj, ex;
-  for (int r = 0; r < rows; ++r) {
+  for (int r = lane; r < rows; r += 64) {
     ek.add(p[3 * r + 0]);
     jj.add(p[3 * r + 1]);
     ex.add(p[3 * r + 2]);
   }
+  comp_wave_sum(ek);
+  comp_wave_sum(jj);
+  comp_wave_sum(ex);
+  if (lane != 0) return;
   const double n = p[3 * rows + 0], ei = p[3 * rows + 1], eh = p[3 * rows + 2];
   CompSum et;
   et.add(ek.s);
@@ -746,17 +771,20 @@ __device__ __forceinline__ void obs_reduce_slot(const double* p, int rows, doubl
   o[6] = 0.5 * ex.value();
 }
 
-__global__ void obs_reduce_kernel(const double* obs, int stride, int rows, int nslots, double dv,
-                                  double vcell, double* out) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+// Four waves (slots) per workgroup.
+__global__ void __launch_bounds__(256) obs_reduce_kernel(const double* obs, int stride, int rows,
+                                                         int nslots, double dv, double vcell,
+                                                         double* out) {
+  const int s = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (s >= nslots) return;
   obs_reduce_slot(obs + (size_t)s * stride, rows, dv, vcell, out + (size_t)7 * s);
 }
 
-// Batched variant: one thread per (trajectory, slot); out[(t*nslots + s)*7].
-__global__ void obs_reduce_batch_kernel(const TrajDesc* td, int ntraj, int nb, int nslots,
-                                        double dv, double vcell, double* out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// Batched variant: one wave per (trajectory, slot); out[(t*nslots + s)*7].
+__global__ void __launch_bounds__(256) obs_reduce_batch_kernel(const TrajDesc* td, int ntraj,
+                                                               int nb, int nslots, double dv,
+                                                               double vcell, double* out) {
+  const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (i >= ntraj * nslots) return;
   const int t = i / nslots, s = i - t * nslots;
   obs_reduce_slot(td[t].obs + (size_t)s * td[t].obs_stride, nb * td[t].nk, dv, vcell,
@@ -832,6 +860,7 @@ __global__ void ion_kernel(int ng, int nk, double ax, int nion, const double* z,
   if (x < ng) vion[x] = v - top;
 }
 
+// Gram_Schmidt for more bands than orth_kernel holds in LDS.
 // Block-wide deterministic sum over blockDim.x (power of two, <= 128).
 __device__ __forceinline__ double block_sum(double v, double* red) {
   const int t = threadIdx.x;

@@ -803,6 +803,7 @@ struct KLayoutArgs {
   const zd* src;
   zd* dst;
   int ng, nb, nk, n;
+  int ld;                   // columns per k-point of the (NG,.,NK) side (0: nb)
   size_t sstride, dstride;  // per trajectory (grid z = trajectory * nb + band)
   // batch: offsets and k-meshes of the trajectories instead
   const TrajDesc* td;
@@ -814,7 +815,7 @@ struct KLayoutArgs {
 // 16 x 16 tiles through LDS, so that both sides move 256-byte runs.
 __global__ void __launch_bounds__(256) kspace_layout_kernel(KLayoutArgs a) {
   __shared__ zd s[16][17];
-  const int tr = blockIdx.z / a.nb, b = blockIdx.z - tr * a.nb;
+  const int tr = blockIdx.z / a.nb, b = blockIdx.z - tr * a.nb, ld = a.ld ? a.ld : a.nb;
   int nk = a.nk, n = a.n;
   size_t ro = a.to_k ? tr * a.sstride : tr * a.dstride;
   size_t ko = a.to_k ? tr * a.dstride : tr * a.sstride;
@@ -829,7 +830,7 @@ __global__ void __launch_bounds__(256) kspace_layout_kernel(KLayoutArgs a) {
   const int p = threadIdx.x & 15, q = threadIdx.x >> 4;
   if (a.to_k) {
     const int k = k0 + q;
-    s[q][p] = k < nk ? a.src[ro + (size_t)(x0 + p) + (size_t)a.ng * (b + (size_t)a.nb * k)]
+    s[q][p] = k < nk ? a.src[ro + (size_t)(x0 + p) + (size_t)a.ng * (b + (size_t)ld * k)]
                      : mk(0.0, 0.0);
     __syncthreads();
     a.dst[ko + ((size_t)(x0 + q) * a.nb + b) * n + k0 + p] = s[p][q];
@@ -837,7 +838,7 @@ __global__ void __launch_bounds__(256) kspace_layout_kernel(KLayoutArgs a) {
     s[q][p] = a.src[ko + ((size_t)(x0 + q) * a.nb + b) * n + k0 + p];
     __syncthreads();
     const int k = k0 + q;
-    if (k < nk) a.dst[ro + (size_t)(x0 + p) + (size_t)a.ng * (b + (size_t)a.nb * k)] = s[p][q];
+    if (k < nk) a.dst[ro + (size_t)(x0 + p) + (size_t)a.ng * (b + (size_t)ld * k)] = s[p][q];
   }
 }
 
@@ -860,18 +861,7 @@ __global__ void __launch_bounds__(256) kspace_obs_reduce_kernel(const double* ob
   CompSum c[6];
   for (int x = lane; x < ng; x += 64)
     for (int m = 0; m < 6; ++m) c[m].add(p[6 * x + m]);
-#pragma unroll
-  for (int m = 0; m < 6; ++m)
-    for (int off = 1; off < 64; off <<= 1) {
-      const double os = __shfl_xor(c[m].s, off), oc = __shfl_xor(c[m].c, off);
-      // the same pair of operands in both lanes of the exchange
-      const double lo = (lane & off) ? os : c[m].s, hi = (lane & off) ? c[m].s : os;
-      CompSum r;
-      r.add(lo);
-      r.add(hi);
-      r.c += c[m].c + oc;
-      c[m] = r;
-    }
+  for (int m = 0; m < 6; ++m) comp_wave_sum(c[m]);
   if (lane == 0) {
     CompSum et;
     et.add(c[0].s);

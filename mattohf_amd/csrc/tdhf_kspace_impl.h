@@ -181,6 +181,8 @@ tdhf::KArgs kspace_args(const tdhf_ctx* c, const tdhf::ApplyArgs& a) {
   k.n = c->kn;
   k.nchunk = kspace_chunks(a.nbw);
   k.ktab = c->d_ktab;
+  k.hm = c->d_hm;
+  k.nx = c->d_nx;
   k.tw[kspace_class(c->kn)] = c->d_ktw;
   k.om[kspace_class(c->kn)] = c->d_om;
   return k;
@@ -193,13 +195,37 @@ struct KScratch {
   size_t hstride, nstride;
 };
 
+// The matrices of the states a.u.
+int launch_kmat(tdhf_ctx* c, tdhf::KArgs& k, int ntraj, hipStream_t s) {
+  void* args[] = {&k};
+  const bool obs = k.a.mode == tdhf::M_S1 || k.a.mode == tdhf::M_OBS;
+  const long tasks = (long)tdhf::kmat_tasks(c->ng, kspace_gpw(c->kn)) * ntraj;
+  const int wa = kmat_waves(tasks);
+  HIPCHK(c, hipLaunchKernel(kmat_fn_for(c->kn, obs, kmat_deep(tasks)),
+                            dim3(kmat_groups(c->kn, c->ng, wa), ntraj), dim3(64 * wa), args,
+                            kmat_lds_for(c->kn, wa, c->ng), s));
+  return 0;
+}
+// Their product with the columns a.w and the stage update.
+int launch_kapply(tdhf_ctx* c, tdhf::KArgs& k, int ntraj, hipStream_t s) {
+  void* args[] = {&k};
+  const int wb = kapply_waves(c->kn, c->ng), nbt = kspace_nbt(k.a.nbw);
+  const int xt = kapply_points((long)kapply_groups(c->kn, c->ng, k.a.nbw, 1) * ntraj);
+  HIPCHK(c, hipLaunchKernel(kapply_fn(nbt, xt),
+                            dim3(kapply_groups(c->kn, c->ng, k.a.nbw, xt), ntraj), dim3(64 * wb),
+                            args, tdhf::kapply_lds(wb, nbt, xt), s));
+  return 0;
+}
+
 int launch_kspace(tdhf_ctx* c, const tdhf::ApplyArgs& a, int ntraj = 1,
                   hipStream_t st = nullptr, const KScratch* sc = nullptr) {
   tdhf::KArgs k = kspace_args(c, a);
-  k.hm = sc ? sc->hm : c->d_hm;
-  k.nx = sc ? sc->nx : c->d_nx;
-  k.hstride = sc ? sc->hstride : 0;
-  k.nstride = sc ? sc->nstride : 0;
+  if (sc) {
+    k.hm = sc->hm;
+    k.nx = sc->nx;
+    k.hstride = sc->hstride;
+    k.nstride = sc->nstride;
+  }
   const bool timed = c->timing && !st;
   hipStream_t s = st ? st : c->stream;
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -207,18 +233,8 @@ int launch_kspace(tdhf_ctx* c, const tdhf::ApplyArgs& a, int ntraj = 1,
     CHKRET(take_events(c, &e0, &e1));
     HIPCHK(c, hipEventRecord(e0, c->stream));
   }
-  const bool obs = a.mode == tdhf::M_S1 || a.mode == tdhf::M_OBS;
-  void* args[] = {&k};
-  const long tasks = (long)tdhf::kmat_tasks(c->ng, kspace_gpw(c->kn)) * ntraj;
-  const int wa = kmat_waves(tasks);
-  HIPCHK(c, hipLaunchKernel(kmat_fn_for(c->kn, obs, kmat_deep(tasks)),
-                            dim3(kmat_groups(c->kn, c->ng, wa), ntraj), dim3(64 * wa), args,
-                            kmat_lds_for(c->kn, wa, c->ng), s));
-  const int wb = kapply_waves(c->kn, c->ng), nbt = kspace_nbt(a.nbw);
-  const int xt = kapply_points((long)kapply_groups(c->kn, c->ng, a.nbw, 1) * ntraj);
-  HIPCHK(c, hipLaunchKernel(kapply_fn(nbt, xt),
-                            dim3(kapply_groups(c->kn, c->ng, a.nbw, xt), ntraj), dim3(64 * wb),
-                            args, tdhf::kapply_lds(wb, nbt, xt), s));
+  CHKRET(launch_kmat(c, k, ntraj, s));
+  CHKRET(launch_kapply(c, k, ntraj, s));
   if (timed) HIPCHK(c, hipEventRecord(e1, c->stream));
   return 0;
 }
@@ -228,20 +244,23 @@ int launch_stage(tdhf_ctx* c, const tdhf::ApplyArgs& a) {
   return c->kpath ? launch_kspace(c, a) : launch_apply(c, a, c->nb * c->nk);
 }
 
-// dst = src in the other layout, for ntraj states back to back.
+// dst = src in the other layout, for ntraj states back to back (or nb columns
+// per k-point, held in ld on the host layout's side).
 int kspace_layout(tdhf_ctx* c, const zd* src, zd* dst, bool to_k, int ntraj = 1,
-                  hipStream_t st = nullptr) {
+                  hipStream_t st = nullptr, int nb = 0, int ld = 0) {
+  if (nb == 0) nb = c->nb;
   tdhf::KLayoutArgs l{};
   l.src = src;
   l.dst = dst;
   l.ng = c->ng;
-  l.nb = c->nb;
+  l.nb = nb;
+  l.ld = ld;
   l.nk = c->nk;
   l.n = c->kn;
   l.sstride = to_k ? nstate(c) : kcount(c);
   l.dstride = to_k ? kcount(c) : nstate(c);
   l.to_k = to_k;
-  hipLaunchKernelGGL(tdhf::kspace_layout_kernel, dim3(c->ng / 16, c->kn / 16, c->nb * ntraj),
+  hipLaunchKernelGGL(tdhf::kspace_layout_kernel, dim3(c->ng / 16, c->kn / 16, nb * ntraj),
                      dim3(256), 0, st ? st : c->stream, l);
   HIPCHK(c, hipGetLastError());
   return 0;

@@ -83,7 +83,8 @@ extern "C" int tdhf_gs_run_diag(tdhf_ctx* c, double* u, int nscf, int ncg, doubl
     return r;
   };
   auto step_diag = [&](int mode, int it) -> int {
-    CHKRET(tdhf::ctx_apply(c, c->d_u0, c->d_u0, c->nb, 0.0, c->gs.HW));
+    CHKRET(gs_hamiltonian(c, c->d_u0));
+    CHKRET(gs_product(c, c->d_u0, c->d_u0, c->nb, c->nb, c->gs.HW));
     hipLaunchKernelGGL(tdhf::epsbk_kernel, dim3(rows), dim3(c->ng), 0, c->stream, c->d_u0,
                        c->gs.HW, c->ng, c->dv, c->gs.eps, c->gs.eps + rows);
     HIPCHK(c, hipGetLastError());
@@ -95,15 +96,13 @@ extern "C" int tdhf_gs_run_diag(tdhf_ctx* c, double* u, int nscf, int ncg, doubl
   };
   if ((rc = gs_flag_clear(c)) || (rc = upload(c, c->d_u0, u))) return done(rc);
   c->u0_padded = false;
-  double r[7];
-  if ((rc = observables_of(c, c->d_u0, 0.0, r))) return done(rc);
+  double r[1];
+  if ((rc = ensure_obs(c, 1)) || (rc = gs_observe(c, 0)) || (rc = gs_energies(c, 0, 1, r))) return done(rc);
   if (etot_hist) etot_hist[0] = r[0];
   if ((rc = step_diag(0, 0))) return done(rc);
   for (int it = 1; it <= nscf; ++it) {
-    if ((rc = launch_gs_orth(c, c->d_u0)) || (rc = gs_krylov(c, ncg)) ||
-        (rc = launch_gs_orth(c, c->d_u0)) || (rc = gs_subspace(c)))
-      return done(rc);
-    if ((rc = observables_of(c, c->d_u0, 0.0, r))) return done(rc);
+    if ((rc = gs_krylov(c, ncg)) || (rc = gs_subspace(c))) return done(rc);
+    if ((rc = gs_observe(c, 0)) || (rc = gs_energies(c, 0, 1, r))) return done(rc);
     if (etot_hist) etot_hist[it] = r[0];
     if (!std::isfinite(r[0]))
       return done(fail(c, TDHF_ENUMERIC, "GS energy is not finite at iteration %d", it));
