@@ -197,32 +197,34 @@ extern "C" int tdhf_gs_run(tdhf_ctx* c, double* u, int nscf, int ncg, double tol
   CHKRET(gs_flag_clear(c));
   CHKRET(upload(c, c->d_u0, u));
   c->u0_padded = false;
-  // the energies are read as they come where the loop may end on them, else
-  // after it
+  // the energies are read one by one where the loop may end on them, else 256 at
+  // a time (a read waits for the iteration: 20 us of an idle device)
   const bool each = tol > 0.0;
-  const long slots = each ? 2 : (long)nscf + 1;
-  std::vector<double> eh((size_t)nscf + 1);
-  CHKRET(ensure_obs(c, slots));
-  CHKRET(gs_observe(c, 0));
-  if (each) CHKRET(gs_energies(c, 0, 1, &eh[0]));
-  int it = 0, last = nscf;
-  for (it = 1; it <= nscf; ++it) {
+  const int cap = each ? 1 : std::min(nscf, 255) + 1;
+  double e[256], eprev = 0.0;
+  CHKRET(ensure_obs(c, cap));
+  int it = 0;
+  for (int n = 0;; ++it) {
+    CHKRET(gs_observe(c, n++));
+    bool conv = false;
+    if (n == cap || it == nscf) {
+      CHKRET(gs_energies(c, 0, n, e));
+      for (int i = 0; i < n; ++i) {
+        const int at = it + 1 - n + i;
+        if (etot_hist) etot_hist[at] = e[i];
+        if (at > 0 && !std::isfinite(e[i]))
+          return fail(c, TDHF_ENUMERIC, "GS energy is not finite at iteration %d", at);
+      }
+      conv = each && it > 0 && std::fabs(e[0] - eprev) < tol;
+      eprev = e[0];
+      n = 0;
+    }
+    if (conv || it == nscf) break;
     CHKRET(gs_krylov(c, ncg));
     CHKRET(gs_subspace(c));
-    CHKRET(gs_observe(c, each ? 0 : it));
-    if (!each) continue;
-    CHKRET(gs_energies(c, 0, 1, &eh[it]));
-    last = it;
-    if (!std::isfinite(eh[it]) || std::fabs(eh[it] - eh[it - 1]) < tol) break;
-  }
-  if (!each) CHKRET(gs_energies(c, 0, slots, eh.data()));
-  for (int i = 0; i <= last; ++i) {
-    if (etot_hist) etot_hist[i] = eh[i];
-    if (i > 0 && !std::isfinite(eh[i]))
-      return fail(c, TDHF_ENUMERIC, "GS energy is not finite at iteration %d", i);
   }
   CHKRET(gs_flag_check(c));
-  if (niter) *niter = it > nscf ? nscf : it;
+  if (niter) *niter = it;
   if (epsbk || epserr) {
     CHKRET(gs_hamiltonian(c, c->d_u0));
     CHKRET(gs_product(c, c->d_u0, c->d_u0, c->nb, c->nb, c->gs.HW));
