@@ -69,6 +69,19 @@ __device__ __forceinline__ void gstore(zd* p, zd v) {
 }
 __device__ __forceinline__ void gstore(double* p, double v) { *(TDHF_GLOBAL double*)(p) = v; }
 
+// Zero in a vector register whose value the compiler does not know.  An address
+// that it is added to is loaded through the vector memory path although every
+// lane's is the same: scalar loads return out of order, so waiting for one, or
+// for an LDS access, waits for all of them.
+__device__ __forceinline__ int lane_zero() {
+  int z;
+  asm("v_mov_b32 %0, 0" : "=v"(z));
+  return z;
+}
+__device__ __forceinline__ int gload_lanes(const int* p, int zero) {
+  return *(const TDHF_GLOBAL int*)(p + zero);
+}
+
 template <int B, int E, typename F>
 __device__ __forceinline__ void static_for(F&& f) {
   if constexpr (B < E) {
@@ -208,6 +221,21 @@ struct GroupFFT {
       static_for<0, R>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         iw[i] = gload(tw + NG + l * R + i);
+      });
+    }
+  }
+
+  // The same from a copy of the table's first TWL entries in LDS.
+  static constexpr int TWL = Q > 1 ? 2 * NG : NG;
+  __device__ __forceinline__ void init_lds(const zd* tw, int l) {
+    static_for<0, R>([&](auto gc) {
+      constexpr int g0 = decltype(gc)::value;
+      fw[g0] = tw[l * R + g0];
+    });
+    if constexpr (Q > 1) {
+      static_for<0, R>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        iw[i] = tw[NG + l * R + i];
       });
     }
   }
@@ -357,6 +385,19 @@ struct GroupFFT<128> {
     static_for<0, 4>([&](auto hc) {
       constexpr int h = decltype(hc)::value;
       fq[h] = gload(tw + 128 + (l & 3) * 4 + h);
+    });
+  }
+
+  // The same from a copy of the table's first TWL entries in LDS.
+  static constexpr int TWL = 144;
+  __device__ __forceinline__ void init_lds(const zd* tw, int l) {
+    static_for<0, 8>([&](auto gc) {
+      constexpr int g0 = decltype(gc)::value;
+      fw[g0] = tw[l * 8 + g0];
+    });
+    static_for<0, 4>([&](auto hc) {
+      constexpr int h = decltype(hc)::value;
+      fq[h] = tw[128 + (l & 3) * 4 + h];
     });
   }
 

@@ -153,6 +153,24 @@ __device__ __forceinline__ double pair_sum_bit2(double x, double y, bool bit) {
   return keep + __shfl_xor(send, 4);
 }
 
+// Sum of v over the 64 lanes of a wave, the same in every lane, without LDS:
+// DPP within 16 lanes (lane ^ 1, ^ 2, then mirrors, which act as ^ 4 and ^ 8
+// once the quads and half rows are equal), permlane swaps across them.
+__device__ __forceinline__ double wave_sum(double v) {
+  auto dpp = [](double x, auto ctrl) {
+    constexpr int c = decltype(ctrl)::value;
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), c, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), c, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+  };
+  v += dpp(v, std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
+  v += dpp(v, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+  v += dpp(v, std::integral_constant<int, 0x141>{});  // row_half_mirror
+  v += dpp(v, std::integral_constant<int, 0x140>{});  // row_mirror
+  v = pair_sum_bit4(v, v);
+  return pair_sum_bit5(v, v);
+}
+
 // Sums the NV values v[] of every lane over the groups of L lanes of a wave
 // (lane bits log2(L)..5) without LDS, as a reduce-scatter: each step hands
 // half of the values to the partner lane of one lane bit and keeps the other
@@ -160,17 +178,19 @@ __device__ __forceinline__ double pair_sum_bit2(double x, double y, bool bit) {
 // wave's groups of value k + (NV L / 64) gw, where gw = lane / L.
 template <int L, int NV>
 __device__ __forceinline__ void wave_reduce_scatter(double* v) {
-  static_assert(L == 4 || L == 8 || L == 16, "lane groups of 4, 8 or 16");
+  static_assert(L == 4 || L == 8 || L == 16 || L == 32, "lane groups of 4 to 32");
   static_assert((NV * L) % 64 == 0, "values must split evenly over the groups");
   const int lane = threadIdx.x & 63;
   static_for<0, NV / 2>([&](auto kc) {
     constexpr int k = decltype(kc)::value;
     v[k] = pair_sum_bit5(v[k], v[k + NV / 2]);
   });
-  static_for<0, NV / 4>([&](auto kc) {
-    constexpr int k = decltype(kc)::value;
-    v[k] = pair_sum_bit4(v[k], v[k + NV / 4]);
-  });
+  if constexpr (L <= 16) {
+    static_for<0, NV / 4>([&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      v[k] = pair_sum_bit4(v[k], v[k + NV / 4]);
+    });
+  }
   if constexpr (L <= 8) {
     const bool b3 = (lane & 8) != 0;
     static_for<0, NV / 8>([&](auto kc) {
@@ -187,6 +207,19 @@ __device__ __forceinline__ void wave_reduce_scatter(double* v) {
   }
 }
 
+// p[0] + p[stride] + ... (n terms in order), the reads of up to four ahead of
+// the sums.
+__device__ __forceinline__ double ordered_sum(const double* p, int stride, int n) {
+  double s = 0.0;
+  int i = 0;
+  for (; i + 4 <= n; i += 4, p += 4 * stride) {
+    const double a = p[0], b = p[stride], c = p[2 * stride], d = p[3 * stride];
+    s = (((s + a) + b) + c) + d;
+  }
+  for (; i < n; ++i, p += stride) s += p[0];
+  return s;
+}
+
 // Sets the issue priority (0..3) of the executing wave; p must be the same in
 // every lane of the wave.
 __device__ __forceinline__ void set_wave_priority(int p) {
@@ -196,12 +229,6 @@ __device__ __forceinline__ void set_wave_priority(int p) {
     case 1: __builtin_amdgcn_s_setprio(1); break;
     default: __builtin_amdgcn_s_setprio(0); break;
   }
-}
-
-// Scratch doubles after the fixed LDS arrays of apply_kernel (the chunk sums
-// of the observables), max(threads, 3 NG).
-__host__ __device__ constexpr size_t apply_part_doubles(int nw, int NG) {
-  return (size_t)64 * nw > (size_t)3 * NG ? (size_t)64 * nw : (size_t)3 * NG;
 }
 
 // Per-group LDS slot of apply_kernel (complex elements): the transpose tile
@@ -221,14 +248,26 @@ __host__ __device__ constexpr int apply_slot() {
 // (also the circulant-product partials and observables staging after the
 // pair loop), then w, V_F w (followed by rho), K_1 or T w (complex NG each),
 // rho, K_H or vH, K_2 or vCG/NG in the G layout (NG doubles each), a small
-// scratch and the reduction scratch.
+// scratch and the twiddle table.
 template <int NG>
 __host__ __device__ constexpr size_t apply_lds_bytes(int nw) {
   return (size_t)nw * (64 / GroupFFT<NG>::L) * apply_slot<NG>() * sizeof(zd) +
          3 * NG * sizeof(zd) + 3 * NG * sizeof(double) + 16 * sizeof(double) +
-         apply_part_doubles(nw, NG) * sizeof(double);
+         GroupFFT<NG>::TWL * sizeof(zd);
 }
 
+// A launch of a small system is a chain of latencies, of which an empty kernel in
+// a graph takes 1.6 us: the arguments, one round trip to memory, the transforms
+// of one pair, two reductions, the stores.  So each link has one wait: scalar
+// loads in one batch, field values and twiddles off the way of the operands,
+// sums whose reads go ahead.  Per RK4 stage, against one
+// batch per use and one read per product:
+//   NG 16, 40 k-points, 8 bands, 1 occupied   5.55 -> 4.93 us
+//   NG 32, 32 k-points, 2 bands               7.51 -> 5.80 us
+//   NG 64, 21 k-points, 3 bands               8.55 -> 7.14 us
+//   NG 64, 64 k-points, 4 bands               15.9 -> 14.4 us (four passes per wave)
+//   NG 128, 16 k-points, 4 bands              13.75 -> 12.8 us
+//
 // TE: the Hartree and kinetic round trips as transforms (else circulant
 // products); the launcher chooses (apply_by_transforms).
 template <int NG>
@@ -237,21 +276,22 @@ __host__ __device__ constexpr bool apply_by_transforms(int nw) {
 }
 
 template <int NG, bool TE>
-__global__ void __launch_bounds__(512) apply_kernel(ApplyArgs a) {
+__global__ void __launch_bounds__(512, NG == 16 ? 4 : 2) apply_kernel(ApplyArgs a) {
   using F = GroupFFT<NG>;
   constexpr int R = F::R, L = F::L, GPW = 64 / L;
   constexpr int SSZ = apply_slot<NG>();
-  // after the reduction the slot area holds 5 partials per thread and the
-  // observables staging (7 NG doubles at 5 * blockDim); checked at the
-  // smallest launch (one wave, or NG/64 waves)
-  static_assert(5 * 64 * (NG > 64 ? NG / 64 : 1) + 7 * NG <=
-                    2 * SSZ * GPW * (NG > 64 ? NG / 64 : 1),
+  // circulant products: points of a block, and waves that work on them
+  constexpr int CB = NG >= 64 ? 4 : 2, CW = (NG / CB) * (NG / CB) / 64;
+  // after the reduction the slot area holds 5 NG partials per wave and the
+  // observables staging (6 NG doubles); checked at the smallest launch (one
+  // wave, or NG/64 waves)
+  constexpr int NW1 = NG > 64 ? NG / 64 : 1;
+  static_assert(5 * NG * NW1 + 6 * NG <= 2 * SSZ * GPW * NW1,
                 "slot area too small for the epilogue scratch");
   extern __shared__ zd smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int nw = blockDim.x >> 6;
   const int l = lane % L, gw = lane / L;
-  const int grp = wave * GPW + gw, ngrp = nw * GPW;
+  const int lane0 = lane_zero();
   // per-workgroup operands: from the arguments, or from the trajectory table
   int row = blockIdx.x;
   int nk = a.nk, obs_stride = a.obs_stride;
@@ -261,6 +301,15 @@ __global__ void __launch_bounds__(512) apply_kernel(ApplyArgs a) {
   const zd *u = a.u, *w = a.w;
   zd *u0 = a.u0, *ksum = a.ksum, *unext = a.unext, *out = a.out;
   double* obs = a.obs;
+  // read in one batch of scalar loads (where each is first used, they are a
+  // chain of five batches, 0.5 us)
+  int mode = a.mode, jstep = a.jstep, nbw = a.nbw;
+  const int* step_base = a.step_base;
+  asm("" : "+s"(nk), "+s"(nbw), "+s"(mode), "+s"(jstep), "+s"(step_base), "+s"(kx), "+s"(vtl),
+           "+s"(kc), "+s"(u), "+s"(w), "+s"(u0), "+s"(ksum), "+s"(unext), "+s"(obs));
+  int wld = a.wld, balance = a.balance, nthr = blockDim.x;
+  zd* tape = a.tape;
+  asm("" : "+s"(row), "+s"(wld), "+s"(balance), "+s"(nthr), "+s"(tape), "+s"(vion));
   const int tr = blockIdx.y;  // trajectory of a uniform batch (0 otherwise)
   if (tr > 0) {
     Aarr += (size_t)tr * a.fstride;
@@ -284,7 +333,7 @@ __global__ void __launch_bounds__(512) apply_kernel(ApplyArgs a) {
     u0 = t.u0;
     ksum = t.ksum;
     obs = t.obs;
-    switch (a.mode) {
+    switch (mode) {
       case M_S1: u = t.u0; unext = t.sa; break;
       case M_S2: u = t.sa; unext = t.sb; break;
       case M_S3: u = t.sb; unext = t.sa; break;
@@ -293,25 +342,27 @@ __global__ void __launch_bounds__(512) apply_kernel(ApplyArgs a) {
     }
     w = u;
   }
-  const int ik = row / a.nbw, ib = row - ik * a.nbw;
+  const int ik = row / nbw, ib = row - ik * nbw;
 
+  const int nw = nthr >> 6;
+  const int grp = wave * GPW + gw, ngrp = nw * GPW;
   zd* T = smem + grp * SSZ;
   zd* sW = smem + ngrp * SSZ;
   zd* sVF = sW + NG;
   double* sRho = reinterpret_cast<double*>(sVF + NG);  // follows V_F w (one reduction)
-  const int P = blockDim.x / NG;  // >= 1: at least NG threads
   zd* sK1 = reinterpret_cast<zd*>(sRho + NG);          // K_1, or T w
   double* sKH = reinterpret_cast<double*>(sK1 + NG);   // K_H, or vH
   double* sK2 = sKH + NG;                              // K_2, or vCG/NG (G layout)
   double* sRed = sK2 + NG;
-  double* sPart = sRed + 16;  // apply_part_doubles(nw, NG)
+  zd* sTw = reinterpret_cast<zd*>(sRed + 16);  // twiddle table (GroupFFT<NG>::TWL)
 
   // taped forward: the stage states live in the tape slots of this step
+  const bool fields = step_base != nullptr;  // field arrays at the device step counter
+  const int step0 = gload_lanes(fields ? step_base : reinterpret_cast<const int*>(a.tw), lane0);
   zd* tape0 = nullptr;
-  if (a.tape && a.step_base) {
-    const int tstep = *a.step_base + a.jstep;
-    zd* tp = a.tape + (size_t)(tstep % a.tape_seg) * 4 * a.nstate;
-    switch (a.mode) {
+  if (tape && step_base) {
+    zd* tp = tape + (size_t)((__builtin_amdgcn_readfirstlane(step0) + jstep) % a.tape_seg) * 4 * a.nstate;
+    switch (mode) {
       case M_S1: tape0 = tp; unext = tp + a.nstate; break;
       case M_S2: u = w = tp + a.nstate; unext = tp + 2 * a.nstate; break;
       case M_S3: u = w = tp + 2 * a.nstate; unext = tp + 3 * a.nstate; break;
@@ -332,34 +383,14 @@ __global__ void __launch_bounds__(512) apply_kernel(ApplyArgs a) {
   }
 
   // ---- prologue: every operand load of the first pass is issued before the
-  // first wait, so the loop starts after one memory round trip: the lane
-  // twiddles, the first u(q,j), then w of this row and the kinetic kernels,
-  // which go to LDS ----
-  const size_t o = (size_t)NG * (a.wld ? ib + a.wld * ik : row) + (tid < NG ? tid : 0);
-  F fft;
-  fft.init(a.tw, l);
-
-  zd acc[R], un[R];
-  double den[R];
-
-  // ---- exchange pair loop (ubkwbk_vFwbk, src/Functions.f90:247-257) ----
-  // u(q,j) of the next pair is fetched while the current pair is transformed;
-  // the multipliers of the current pair are loaded before that prefetch, so
-  // waiting for them leaves the prefetch in flight.
-  const int nitem = nk * a.nbocc;
-  // item = jb + nbocc iq; a group's items are ngrp apart
-  const int dq = ngrp / a.nbocc, dj = ngrp - dq * a.nbocc;
-  int cq = grp / a.nbocc, cj = grp - cq * a.nbocc;  // item of the current pass
-  auto fetch = [&](int iq, int jb) {
-    const zd* urow = u + (size_t)NG * (jb + a.nb * iq);
-    static_for<0, R>([&](auto mc) {
-      constexpr int m = decltype(mc)::value;
-      un[m] = gload(urow + L * m + l);
-    });
-  };
-  if (grp < nitem) fetch(cq, cj);
-  zd w_o = mk(0.0, 0.0), k1_o = mk(0.0, 0.0);
+  // first wait, so the loop starts after one memory round trip: w of this row,
+  // the kinetic kernels and the twiddle table, which go to LDS (each wave
+  // loading its lanes' twiddles itself kept the L1 of the CU busy for 1 us),
+  // then the first u(q,j) and multipliers ----
+  const size_t o = (size_t)NG * (wld ? ib + wld * ik : row) + (tid < NG ? tid : 0);
+  zd w_o = mk(0.0, 0.0), k1_o = mk(0.0, 0.0), tw_o[2];
   double k2_o = 0.0;
+  const double kxv = gload(kx + (ik + lane0));
   if (tid < NG) {
     w_o = gload(w + o);
     if constexpr (TE) {
@@ -369,7 +400,42 @@ __global__ void __launch_bounds__(512) apply_kernel(ApplyArgs a) {
       k1_o = gload(reinterpret_cast<const zd*>(kc + 2 * NG) + tid);
     }
   }
-  const double kxv = gload(kx + ik);
+  static_for<0, 2>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    const int t = tid + i * nthr;
+    if ((i == 0 || NG == 128) && t < F::TWL) tw_o[i] = gload(a.tw + t);
+  });
+
+  zd acc[R], un[R];
+  double den[R], vtr[R];
+
+  // ---- exchange pair loop (ubkwbk_vFwbk, src/Functions.f90:247-257) ----
+  // u(q,j) and the multipliers of the next pair are fetched while the current
+  // pair is transformed; the last pass, the only one of a small system, fetches
+  // nothing.
+  const int nitem = nk * a.nbocc;
+  // item = jb + nbocc iq; a group's items are ngrp apart
+  const int dq = ngrp / a.nbocc, dj = ngrp - dq * a.nbocc;
+  // item of the current pass (a group without one loads the last: the waits
+  // for w and the twiddles then count exactly the loads issued after them)
+  const int item0 = grp < nitem ? grp : nitem - 1;
+  int cq = item0 / a.nbocc, cj = item0 - cq * a.nbocc;
+  auto fetch_u = [&](int iq, int jb) {
+    const zd* urow = u + (size_t)NG * (jb + a.nb * iq);
+    static_for<0, R>([&](auto mc) {
+      constexpr int m = decltype(mc)::value;
+      un[m] = gload(urow + L * m + l);
+    });
+  };
+  auto fetch_v = [&](int iq) {
+    const double* vt = vtl + (size_t)(ik - iq + nk - 1) * NG + l * R;
+    static_for<0, R>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      vtr[j] = gload(vt + j);
+    });
+  };
+  fetch_u(cq, cj);
+  fetch_v(cq);
   static_for<0, R>([&](auto mc) {
     constexpr int m = decltype(mc)::value;
     acc[m] = mk(0.0, 0.0);
@@ -380,54 +446,75 @@ __global__ void __launch_bounds__(512) apply_kernel(ApplyArgs a) {
     sK2[tid] = k2_o;
     sK1[tid] = k1_o;
   }
+  static_for<0, 2>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    const int t = tid + i * nthr;
+    if ((i == 0 || NG == 128) && t < F::TWL) sTw[t] = tw_o[i];
+  });
   // When the whole grid is one workgroup per CU, the two waves sharing a SIMD
   // belong to this workgroup and would otherwise finish far apart (the older
   // one is issued first whenever both are ready, and the other then runs the
   // rest of its items alone), while the workgroup waits for the later one.
-  // With a.balance each wave lowers its issue priority as it passes quarters
+  // With balance each wave lowers its issue priority as it passes quarters
   // of its items, so a wave that falls behind is issued first until it
   // catches up.  With more workgroups than CUs the partner wave belongs to
   // another workgroup and the default (oldest first) order is faster.
-  const int wave_items = (nitem - wave * GPW + ngrp - 1) / ngrp;  // of its first group
-  lds_barrier();  // sW visible
+  const int wave_items =  // of its first group
+      __builtin_amdgcn_readfirstlane((nitem - wave * GPW + ngrp - 1) / ngrp);
+  lds_barrier();  // sW and sTw visible
+  // NG = 16 reads the twiddles where they are used (in registers they would cost
+  // it its occupancy), NG = 32 one of its two sets (they would spill)
+  F fft;
+  if constexpr (NG > 16) fft.init_lds(sTw, l);
+  auto fwd = [&](zd (&v)[R]) {
+    if constexpr (NG == 16)
+      fft.fwd_lds(v, T, l, sTw);
+    else
+      fft.fwd(v, T, l);
+  };
+  auto inv = [&](zd (&v)[R]) {
+    if constexpr (NG == 16)
+      fft.inv_lds(v, T, l, sTw);
+    else if constexpr (NG == 32)
+      fft.inv_t(v, T, l, [&](int g0) { return fft.fw[g0]; },
+                [&](int i) { return sTw[NG + l * R + i]; });
+    else
+      fft.inv(v, T, l);
+  };
 
   int it = 0;
-  for (int item = grp; item < nitem; item += ngrp, ++it) {
-    if (a.balance) set_wave_priority(3 - (4 * it) / (wave_items > 0 ? wave_items : 1));
+  auto pass = [&](auto lastc) {
+    constexpr bool last = decltype(lastc)::value;
+    if (balance) set_wave_priority(3 - (4 * it) / wave_items);
     zd uq[R], v[R];
     static_for<0, R>([&](auto mc) {
       constexpr int m = decltype(mc)::value;
       uq[m] = un[m];
     });
-    const double* vt = vtl + (size_t)(ik - cq + nk - 1) * NG + l * R;
-    double vtr[R];
-    static_for<0, R>([&](auto jc) {
-      constexpr int j = decltype(jc)::value;
-      vtr[j] = gload(vt + j);
-    });
-    // unconditional (the last pass re-reads its own item), so the wait for
-    // vtr above counts exactly the loads issued after it
-    int nq = cq + dq, nj = cj + dj;
-    if (nj >= a.nbocc) {
-      nj -= a.nbocc;
-      ++nq;
+    if constexpr (!last) {
+      // (a group without a next item re-reads its own)
+      if (grp + (it + 1) * ngrp < nitem) {
+        cq += dq;
+        cj += dj;
+        if (cj >= a.nbocc) {
+          cj -= a.nbocc;
+          ++cq;
+        }
+      }
+      fetch_u(cq, cj);
     }
-    if (item + ngrp >= nitem) {
-      nq = cq;
-      nj = cj;
-    }
-    fetch(nq, nj);
     static_for<0, R>([&](auto mc) {
       constexpr int m = decltype(mc)::value;
       v[m] = zmulc(sW[L * m + l], uq[m]);
       den[m] += zabs2(uq[m]);
     });
-    fft.fwd(v, T, l);
+    fwd(v);
     static_for<0, R>([&](auto jc) {
       constexpr int j = decltype(jc)::value;
       v[j] = zscal(v[j], vtr[j]);
     });
-    fft.inv(v, T, l);
+    if constexpr (!last) fetch_v(cq);
+    inv(v);
     static_for<0, R>([&](auto mc) {
       constexpr int m = decltype(mc)::value;
       acc[m].x = fma(v[m].x, uq[m].x, acc[m].x);
@@ -435,33 +522,26 @@ __global__ void __launch_bounds__(512) apply_kernel(ApplyArgs a) {
       acc[m].y = fma(v[m].x, uq[m].y, acc[m].y);
       acc[m].y = fma(v[m].y, uq[m].x, acc[m].y);
     });
-    cq = nq;
-    cj = nj;
-  }
-  if (a.balance) set_wave_priority(0);
+  };
+  for (; it + 1 < wave_items; ++it) pass(std::false_type{});
+  if (grp + it * ngrp < nitem) pass(std::true_type{});
+  if (balance) set_wave_priority(0);
 
-  // field values of this launch: read only now, so that the device step
-  // counter and the field arrays (a chain of two dependent loads) do not
-  // hold back the operand loads of the pair loop
-  int slot = a.obs_slot;
-  double Akin = a.A, Aobs = a.Aobs;
-  if (a.step_base) {
-    const int step = *a.step_base + a.jstep;
-    const double At = gload(Aarr + step), Aav = gload(Aavearr + step);
-    if (a.mode == M_S1) {
-      Akin = 2.0 * Aav - At;  // A(it-1) as in RT_RK4_ubk
-      Aobs = step > 0 ? gload(Aarr + step - 1) : 0.0;
-      slot = step;
-    } else if (a.mode == M_S2 || a.mode == M_S3) {
-      Akin = Aav;
-    } else if (a.mode == M_S4) {
-      Akin = At;
-    } else {  // M_OBS after step 'step'
-      Akin = At;
-      Aobs = At;
-      slot = step + 1;
-    }
-  }
+  // field values of this launch: read only now, so that they do not hold back
+  // the operand loads of the pair loop, and looked at only when they are used
+  const int step = step0 + jstep;
+  const double* none = reinterpret_cast<const double*>(a.tw);
+  const int fi = fields ? step : 0;
+  const double At = gload((fields ? Aarr : none) + fi), Aav = gload((fields ? Aavearr : none) + fi),
+               Ap = gload((fields ? Aarr : none) + (fi > 0 ? fi - 1 : 0));
+  auto akin = [&] {  // stage 1: A(it-1) as in RT_RK4_ubk
+    return !fields ? a.A
+           : mode == M_S1 ? 2.0 * Aav - At
+           : mode == M_S2 || mode == M_S3 ? Aav : At;
+  };
+  auto aobs = [&] {  // of the stage input, or (M_OBS) after the step
+    return !fields ? a.Aobs : mode != M_S1 ? At : step > 0 ? Ap : 0.0;
+  };
 
   // epilogue operands: loaded now, used after the reduction (whose barriers
   // order LDS only, so these loads stay in flight meanwhile)
@@ -470,9 +550,9 @@ __global__ void __launch_bounds__(512) apply_kernel(ApplyArgs a) {
   if (tid < NG) {
     if constexpr (!TE) khv = gload(kc + tid);
     vionv = gload(vion + tid);
-    if (a.mode >= M_S1 && a.mode <= M_S4) {
+    if (mode >= M_S1 && mode <= M_S4) {
       u0v = gload(u0 + o);
-      if (a.mode != M_S1) ksv = gload(ksum + o);
+      if (mode != M_S1) ksv = gload(ksum + o);
     }
   }
 
@@ -500,11 +580,9 @@ __global__ void __launch_bounds__(512) apply_kernel(ApplyArgs a) {
       if (vi < 3 * R) wp[(vi % 3) * NG + L * (vi / 3) + l] = v3[k];
     });
     lds_barrier();
-    for (int t = tid; t < 3 * NG; t += blockDim.x) {
+    for (int t = tid; t < 3 * NG; t += nthr) {
       const int c = t / NG, x = t - c * NG;
-      double sum = 0.0;
-      for (int w2 = 0; w2 < nw; ++w2)
-        sum += reinterpret_cast<const double*>(smem + (size_t)w2 * GPW * SSZ)[t];
+      const double sum = ordered_sum(reinterpret_cast<const double*>(smem) + t, 2 * GPW * SSZ, nw);
       if (c < 2)
         reinterpret_cast<double*>(sVF)[2 * x + c] = sum;
       else
@@ -514,20 +592,20 @@ __global__ void __launch_bounds__(512) apply_kernel(ApplyArgs a) {
   if (!TE && tid < NG) sKH[tid] = khv;
   lds_barrier();  // V_F w and rho complete; the slot area is free
 
-  const bool want_obs = (a.mode == M_S1 || a.mode == M_OBS) && obs != nullptr;
+  const bool want_obs = (mode == M_S1 || mode == M_OBS) && obs != nullptr;
   if constexpr (TE) {
     // ---- one transform round trip each: group 0 of the first wave on rho,
     // group 1 on w (the wave's other groups repeat group 1's work and store
     // nothing); group 1 also sums Ekin and J of the row by Parseval ----
     if (wave == 0) {
-      const double kA = kxv + Akin, kAo = kxv + Aobs;
+      const double kA = kxv + akin(), kAo = kxv + aobs();
       zd v[R];
       static_for<0, R>([&](auto mc) {
         constexpr int m = decltype(mc)::value;
         const int x = L * m + l;
         v[m] = gw == 0 ? mk(sRho[x], 0.0) : sW[x];
       });
-      fft.fwd(v, T, l);
+      fwd(v);
       double ek = 0.0, jc = 0.0;
       static_for<0, R>([&](auto jc_) {
         constexpr int j = decltype(jc_)::value;
@@ -540,7 +618,7 @@ __global__ void __launch_bounds__(512) apply_kernel(ApplyArgs a) {
         const double q = G + kA;
         v[j] = zscal(v[j], gw == 0 ? sK2[l * R + j] : (0.5 / NG) * q * q);
       });
-      fft.inv(v, T, l);
+      inv(v);
       static_for<0, R>([&](auto mc) {
         constexpr int m = decltype(mc)::value;
         const int x = L * m + l;
@@ -560,38 +638,57 @@ __global__ void __launch_bounds__(512) apply_kernel(ApplyArgs a) {
       }
     }
   } else {
-    // ---- circulant products over all threads: K_H * rho, K_2 * w, K_1 * w;
-    // thread (p, x) sums the terms y = p, p + P, ... into partials parked in
-    // the slot area (free after the reduction), then thread x adds the P
-    // partials in order ----
-    const int x = tid % NG, p = tid / NG;
-    if (p < P) {
-      double vh = 0.0;
-      zd c2 = mk(0.0, 0.0), c1 = mk(0.0, 0.0);
-      for (int y = p; y < NG; y += P) {
-        const int d = (x - y) & (NG - 1);
-        const zd wy = sW[y];
-        const double k2 = sK2[d];
-        const zd k1 = sK1[d];
-        vh = fma(sKH[d], sRho[y], vh);
-        c2.x = fma(k2, wy.x, c2.x);
-        c2.y = fma(k2, wy.y, c2.y);
-        c1.x = fma(k1.x, wy.x, c1.x);
-        c1.x = fma(-k1.y, wy.y, c1.x);
-        c1.y = fma(k1.x, wy.y, c1.y);
-        c1.y = fma(k1.y, wy.x, c1.y);
+    // ---- circulant products K_H * rho, K_2 * w, K_1 * w: thread (x, y) takes
+    // the B x B points x, x + XN, ... and y, y + XN, ... (XN = NG/B), between
+    // which only B differences mod NG occur, so B reads of each operand serve
+    // B^2 products (one read each per product: the LDS bandwidth, 0.85 us at
+    // NG = 64, now 0.4).  The threads of a wave with the same x add theirs in
+    // registers; the sums are parked in the slot area (free after the
+    // reduction) as [wave][value][x], and thread x adds those in order ----
+    constexpr int B = CB, XN = NG / B, NV = (5 * B * XN + 63) / 64 * 64 / XN, VF = NV * XN / 64;
+    const int xr = tid % XN;
+    if (wave < CW) {
+      double s5[NV];
+      static_for<0, NV>([&](auto kc) { s5[decltype(kc)::value] = 0.0; });
+      for (int yr = tid / XN; yr < XN; yr += nthr / XN) {
+        double kh[B], k2[B];
+        zd k1[B];
+        static_for<0, B>([&](auto ic) {
+          constexpr int i = decltype(ic)::value;
+          const int d = (xr - yr + i * XN) & (NG - 1);
+          kh[i] = sKH[d];
+          k2[i] = sK2[d];
+          k1[i] = sK1[d];
+        });
+        static_for<0, B>([&](auto jc) {
+          constexpr int jj = decltype(jc)::value;
+          const zd wy = sW[yr + jj * XN];
+          const double ry = sRho[yr + jj * XN];
+          static_for<0, B>([&](auto ic) {
+            constexpr int i = decltype(ic)::value, m = (i - jj + B) % B;
+            s5[i] = fma(kh[m], ry, s5[i]);
+            s5[B + i] = fma(k2[m], wy.x, s5[B + i]);
+            s5[2 * B + i] = fma(k2[m], wy.y, s5[2 * B + i]);
+            s5[3 * B + i] = fma(k1[m].x, wy.x, s5[3 * B + i]);
+            s5[3 * B + i] = fma(-k1[m].y, wy.y, s5[3 * B + i]);
+            s5[4 * B + i] = fma(k1[m].x, wy.y, s5[4 * B + i]);
+            s5[4 * B + i] = fma(k1[m].y, wy.x, s5[4 * B + i]);
+          });
+        });
       }
-      double* q = reinterpret_cast<double*>(smem) + 5 * (size_t)tid;
-      q[0] = vh;
-      q[1] = c2.x;
-      q[2] = c2.y;
-      q[3] = c1.x;
-      q[4] = c1.y;
+      wave_reduce_scatter<XN, NV>(s5);
+      double* q = reinterpret_cast<double*>(smem) + 5 * NG * (size_t)wave + xr;
+      static_for<0, VF>([&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        const int vi = k + VF * (lane / XN);
+        if (vi < 5 * B) q[vi * XN] = s5[k];
+      });
     }
   }
   lds_barrier();
 
   // ---- epilogue: H w and the mode-specific update ----
+  const int np = nw < CW ? nw : CW;  // circulant partials
   if (tid < NG) {
     const zd wv = sW[tid];
     const zd vf = sVF[tid];
@@ -604,20 +701,21 @@ __global__ void __launch_bounds__(512) apply_kernel(ApplyArgs a) {
       const double* cp = reinterpret_cast<const double*>(smem);
       zd c2 = mk(0.0, 0.0), c1 = mk(0.0, 0.0);
       vh = 0.0;
-      for (int p = 0; p < P; ++p) {
-        const double* q = cp + 5 * (size_t)(p * NG + tid);
+#pragma unroll 4
+      for (int p = 0; p < np; ++p) {
+        const double* q = cp + 5 * NG * (size_t)p + tid;
         vh += q[0];
-        c2.x += q[1];
-        c2.y += q[2];
-        c1.x += q[3];
-        c1.y += q[4];
+        c2.x += q[NG];
+        c2.y += q[2 * NG];
+        c1.x += q[3 * NG];
+        c1.y += q[4 * NG];
       }
       vh *= occ;  // the density sum holds sum |u|^2
-      const double kA = kxv + Akin;
+      const double kA = kxv + akin();
       // T w = K_2 * w + (k+A) K_1 * w + (k+A)^2/2 w
       tw = mk(c2.x + kA * c1.x + 0.5 * kA * kA * wv.x, c2.y + kA * c1.y + 0.5 * kA * kA * wv.y);
       if (want_obs) {
-        const double kAo = kxv + Aobs;
+        const double kAo = kxv + aobs();
         const double w2 = zabs2(wv);
         const double wc1 = wv.x * c1.x + wv.y * c1.y;  // Re conj(w) (K_1 * w)
         const double wc2 = wv.x * c2.x + wv.y * c2.y;
@@ -627,18 +725,18 @@ __global__ void __launch_bounds__(512) apply_kernel(ApplyArgs a) {
     }
     zd h = zadd(tw, zscal(wv, vh + vionv));
     h = zadd(h, vf);
-    if (a.mode == M_HPSI) {
+    if (mode == M_HPSI) {
       gstore(out + o, h);
-    } else if (a.mode >= M_S1 && a.mode <= M_S4) {
+    } else if (mode >= M_S1 && mode <= M_S4) {
       const zd kk = mk(h.y, -h.x);  // -i * H w
       const double hdt = 0.5 * a.dt;
-      if (a.mode == M_S1) {
+      if (mode == M_S1) {
         if (tape0) gstore(tape0 + o, u0v);
         gstore(ksum + o, kk);
         gstore(unext + o, mk(u0v.x + hdt * kk.x, u0v.y + hdt * kk.y));
-      } else if (a.mode == M_S2 || a.mode == M_S3) {
+      } else if (mode == M_S2 || mode == M_S3) {
         gstore(ksum + o, mk(ksv.x + 2.0 * kk.x, ksv.y + 2.0 * kk.y));
-        const double c = (a.mode == M_S2) ? hdt : a.dt;
+        const double c = (mode == M_S2) ? hdt : a.dt;
         gstore(unext + o, mk(u0v.x + c * kk.x, u0v.y + c * kk.y));
       } else {
         gstore(u0 + o,
@@ -649,7 +747,7 @@ __global__ void __launch_bounds__(512) apply_kernel(ApplyArgs a) {
       // per-point terms of Ekin, J (circulant form), Ex (this row) and N,
       // Eion, EH (row 0)
       const double rho = occ * sRho[tid];
-      double* st = reinterpret_cast<double*>(smem) + 5 * (size_t)blockDim.x;
+      double* st = reinterpret_cast<double*>(smem) + 5 * NG * np;
       st[0 * NG + tid] = ekt;
       st[1 * NG + tid] = jt;
       st[2 * NG + tid] = wv.x * vf.x + wv.y * vf.y;
@@ -659,42 +757,26 @@ __global__ void __launch_bounds__(512) apply_kernel(ApplyArgs a) {
     }
   }
   if (want_obs) {
-    // six fixed-order sums over x: chunks of 8 points, then the chunks
-    constexpr int NCH = (NG + 7) / 8;
+    // six fixed-order sums over x, one wave each in turn
     const int nv = row == 0 ? 6 : 3;
     lds_barrier();
-    const double* st = reinterpret_cast<const double*>(smem) + 5 * (size_t)blockDim.x;
-    double* ch = sPart;
-    if (tid < nv * NCH) {
-      const int v = tid / NCH, c = tid - v * NCH;
-      const double* src = st + v * NG + 8 * c;
+    const double* st = reinterpret_cast<const double*>(smem) + 5 * NG * np;
+    const int slot = !fields ? a.obs_slot : mode == M_S1 ? step : step + 1;
+    double* p = obs + (size_t)slot * obs_stride;
+    const double occr = ib < a.nbocc ? occ : 0.0;
+    for (int v = wave; v < nv; v += nw) {
       double s = 0.0;
-      for (int i = 0; i < 8 && 8 * c + i < NG; ++i) s += src[i];
-      ch[tid] = s;
-    }
-    lds_barrier();
-    if (tid == 0) {
-      double t[6];
-      for (int v = 0; v < nv; ++v) {
-        double s = 0.0;
-        for (int c = 0; c < NCH; ++c) s += ch[v * NCH + c];
-        t[v] = s;
-      }
+      static_for<0, (NG + 63) / 64>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        if (lane + 64 * i < NG) s += st[v * NG + 64 * i + lane];
+      });
+      s = wave_sum(s);
       if constexpr (TE) {  // Ekin and J from the transform of w
-        t[0] = sRed[0];
-        t[1] = sRed[1];
+        if (v < 2) s = sRed[v];
       }
-      const double occr = ib < a.nbocc ? occ : 0.0;
-      double* p = obs + (size_t)slot * obs_stride;
-      gstore(p + 3 * row + 0, occr * t[0] * a.dv);
-      gstore(p + 3 * row + 1, occr * t[1]);
-      gstore(p + 3 * row + 2, occr * t[2] * a.dv);
-      if (row == 0) {
-        const int rows = a.nbw * nk;
-        gstore(p + 3 * rows + 0, t[3] * a.dv);
-        gstore(p + 3 * rows + 1, t[4] * a.dv);
-        gstore(p + 3 * rows + 2, 0.5 * t[5] * a.dv);
-      }
+      s *= v < 3 ? occr : v == 5 ? 0.5 : 1.0;
+      if (v != 1) s *= a.dv;
+      if (lane == 0) gstore(p + (v < 3 ? 3 * row : 3 * nbw * nk - 3) + v, s);
     }
   }
 }

@@ -130,24 +130,6 @@ __device__ __forceinline__ int kspace_tw_slot(int i) {
   else return N + (r % F::R) * F::L + r / F::R;
 }
 
-// Sum of v over the 64 lanes of a wave, the same in every lane, without LDS:
-// DPP within 16 lanes (lane ^ 1, ^ 2, then mirrors, which act as ^ 4 and ^ 8
-// once the quads and half rows are equal), permlane swaps across them.
-__device__ __forceinline__ double wave_sum(double v) {
-  auto dpp = [](double x, auto ctrl) {
-    constexpr int c = decltype(ctrl)::value;
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), c, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), c, 0xf, 0xf, false);
-    return __hiloint2double(hi, lo);
-  };
-  v += dpp(v, std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
-  v += dpp(v, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
-  v += dpp(v, std::integral_constant<int, 0x141>{});  // row_half_mirror
-  v += dpp(v, std::integral_constant<int, 0x140>{});  // row_mirror
-  v = pair_sum_bit4(v, v);
-  return pair_sum_bit5(v, v);
-}
-
 __device__ __forceinline__ void zfma(zd& s, zd a, zd b) {  // s += a b
   s.x = fma(a.x, b.x, s.x);
   s.x = fma(-a.y, b.y, s.x);

@@ -1,0 +1,51 @@
+"""The row-wise kernels at the edges of their split: every number of waves, a
+last pass in which one or all but one of the lane groups of a wave have a pair,
+one pair in all, more bands than are occupied.  Against the oracle, at the
+tolerances of the density-matrix path's tests."""
+import numpy as np
+import pytest
+
+from test_gpu_kspace import orbitals, rel, system
+
+pytestmark = pytest.mark.gpu
+
+A16, A32, A64, A128 = (3.6, 1.0), (8.0, 4.0), (10.0, 6.0), (12.0, 6.0)
+# (ng, nk, nb, nbocc, acell, Z): NG = 16 and 32 hold 16 pairs per wave, 64
+# eight, 128 four
+CASES = [(16, 1, 1, 1) + A16, (16, 17, 2, 1) + A16, (16, 11, 3, 3) + A16, (16, 43, 3, 3) + A16,
+         (32, 1, 1, 1) + A32, (32, 16, 2, 1) + A32, (32, 7, 5, 5) + A32, (32, 19, 5, 5) + A32,
+         (64, 1, 2, 1) + A64, (64, 3, 3, 3) + A64, (64, 21, 3, 3) + A64, (64, 13, 5, 5) + A64,
+         (64, 5, 13, 13) + A64, (128, 1, 1, 1) + A128, (128, 3, 3, 3) + A128, (128, 7, 3, 3) + A128,
+         (128, 11, 3, 3) + A128]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"ng{c[0]}_nk{c[1]}_nb{c[2]}_{c[3]}")
+def test_rows_match_oracle(case):
+    S, O, G, _ = system(case)
+    u, w = orbitals(case, 1), orbitals(case, 2)
+    with G:
+        assert rel(G.ubkwbk_hwbk(u, w, 0.23), O.ubkwbk_hwbk(u, w, 0.23)) < 1e-12
+        _, ec, n, j = G.observables(u, -0.17)
+        assert rel(ec, O.ubk_Ecomps(u, -0.17)) < 1e-12
+        assert abs(n - O.nele(u)) < 1e-12 and abs(j - O.ubk_Je(u, -0.17)) < 1e-12 * max(1.0, abs(j))
+        A, Aave = np.array([0.1, 0.25, -0.1]), np.array([0.05, 0.175, 0.075])
+        ug, eg, _, jg, i3 = G.RT_calculation(u, A, Aave)
+        uo, eo, _, jo, i3o = O.RT_calculation(u, G.dt, A, Aave)
+        assert rel(ug, uo) < 1e-12 and np.abs(eg - eo).max() < 1e-10
+        assert rel(jg, jo) < 1e-8 and np.abs(i3 - i3o).max() < 1e-10
+
+
+# (the adjoint takes occupied bands only)
+@pytest.mark.parametrize("case", [c for c in CASES if c[2] == c[3]],
+                         ids=lambda c: f"ng{c[0]}_nk{c[1]}_nb{c[2]}_{c[3]}")
+def test_row_adjoint_matches_oracle(case):
+    S, O, G, _ = system(case)
+    u, A = orbitals(case, 3), np.array([0.1, -0.05])
+    for objective, oracle in (("energy", "adjoint_energy"), ("jsq", "adjoint_jsq")):
+        L, _, _, _, _ = G.fwd_batch([u], A[None], objective=objective)
+        g, gu = G.bwd_batch()
+        ref = getattr(O, oracle)(u, G.dt, A)
+        assert abs(L[0] - ref[0]) < 1e-11 * max(1.0, abs(ref[0]))
+        assert np.abs(g[0] - ref[1]).max() < 1e-9 * np.abs(ref[1]).max()
+        assert np.abs(gu[0] - ref[2]).max() < 1e-9 * np.abs(ref[2]).max()
+    G.close()
