@@ -85,75 +85,79 @@ __host__ __device__ constexpr int adjoint_slot() {
 // more workgroups share a CU.
 template <int NG>
 __host__ __device__ constexpr int adjoint_epi_slot() {
-  constexpr int nwmin = NG > 64 ? NG / 64 : 1, gpw = 64 / GroupFFT<NG>::L;
-  constexpr int need = (8 * 64 * nwmin + NG + 2 * gpw * nwmin - 1) / (2 * gpw * nwmin);
+  constexpr int gpw = 64 / GroupFFT<NG>::L;
+  constexpr int need = (8 * NG + 2 * gpw - 1) / (2 * gpw);
   return need + ((8 - need % 16) + 16) % 16;
 }
 
 // LDS of adjoint_kernel<NG> with nw waves (bytes): the groups' tiles (pair
-// transposes, then reduction partials, circulant-product partials and the
-// field derivative staging), y, gbar, the exchange sum and K_1 (complex NG
-// each), rho, s, K_H, K_2 (NG doubles each), a small scratch and the chunk-sum
-// scratch (epilogue_only: the smaller slots of adjoint_kernel<NG, true>).
-// NG = 32 reads the transforms' lane twiddles from an LDS copy of the table:
-// its geometry (two register sets of twiddles) would otherwise push the
-// kernel's registers into spills.
-template <int NG>
-__host__ __device__ constexpr bool adjoint_lds_twiddles() {
-  return NG == 32;
-}
-
+// transposes, then reduction partials and circulant-product partials), y,
+// gbar, the exchange sum and K_1 (complex NG each), rho, s, K_H, K_2 (NG
+// doubles each), a small scratch and, with a pair loop, the twiddle table.
 template <int NG>
 __host__ __device__ constexpr size_t adjoint_lds_bytes(int nw, bool epilogue_only = false) {
   return (size_t)nw * (64 / GroupFFT<NG>::L) *
              (epilogue_only ? adjoint_epi_slot<NG>() : adjoint_slot<NG>()) * sizeof(zd) +
          4 * NG * sizeof(zd) + 4 * NG * sizeof(double) + 16 * sizeof(double) +
-         ((size_t)64 * nw > 4 * NG ? (size_t)64 * nw : 4 * NG) * sizeof(double) +
-         (adjoint_lds_twiddles<NG>() ? GroupFFT<NG>::TWN * sizeof(zd) : 0);
+         (epilogue_only ? 0 : GroupFFT<NG>::TWL * sizeof(zd));
 }
 
+// Bound, like apply_kernel, by the chain of latencies of a launch, and built the
+// same way; each pair has two transform round trips here (1.3 us at one wave per
+// SIMD, the FP64 rate).  Per reverse stage, against a load where each operand is
+// used and one read per product of the circulants:
+//   NG 16, 40 k-points, 2 bands   8.7 -> 6.9 us
+//   NG 32, 32 k-points, 2 bands  10.7 -> 9.05 us
+//   NG 64, 21 k-points, 3 bands  16.9 -> 14.4 us
+//   NG 64, 40 k-points, 4 bands  25.9 -> 22.0 us
+// (dE/du in an instantiation of its own: one that held both forms spilt 100
+// registers.)
+//
 // XP: the exchange part, the density and s come from the pair tiles' partial
-// sums (adjtile_kernel): the pair loop is compiled out.
-template <int NG, bool XP = false>
-__global__ void __launch_bounds__(512) adjoint_kernel(AdjArgs a0) {
-  // per-trajectory view of the arguments
+// sums (adjtile_kernel): the pair loop is compiled out.  EG: A_EGRAD (else the
+// reverse stages).
+template <int NG, bool XP = false, bool EG = false>
+__global__ void __launch_bounds__(512, XP ? 3 : 2) adjoint_kernel(AdjArgs a0) {
+  using F = GroupFFT<NG>;
+  constexpr int R = F::R, L = F::L, GPW = 64 / L;
+  constexpr int JNYQ = F::NYQ_REG;  // register of lane 0 holding G index NG/2
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int l = lane % L, gw = lane / L;
+  const int lane0 = lane_zero();
+  // per-trajectory view of the arguments, read in two batches of scalar loads
   AdjArgs a = a0;
+  int row = blockIdx.x, nthr = blockDim.x;
+  asm("" : "+s"(a.nk), "+s"(a.nb), "+s"(a.mode), "+s"(a.step_base), "+s"(a.jstep), "+s"(a.kx),
+           "+s"(a.vion), "+s"(a.vtl), "+s"(a.kc), "+s"(a.tw), "+s"(a.gb), "+s"(a.ub), "+s"(a.ua),
+           "+s"(a.gout));
+  asm("" : "+s"(row), "+s"(nthr), "+s"(a.y), "+s"(a.Aarr), "+s"(a.Aavearr), "+s"(a.step),
+           "+s"(a.tape), "+s"(a.tape_seg), "+s"(a.blk), "+s"(a.abar), "+s"(a.tstride),
+           "+s"(a.fstride));
   const int tr = blockIdx.y;
-  if (a0.step_base) {
-    a.step = *a0.step_base - a0.jstep;
-    const size_t slot = (size_t)(a.step % a0.tape_seg) * 4 + (a0.mode - 1);
-    a.y = a0.tape + slot * a0.blk;
-    if (a.abar) a.abar = a0.abar + slot * (size_t)(a0.nk * a0.nb);
+  if (a.step_base) {
+    a.step = *a.step_base - a.jstep;
+    const size_t slot = (size_t)(a.step % a.tape_seg) * 4 + (a.mode - 1);
+    a.y = a.tape + slot * a.blk;
+    if (a.abar) a.abar += slot * (size_t)(a.nk * a.nb);
   }
-  {
-    const size_t so = (size_t)tr * a0.tstride;
+  if (tr > 0) {
+    const size_t so = (size_t)tr * a.tstride;
     a.y += so;
     if (a.gb) a.gb += so;
     if (a.ub) a.ub += so;
     if (a.ua) a.ua += so;
     if (a.gout) a.gout += so;
     if (a.cout) a.cout += so;
-    if (a.abar) a.abar += (size_t)tr * a0.abar_tstride;
+    if (a.abar) a.abar += (size_t)tr * a.abar_tstride;
   }
-  double fa;
-  {
-    const double At = a.Aarr[(size_t)tr * a.fstride + a.step];
-    const double Av = a.Aavearr[(size_t)tr * a.fstride + a.step];
-    fa = a.mode == A_S1 ? 2.0 * Av - At : (a.mode == A_S2 || a.mode == A_S3) ? Av : At;
-  }
-  using F = GroupFFT<NG>;
-  constexpr int R = F::R, L = F::L, GPW = 64 / L;
-  constexpr int JNYQ = F::NYQ_REG;  // register of lane 0 holding G index NG/2
   extern __shared__ zd smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int nw = blockDim.x >> 6;
-  const int l = lane % L, gw = lane / L;
+  const int nw = nthr >> 6;
   const int grp = wave * GPW + gw, ngrp = nw * GPW;
-  const int row = blockIdx.x;
-  const int ik = row / a.nb, ib = row - ik * a.nb;
-  const bool egrad = a.mode == A_EGRAD;
-  const zd* gbar = egrad ? a.y : a.gb;
+  const int ik = row / a.nb;
+  const zd* gbar = EG ? a.y : a.gb;
 
+  // circulant products: points of a block, and waves that work on them
+  constexpr int CB = NG >= 64 ? 4 : 2, CW = (NG / CB) * (NG / CB) / 64;
   constexpr int SSZ = XP ? adjoint_epi_slot<NG>() : adjoint_slot<NG>();
   zd* T = smem + grp * SSZ;
   zd* sY = smem + ngrp * SSZ;      // y_ki
@@ -165,34 +169,64 @@ __global__ void __launch_bounds__(512) adjoint_kernel(AdjArgs a0) {
   double* sKH = sS + NG;
   double* sK2 = sKH + NG;
   double* sRed = sK2 + NG;
-  double* sPart = sRed + 16;  // max(blockDim.x, 4 NG) doubles (chunk sums)
-  constexpr bool LTW = adjoint_lds_twiddles<NG>();
-  zd* sTw = reinterpret_cast<zd*>(sPart + (64 * nw > 4 * NG ? 64 * nw : 4 * NG));
-  static_assert(8 * 64 * (NG > 64 ? NG / 64 : 1) + NG <= 2 * SSZ * GPW * (NG > 64 ? NG / 64 : 1),
-                "slot area too small for the epilogue scratch");
+  zd* sTw = reinterpret_cast<zd*>(sRed + 16);  // GroupFFT<NG>::TWL (not with XP)
+  static_assert(8 * NG <= 2 * SSZ * GPW, "slot area too small for the circulant partials");
   // XP: the runs of partial sums, 4 NG doubles per thread of a grid point
   // (256 per wave), also fit the slot area
   static_assert(!XP || 128 <= SSZ * GPW, "slot area too small for the partial-sum runs");
 
   const size_t o = (size_t)NG * row + (tid < NG ? tid : 0);
-  zd yv = mk(0.0, 0.0), gv = mk(0.0, 0.0);
-  double vionv = 0.0;
+  zd y_o = mk(0.0, 0.0), g_o = mk(0.0, 0.0), k1_o = mk(0.0, 0.0), tw_o[2];
+  double kh_o = 0.0, k2_o = 0.0;
   if (tid < NG) {
-    yv = gload(a.y + o);
-    gv = gload(gbar + o);
-    sY[tid] = yv;
-    sG[tid] = gv;
-    vionv = gload(a.vion + tid);
-    sKH[tid] = gload(a.kc + tid);
-    sK2[tid] = gload(a.kc + NG + tid);
-    sK1[tid] = gload(reinterpret_cast<const zd*>(a.kc + 2 * NG) + tid);
+    y_o = gload(a.y + o);
+    g_o = gload(gbar + o);
+    kh_o = gload(a.kc + tid);
+    k2_o = gload(a.kc + NG + tid);
+    k1_o = gload(reinterpret_cast<const zd*>(a.kc + 2 * NG) + tid);
   }
-  const double kxv = gload(a.kx + ik);
-  F fft;
-  if constexpr (LTW) {
-    for (int i = tid; i < F::TWN; i += blockDim.x) sTw[i] = gload(a.tw + i);
-  } else if constexpr (!XP) {
-    fft.init(a.tw, l);
+  if constexpr (!XP) {
+    static_for<0, 2>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      const int t = tid + i * nthr;
+      if ((i == 0 || NG == 128) && t < F::TWL) tw_o[i] = gload(a.tw + t);
+    });
+  }
+  // operands of the first pair (a group without one loads the last)
+  const int nitem = XP ? 0 : a.nk * a.nb;  // pair tiles: no pairs here
+  zd uq[R], gq[R];
+  double vtr[R], dnyq = 0.0;
+  auto fetch = [&](int item) {
+    const int iq = item / a.nb, jb = item - iq * a.nb;
+    const size_t prow = (size_t)NG * (jb + a.nb * iq);
+    static_for<0, R>([&](auto mc) {
+      constexpr int m = decltype(mc)::value;
+      uq[m] = gload(a.y + prow + L * m + l);
+      gq[m] = gload(gbar + prow + L * m + l);
+    });
+    const double* vt = a.vtl + (size_t)(ik - iq + a.nk - 1) * NG + l * R;
+    static_for<0, R>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      vtr[j] = gload(vt + j);
+    });
+    // D_kq = vt_qk(NG/2) - vt_kq(NG/2): G-layout position L/2 of rows (q-k), (k-q)
+    dnyq = gload(a.vtl + (size_t)(iq - ik + a.nk - 1) * NG + JNYQ) -
+           gload(a.vtl + (size_t)(ik - iq + a.nk - 1) * NG + JNYQ);
+  };
+  if constexpr (!XP) fetch(grp < nitem ? grp : nitem - 1);
+  if (tid < NG) {
+    sY[tid] = y_o;
+    sG[tid] = g_o;
+    sKH[tid] = kh_o;
+    sK2[tid] = k2_o;
+    sK1[tid] = k1_o;
+  }
+  if constexpr (!XP) {
+    static_for<0, 2>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      const int t = tid + i * nthr;
+      if ((i == 0 || NG == 128) && t < F::TWL) sTw[t] = tw_o[i];
+    });
   }
   // pair tiles: the exchange part, the density and s of this row from their
   // partials.  The H = blockDim / NG threads of a grid point each add a
@@ -236,14 +270,7 @@ __global__ void __launch_bounds__(512) adjoint_kernel(AdjArgs a0) {
       hp[3 * NG + x] = xs;
     }
   }
-  auto fwd = [&](zd (&v)[R]) {
-    if constexpr (LTW) fft.fwd_lds(v, T, l, sTw); else fft.fwd(v, T, l);
-  };
-  auto inv = [&](zd (&v)[R]) {
-    if constexpr (LTW) fft.inv_lds(v, T, l, sTw); else fft.inv(v, T, l);
-  };
   const double sgn = (l & 1) ? -1.0 : 1.0;  // (-1)^x for x = L*m + l, L even
-  const bool out_occ = ib < a.nbocc;
 
   zd acc[R];
   double den[R], sv[R];
@@ -254,69 +281,61 @@ __global__ void __launch_bounds__(512) adjoint_kernel(AdjArgs a0) {
     sv[m] = 0.0;
   });
   lds_barrier();
+  // NG = 32 reads the transforms' lane twiddles where they are used: its two
+  // register sets of them would spill
+  F fft;
+  constexpr bool LTW = NG >= 32;
+  if constexpr (!XP && !LTW) fft.init_lds(sTw, l);
+  auto fwd = [&](zd (&v)[R]) {
+    if constexpr (LTW) fft.fwd_lds(v, T, l, sTw); else fft.fwd(v, T, l);
+  };
+  auto inv = [&](zd (&v)[R]) {
+    if constexpr (LTW) fft.inv_lds(v, T, l, sTw); else fft.inv(v, T, l);
+  };
 
-  // ---- pair loop over all partner rows (q, j) ----
-  const int nitem = XP ? 0 : a.nk * a.nb;  // pair tiles: no pairs here
-  for (int item = grp; item < nitem; item += ngrp) {
-    const int iq = item / a.nb, jb = item - iq * a.nb;
-    const size_t prow = (size_t)NG * (jb + a.nb * iq);
-    const bool p_occ = jb < a.nbocc;
-    zd uq[R], gq[R], v[R];
-    static_for<0, R>([&](auto mc) {
-      constexpr int m = decltype(mc)::value;
-      uq[m] = gload(a.y + prow + L * m + l);
-      gq[m] = egrad ? mk(0.0, 0.0) : gload(a.gb + prow + L * m + l);
-      den[m] += p_occ ? zabs2(uq[m]) : 0.0;
-      sv[m] += gq[m].x * uq[m].x + gq[m].y * uq[m].y;
-    });
-    const double* vt = a.vtl + (size_t)(ik - iq + a.nk - 1) * NG + l * R;
-    // D_kq = vt_qk(NG/2) - vt_kq(NG/2): G-layout position L/2 of rows (q-k), (k-q)
-    const double dnyq = gload(a.vtl + (size_t)(iq - ik + a.nk - 1) * NG + JNYQ) -
-                        gload(a.vtl + (size_t)(ik - iq + a.nk - 1) * NG + JNYQ);
-    double vtr[R];
-    static_for<0, R>([&](auto jc) {
-      constexpr int j = decltype(jc)::value;
-      vtr[j] = gload(vt + j);
-    });
+  // ---- pair loop over all partner rows (q, j) (every band is occupied) ----
+  auto pass = [&] {
+    zd v[R];
     // T1: phi' = C'_kq(y_ki conj y_qj); adds phi' gbar_qj (or, for dE/du,
     // (phi + phi') y_qj)
-    if (out_occ && (p_occ || !egrad)) {
+    static_for<0, R>([&](auto mc) {
+      constexpr int m = decltype(mc)::value;
+      v[m] = zmulc(sY[L * m + l], uq[m]);
+      den[m] += zabs2(uq[m]);
+      sv[m] += gq[m].x * uq[m].x + gq[m].y * uq[m].y;  // (dE/du: not used)
+    });
+    fwd(v);
+    // rho_hat(NG/2) sits in lane 0 (of the group), register JNYQ
+    const double nx = __shfl(v[JNYQ].x, gw * L, 64);
+    const double ny = __shfl(v[JNYQ].y, gw * L, 64);
+    static_for<0, R>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      v[j] = zscal(v[j], vtr[j]);
+    });
+    inv(v);
+    const zd fix = mk(sgn * dnyq * nx, sgn * dnyq * ny);
+    if constexpr (EG) {
       static_for<0, R>([&](auto mc) {
         constexpr int m = decltype(mc)::value;
-        v[m] = zmulc(sY[L * m + l], uq[m]);
+        const zd s2 = zadd(v[m], zadd(v[m], fix));  // (C + C')_kq rho
+        acc[m] = zadd(acc[m], zmul(s2, uq[m]));
       });
-      fwd(v);
-      // rho_hat(NG/2) sits in lane 0 (of the group), register JNYQ
-      const double nx = __shfl(v[JNYQ].x, gw * L, 64);
-      const double ny = __shfl(v[JNYQ].y, gw * L, 64);
-      static_for<0, R>([&](auto jc) {
-        constexpr int j = decltype(jc)::value;
-        v[j] = zscal(v[j], vtr[j]);
-      });
-      inv(v);
-      const zd fix = mk(sgn * dnyq * nx, sgn * dnyq * ny);
+    } else {
       static_for<0, R>([&](auto mc) {
         constexpr int m = decltype(mc)::value;
-        const zd ph = v[m];                 // C_kq rho
-        const zd php = zadd(ph, fix);       // C'_kq rho
-        if (egrad) {
-          const zd s2 = zadd(ph, php);
-          acc[m] = zadd(acc[m], zmul(s2, uq[m]));
-        } else {
-          acc[m] = zadd(acc[m], zmul(php, gq[m]));
-        }
+        acc[m] = zadd(acc[m], zmul(zadd(v[m], fix), gq[m]));  // C'_kq rho
       });
-    }
-    // T2: psi = C_kq(gbar_ki conj y_qj + y_ki conj gbar_qj) + D fhat_C(NG/2) (-1)^x
-    if (!egrad) {
+      __builtin_amdgcn_sched_barrier(0);  // (T2's operands early would spill)
+      // T2: psi = C_kq(gbar_ki conj y_qj + y_ki conj gbar_qj) + D fhat_C(NG/2) (-1)^x
       double cx = 0.0, cy = 0.0;
       static_for<0, R>([&](auto mc) {
         constexpr int m = decltype(mc)::value;
-        const zd fb = p_occ ? zmulc(sG[L * m + l], uq[m]) : mk(0.0, 0.0);
-        const zd fc = out_occ ? zmulc(sY[L * m + l], gq[m]) : mk(0.0, 0.0);
+        const zd fb = zmulc(sG[L * m + l], uq[m]);
+        const zd fc = zmulc(sY[L * m + l], gq[m]);
         cx += fc.x;
         cy += fc.y;
         v[m] = zadd(fb, fc);
+        if constexpr (m % 2 == 1) __builtin_amdgcn_sched_barrier(0);
       });
       cx *= sgn;
       cy *= sgn;
@@ -331,11 +350,32 @@ __global__ void __launch_bounds__(512) adjoint_kernel(AdjArgs a0) {
         v[j] = zscal(v[j], vtr[j]);
       });
       inv(v);
-      const zd fix = mk(sgn * dnyq * cx, sgn * dnyq * cy);
+      const zd fix2 = mk(sgn * dnyq * cx, sgn * dnyq * cy);
       static_for<0, R>([&](auto mc) {
         constexpr int m = decltype(mc)::value;
-        acc[m] = zadd(acc[m], zmul(zadd(v[m], fix), uq[m]));
+        acc[m] = zadd(acc[m], zmul(zadd(v[m], fix2), uq[m]));
       });
+    }
+  };
+  const int wave_items =  // of the wave's first group
+      __builtin_amdgcn_readfirstlane((nitem - wave * GPW + ngrp - 1) / ngrp);
+  for (int it = 0, item = grp; it < wave_items; ++it, item += ngrp) {
+    if (it > 0) fetch(item < nitem ? item : nitem - 1);
+    if (item < nitem) pass();
+  }
+
+  // field of the stage and epilogue operands: loaded now, used after the
+  // reduction (whose barriers order LDS only)
+  const size_t fo = (size_t)tr * a.fstride + a.step + lane0;
+  const double At = gload(a.Aarr + fo), Av = gload(a.Aavearr + fo);
+  const double kxv = gload(a.kx + (ik + lane0));
+  double vionv = 0.0;
+  zd ubv = mk(0.0, 0.0), uav = mk(0.0, 0.0);
+  if (tid < NG) {
+    vionv = gload(a.vion + tid);
+    if constexpr (!EG) {
+      ubv = gload(a.ub + o);
+      if (a.mode != A_S4) uav = gload(a.ua + o);
     }
   }
 
@@ -380,114 +420,118 @@ __global__ void __launch_bounds__(512) adjoint_kernel(AdjArgs a0) {
     double* outd = reinterpret_cast<double*>(sACC);
     for (int t = tid; t < 4 * NG; t += blockDim.x) {
       const int c = t / NG, x = t - c * NG;
-      double sum = 0.0;
-      for (int w2 = 0; w2 < nw; ++w2)
-        sum += reinterpret_cast<const double*>(smem + (size_t)w2 * GPW * SSZ)[t];
+      const double sum = ordered_sum(reinterpret_cast<const double*>(smem) + t, 2 * GPW * SSZ, nw);
       outd[c < 2 ? 2 * x + c : NG * c + x] = sum;
     }
   }
   lds_barrier();
 
-  // ---- circulant products over all threads: K_H * rho, K_H * s, K_2 * gbar,
-  // K_1 * gbar, K_1 * y (Hartree potential and response, T_a gbar, P_a y) ----
+  // ---- circulant products K_H * rho, K_H * s, K_2 * gbar, K_1 * gbar, K_1 * y
+  // (Hartree potential and response, T_a gbar, P_a y), in blocks as in
+  // apply_kernel ----
   {
-    const int P = blockDim.x / NG;
-    const int x = tid % NG, p = tid / NG;
-    if (p < P) {
-      double vh = 0.0, ks = 0.0;
-      zd c2 = mk(0.0, 0.0), c1 = mk(0.0, 0.0), py = mk(0.0, 0.0);
-      for (int t = p; t < NG; t += P) {
-        const int d = (x - t) & (NG - 1);
-        const double kh = sKH[d], k2 = sK2[d];
-        const zd k1 = sK1[d], gt = sG[t], yt = sY[t];
-        vh = fma(kh, sRho[t], vh);
-        ks = fma(kh, sS[t], ks);
-        c2.x = fma(k2, gt.x, c2.x);
-        c2.y = fma(k2, gt.y, c2.y);
-        c1 = zadd(c1, zmul(k1, gt));
-        py = zadd(py, zmul(k1, yt));
+    constexpr int B = CB, XN = NG / B, NV = 8 * B, VF = NV * XN / 64;
+    static_assert(NV * XN % 64 == 0, "values must split evenly over the groups");
+    const int xr = tid % XN;
+    if (wave < CW) {
+      double s8[NV];
+      static_for<0, NV>([&](auto kc) { s8[decltype(kc)::value] = 0.0; });
+      for (int yr = tid / XN; yr < XN; yr += nthr / XN) {
+        double kh[B], k2[B];
+        zd k1[B];
+        static_for<0, B>([&](auto ic) {
+          constexpr int i = decltype(ic)::value;
+          const int d = (xr - yr + i * XN) & (NG - 1);
+          kh[i] = sKH[d];
+          k2[i] = sK2[d];
+          k1[i] = sK1[d];
+        });
+        static_for<0, B>([&](auto jc) {
+          constexpr int jj = decltype(jc)::value;
+          const int t = yr + jj * XN;
+          const zd gt = sG[t], yt = sY[t];
+          const double rt = sRho[t], st = sS[t];
+          static_for<0, B>([&](auto ic) {
+            constexpr int i = decltype(ic)::value, m = (i - jj + B) % B;
+            s8[i] = fma(kh[m], rt, s8[i]);
+            s8[B + i] = fma(kh[m], st, s8[B + i]);
+            s8[2 * B + i] = fma(k2[m], gt.x, s8[2 * B + i]);
+            s8[3 * B + i] = fma(k2[m], gt.y, s8[3 * B + i]);
+            s8[4 * B + i] = fma(-k1[m].y, gt.y, fma(k1[m].x, gt.x, s8[4 * B + i]));
+            s8[5 * B + i] = fma(k1[m].y, gt.x, fma(k1[m].x, gt.y, s8[5 * B + i]));
+            s8[6 * B + i] = fma(-k1[m].y, yt.y, fma(k1[m].x, yt.x, s8[6 * B + i]));
+            s8[7 * B + i] = fma(k1[m].y, yt.x, fma(k1[m].x, yt.y, s8[7 * B + i]));
+          });
+        });
       }
-      double* q = reinterpret_cast<double*>(smem) + 8 * (size_t)tid;
-      q[0] = vh;
-      q[1] = ks;
-      q[2] = c2.x;
-      q[3] = c2.y;
-      q[4] = c1.x;
-      q[5] = c1.y;
-      q[6] = py.x;
-      q[7] = py.y;
+      wave_reduce_scatter<XN, NV>(s8);
+      double* q = reinterpret_cast<double*>(smem) + 8 * NG * (size_t)wave + xr;
+      static_for<0, VF>([&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        q[(k + VF * (lane / XN)) * XN] = s8[k];
+      });
     }
   }
   lds_barrier();
 
   // ---- epilogue ----
-  double* stg = reinterpret_cast<double*>(smem) + 8 * (size_t)blockDim.x;  // abar terms
+  double pterm = 0.0;  // dL/da term of the point
   if (tid < NG) {
-    double vh = 0.0, ks = 0.0;
-    zd c2 = mk(0.0, 0.0), c1 = mk(0.0, 0.0), py = mk(0.0, 0.0);
-    const int P = blockDim.x / NG;
-    for (int p = 0; p < P; ++p) {
-      const double* q = reinterpret_cast<const double*>(smem) + 8 * (size_t)(p * NG + tid);
-      vh += q[0];
-      ks += q[1];
-      c2.x += q[2];
-      c2.y += q[3];
-      c1.x += q[4];
-      c1.y += q[5];
-      py.x += q[6];
-      py.y += q[7];
-    }
+    double sums[8];
+    static_for<0, 8>([&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      sums[k] = ordered_sum(reinterpret_cast<const double*>(smem) + k * NG + tid, 8 * NG,
+                            nw < CW ? nw : CW);
+    });
+    double vh = sums[0];
+    const double ks = sums[1];
+    const zd yv = sY[tid], gv = sG[tid];
+    const zd c2 = mk(sums[2], sums[3]), c1 = mk(sums[4], sums[5]), py = mk(sums[6], sums[7]);
+    const double fa = a.mode == A_S1 ? 2.0 * Av - At : (a.mode == A_S2 || a.mode == A_S3) ? Av : At;
     vh *= a.occ;  // the density sum holds sum |y|^2
     const double kA = kxv + fa;
     // T_a gbar = K_2 * gbar + (k+a) K_1 * gbar + (k+a)^2/2 gbar
     const zd tg = mk(c2.x + kA * c1.x + 0.5 * kA * kA * gv.x, c2.y + kA * c1.y + 0.5 * kA * kA * gv.y);
     // dL/da term: Re conj(gbar) P_a y, P_a y = K_1 * y + (k+a) y
-    stg[tid] = gv.x * (py.x + kA * yv.x) + gv.y * (py.y + kA * yv.y);
-    const double occr = out_occ ? a.occ : 0.0;
-    if (egrad) {
+    pterm = gv.x * (py.x + kA * yv.x) + gv.y * (py.y + kA * yv.y);
+    if constexpr (EG) {
       // dE/du = occ dv [2 (T y + (vion + vH) y) + (V_F + V'_F) y]
       const zd h = zadd(tg, zscal(yv, vionv + vh));
-      const zd c = zscal(zadd(zscal(h, 2.0), sACC[tid]), occr * a.dv);
+      const zd c = zscal(zadd(zscal(h, 2.0), sACC[tid]), a.occ * a.dv);
       gstore(a.cout + o, c);
       const double w = a.dt / 6.0;  // gbar_4 = i (dt/6) c
       gstore(a.gout + o, mk(-w * c.y, w * c.x));
     } else {
       zd vj = zadd(tg, zscal(gv, vionv + vh));
-      vj = zadd(vj, zscal(yv, 2.0 * a.occ * (ib < a.nbocc ? 1.0 : 0.0) * ks));
+      vj = zadd(vj, zscal(yv, 2.0 * a.occ * ks));
       vj = zadd(vj, sACC[tid]);
-      const zd ubv = gload(a.ub + o);
-      zd uav, kb;
+      zd kb;
       if (a.mode == A_S4) {
         uav = zadd(ubv, vj);
         kb = zadd(zscal(ubv, a.dt / 3.0), zscal(vj, a.dt));
       } else if (a.mode == A_S3) {
-        uav = zadd(gload(a.ua + o), vj);
+        uav = zadd(uav, vj);
         kb = zadd(zscal(ubv, a.dt / 3.0), zscal(vj, 0.5 * a.dt));
       } else if (a.mode == A_S2) {
-        uav = zadd(gload(a.ua + o), vj);
+        uav = zadd(uav, vj);
         kb = zadd(zscal(ubv, a.dt / 6.0), zscal(vj, 0.5 * a.dt));
       } else {  // A_S1: cotangent of the state before the step; next step's gbar_4
-        uav = zadd(gload(a.ua + o), vj);
+        uav = zadd(uav, vj);
         kb = zscal(uav, a.dt / 6.0);
       }
       gstore(a.ua + o, uav);
       gstore(a.gout + o, mk(-kb.y, kb.x));  // i * kbar
     }
   }
-  if (!egrad && a.abar) {
-    // fixed-order sum of the NG terms: chunks of 8, then the chunks
-    constexpr int NCH = (NG + 7) / 8;
-    lds_barrier();
-    if (tid < NCH) {
-      double s8 = 0.0;
-      for (int i = 0; i < 8 && 8 * tid + i < NG; ++i) s8 += stg[8 * tid + i];
-      sPart[tid] = s8;
-    }
-    lds_barrier();
-    if (tid == 0) {
-      double t = 0.0;
-      for (int c = 0; c < NCH; ++c) t += sPart[c];
-      gstore(a.abar + row, t);
+  if (!EG && a.abar) {
+    if constexpr (NG <= 64) {
+      const double t = wave_sum(pterm);
+      if (tid == 0) gstore(a.abar + row, t);
+    } else {
+      const double t = wave_sum(pterm);
+      if (lane == 0 && tid < NG) sRed[wave] = t;
+      lds_barrier();
+      if (tid == 0) gstore(a.abar + row, sRed[0] + sRed[1]);
     }
   }
 }

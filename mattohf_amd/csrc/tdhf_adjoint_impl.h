@@ -147,6 +147,14 @@ size_t adj_lds_for(int ng, int nw) {
 constexpr int kAdjTileEpiWaves = 4;
 constexpr int kAdjTileWaves = 8;  // adjtile_kernel<8>: 32-row tiles
 
+template <int NG>
+void launch_adj_t(const tdhf::AdjArgs& a, dim3 grid, dim3 block, size_t lds, hipStream_t s) {
+  if (a.mode == tdhf::A_EGRAD)
+    hipLaunchKernelGGL((tdhf::adjoint_kernel<NG, false, true>), grid, block, lds, s, a);
+  else
+    hipLaunchKernelGGL((tdhf::adjoint_kernel<NG>), grid, block, lds, s, a);
+}
+
 // One reverse stage.  With ts holding pair tiles (adj_tiles_setup) and a
 // stage mode, the exchange part comes from adjtile_kernel and
 // adjoint_kernel<128, true> finishes the stage; otherwise adjoint_kernel
@@ -225,10 +233,10 @@ int launch_adj(tdhf_ctx* c, const tdhf::AdjArgs& a, int ntraj, const AdjState* t
   }
   const dim3 grid(rows, ntraj), block(64 * nw);
   switch (c->ng) {
-    case 16: hipLaunchKernelGGL(tdhf::adjoint_kernel<16>, grid, block, lds, c->stream, a); break;
-    case 32: hipLaunchKernelGGL(tdhf::adjoint_kernel<32>, grid, block, lds, c->stream, a); break;
-    case 64: hipLaunchKernelGGL(tdhf::adjoint_kernel<64>, grid, block, lds, c->stream, a); break;
-    case 128: hipLaunchKernelGGL(tdhf::adjoint_kernel<128>, grid, block, lds, c->stream, a); break;
+    case 16: launch_adj_t<16>(a, grid, block, lds, c->stream); break;
+    case 32: launch_adj_t<32>(a, grid, block, lds, c->stream); break;
+    case 64: launch_adj_t<64>(a, grid, block, lds, c->stream); break;
+    case 128: launch_adj_t<128>(a, grid, block, lds, c->stream); break;
   }
   HIPCHK(c, hipGetLastError());
   if (c->timing) HIPCHK(c, hipEventRecord(e1, c->stream));
@@ -242,19 +250,32 @@ int adj_prepare(tdhf_ctx* c) {
   int nw = 8;
   while (nw > (c->ng + 63) / 64 && adj_lds_for(c->ng, nw) > 160 * 1024) --nw;
   const size_t lds = adj_lds_for(c->ng, nw);
-  const void* fn = nullptr;
+  if (lds <= 64 * 1024) return 0;
+  auto set = [lds](const void* fn) {
+    return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  };
   switch (c->ng) {
-    case 16: fn = (const void*)tdhf::adjoint_kernel<16>; break;
-    case 32: fn = (const void*)tdhf::adjoint_kernel<32>; break;
-    case 64: fn = (const void*)tdhf::adjoint_kernel<64>; break;
-    case 128: fn = (const void*)tdhf::adjoint_kernel<128>; break;
+    case 16:
+      HIPCHK(c, set((const void*)tdhf::adjoint_kernel<16>));
+      HIPCHK(c, set((const void*)tdhf::adjoint_kernel<16, false, true>));
+      break;
+    case 32:
+      HIPCHK(c, set((const void*)tdhf::adjoint_kernel<32>));
+      HIPCHK(c, set((const void*)tdhf::adjoint_kernel<32, false, true>));
+      break;
+    case 64:
+      HIPCHK(c, set((const void*)tdhf::adjoint_kernel<64>));
+      HIPCHK(c, set((const void*)tdhf::adjoint_kernel<64, false, true>));
+      break;
+    case 128:
+      HIPCHK(c, set((const void*)tdhf::adjoint_kernel<128>));
+      HIPCHK(c, set((const void*)tdhf::adjoint_kernel<128, false, true>));
+      break;
   }
-  if (lds > 64 * 1024)
-    HIPCHK(c, hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   return 0;
 }
 
-// Pair tiles for the reverse stages (NG = 128, every band occupied): the
+// Pair tiles for the reverse stages (NG = 128, large systems): the
 // partial buffers and the tile list of the record's trajectories, set up once
 // before the first reverse sweep.  Without device memory for them the
 // reverse stages stay row-wise (the same results to rounding).
@@ -264,6 +285,11 @@ int adj_tiles_setup(tdhf_ctx* c, AdjState& s) {
   if ((long)rows >= (1L << 22)) return 0;  // the kernel's float k-point division
   constexpr int TR = tdhf::adjtile_rows(kAdjTileWaves);
   const int nblk = (rows + TR - 1) / TR;
+  // A launch of up to one tile per CU takes 160 to 280 us however few it has
+  // (each tile holds 32 x 32 pairs), the row-wise kernel 21 us at 32 rows, 163 at
+  // 260, 240 at 390 (91 tiles) and 466 at 520 (153 tiles): tiles from half the
+  // CUs on.
+  if ((long)s.ntraj * nblk * (nblk + 1) < device_cus()) return 0;
   std::vector<int4> map;
   for (int pass = 0; pass < 2; ++pass)  // off-diagonal tiles (the costlier) first
     for (int t = 0; t < s.ntraj; ++t)
