@@ -143,49 +143,124 @@ __global__ void __launch_bounds__(256) dos_kernel(int nb, int nk, int nbocc, con
 }
 
 // FourierTr (window 0) / WindowFourierTr (window 1), src/RT_calculation.f90
-// :246-351: block iw computes omega = (iw+1)/nomega * omegam and the filtered
+// :246-351: omega = (iw+1)/nomega * omegam, iw = 0..nomega-1, and the filtered
 // transforms JF, EF, AF = sum_t e^{i omega t} filter (J - j0 | E | A) dt.
 // out[7 iw + ...] = omega, Re/Im JF, Re/Im EF, Re/Im AF.
-__global__ void __launch_bounds__(256) fourier_kernel(int nt, double dt, const double* time,
-                                                      const double* J, double j0,
-                                                      const double* E, const double* A,
-                                                      int nomega, double omegam, int window,
-                                                      double tpulse, int nenvelope, double* out) {
-  __shared__ double red[256];
-  const int iw = blockIdx.x;
-  const double w = (double)(iw + 1) / (double)nomega * omegam;
+//
+// A workgroup takes S frequencies, each thread the times tid, tid + 512, ...
+// Bound by FP64 operations, most of which were the sine and cosine of every
+// (omega, t).  Here a thread takes them of the centre c of its frequencies, and
+// of half their spacing h, once per t: the others are E(c) D and E(c) conj(D)
+// with D = e^{i (2m+1) h t} from products, the arguments c t and h t with their
+// rounding errors.  What is missing to the rounded product omega t, whose phase
+// the transform is made of, is x ~ 1e-13 and enters as 1 + i x, so the phases
+// are those of a sine and cosine of omega t to 1e-15.  4000 frequencies, 20000
+// times: 300 -> 98 us.
+constexpr int kFourierThreads = 512;
+
+// e^{i w t} with the rounding error of the product carried.
+__device__ __forceinline__ zd phase_of(double w, double t) {
+  const double p = w * t, e = fma(w, t, -p);
+  double sn, cs;
+  sincos(p, &sn, &cs);
+  return mk(fma(-e, sn, cs), fma(e, cs, sn));
+}
+
+template <int S>
+__global__ void __launch_bounds__(kFourierThreads)
+    fourier_kernel(int nt, double dt, const double* time, const double* J, double j0,
+                   const double* E, const double* A, int nomega, double omegam, int window,
+                   double tpulse, int nenvelope, double* out) {
+  static_assert(S == 1 || S % 2 == 0, "frequencies in pairs");
+  constexpr int NV = (6 * S + 15) / 16 * 16, VF = NV / 16, NW = kFourierThreads / 64;
+  constexpr int H = S / 2;  // pairs
+  __shared__ double red[NW * NV];
+  const int iw0 = blockIdx.x * S, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  auto freq = [&](int iw) { return (double)(iw + 1) / (double)nomega * omegam; };
   const double tn = time[nt - 1];
+  const double h = 0.5 * (omegam / (double)nomega);
+  const double wc = S == 1 ? freq(iw0) : ((double)(iw0 + 1) + 0.5 * (S - 1)) / (double)nomega * omegam;
+  // freq - wc -+ (2m+1) h, uniform: pair m is the frequencies H - 1 - m and H + m
+  double dl[S], wj[S];
+  auto uniform = [](double v) {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(v)));
+  };
+  static_for<0, S>([&](auto jc) {
+    constexpr int jj = decltype(jc)::value;
+    double d = 0.0;
+    if constexpr (S > 1) {
+      constexpr int m = jj < H ? H - 1 - jj : jj - H;
+      const double w = freq(iw0 + jj), step = (jj < H ? -1.0 : 1.0) * (2 * m + 1) * h;
+      const double a = w - wc, z = a - w;  // a + err = w - wc exactly
+      const double err = (w - (a - z)) + (-wc - z);
+      d = (a - step) + err;
+    }
+    dl[jj] = uniform(d);
+    wj[jj] = uniform(freq(iw0 + jj));
+  });
   int ntp = 0;
   if (window == 1) ntp = (int)fmin(tpulse / dt, (double)nt);
-  double s[6] = {0, 0, 0, 0, 0, 0};
-  for (int it = threadIdx.x; it < nt; it += 256) {
+  double s[NV];
+  static_for<0, NV>([&](auto kc) { s[decltype(kc)::value] = 0.0; });
+  for (int it = threadIdx.x; it < nt; it += kFourierThreads) {
+    const double t = time[it];
     double f;
     if (window == 0) {
-      const double r = time[it] / tn;
+      const double r = t / tn;
       f = 1.0 - 3.0 * r * r + 2.0 * r * r * r;
     } else if (it < ntp) {
-      const double sn = sin(M_PI * time[it] / tpulse);
+      const double sn = sin(M_PI * t / tpulse);
       f = 1.0;
       for (int k = 0; k < nenvelope; ++k) f *= sn;
     } else {
       f = 0.0;
     }
-    double sn, cs;
-    sincos(w * time[it], &sn, &cs);
     const double jt = f * (J[it] - j0), et = f * E[it], at = f * A[it];
-    s[0] += cs * jt;
-    s[1] += sn * jt;
-    s[2] += cs * et;
-    s[3] += sn * et;
-    s[4] += cs * at;
-    s[5] += sn * at;
+    auto add = [&](auto jc, zd ph) {
+      constexpr int jj = decltype(jc)::value;
+      if constexpr (S > 1) {
+        const double p = wj[jj] * t, x = fma(dl[jj], t, -fma(wj[jj], t, -p));
+        ph = mk(fma(-x, ph.y, ph.x), fma(x, ph.x, ph.y));
+      }
+      s[6 * jj + 0] = fma(ph.x, jt, s[6 * jj + 0]);
+      s[6 * jj + 1] = fma(ph.y, jt, s[6 * jj + 1]);
+      s[6 * jj + 2] = fma(ph.x, et, s[6 * jj + 2]);
+      s[6 * jj + 3] = fma(ph.y, et, s[6 * jj + 3]);
+      s[6 * jj + 4] = fma(ph.x, at, s[6 * jj + 4]);
+      s[6 * jj + 5] = fma(ph.y, at, s[6 * jj + 5]);
+    };
+    if constexpr (S == 1) {
+      double sn, cs;
+      sincos(wc * t, &sn, &cs);
+      add(std::integral_constant<int, 0>{}, mk(cs, sn));
+    } else {
+      const zd e = phase_of(wc, t);
+      zd d = phase_of(h, t);
+      const zd d2 = zmul(d, d);  // e^{2 i h t}
+      static_for<0, H>([&](auto mc) {
+        constexpr int m = decltype(mc)::value;
+        if constexpr (m > 0) d = zmul(d, d2);
+        const double xx = e.x * d.x, yx = e.y * d.x;
+        add(std::integral_constant<int, H - 1 - m>{}, mk(fma(e.y, d.y, xx), fma(-e.x, d.y, yx)));
+        add(std::integral_constant<int, H + m>{}, mk(fma(-e.y, d.y, xx), fma(e.x, d.y, yx)));
+      });
+    }
   }
-  double r[6];
-  for (int k = 0; k < 6; ++k) r[k] = sum256(s[k], red);
-  if (threadIdx.x == 0) {
-    double* o = out + (size_t)7 * iw;
-    o[0] = w;
-    for (int k = 0; k < 6; ++k) o[1 + k] = r[k] * dt;
+  // fixed-order sums: the lanes of a wave, then the waves
+  wave_reduce_scatter<4, NV>(s);
+  static_for<0, VF>([&](auto kc) {
+    constexpr int k = decltype(kc)::value;
+    s[k] += __shfl_xor(s[k], 1);
+    s[k] += __shfl_xor(s[k], 2);
+    if ((lane & 3) == 0) red[wave * NV + k + VF * (lane >> 2)] = s[k];
+  });
+  __syncthreads();
+  for (int v = threadIdx.x; v < 7 * S; v += kFourierThreads) {
+    const int jj = v / 7, c = v - 7 * jj, iw = iw0 + jj;
+    if (iw >= nomega) continue;
+    out[(size_t)7 * iw + c] =
+        c == 0 ? freq(iw) : ordered_sum(red + 6 * jj + c - 1, NV, NW) * dt;
   }
 }
 
