@@ -79,6 +79,7 @@ struct tdhf_ctx {
   // orbital buffers (NG*NB*NK complex each, NK padded to kn with kpath)
   zd *d_u0 = nullptr, *d_ksum = nullptr, *d_sa = nullptr, *d_sb = nullptr;
   zd *d_w = nullptr, *d_out = nullptr;
+  zd* h_stage = nullptr;  // three states in pinned memory, small systems (stage_in)
   // observables
   double* d_obs = nullptr;
   long obs_slots = 0;
@@ -673,6 +674,7 @@ void release(tdhf_ctx* c) {
   dfree(c->d_vq); dfree(c->d_vtl); dfree(c->d_tw); dfree(c->d_kc); dfree(c->d_vhg);
   dfree(c->d_u0); dfree(c->d_ksum); dfree(c->d_sa); dfree(c->d_sb);
   dfree(c->d_w); dfree(c->d_out);
+  if (c->h_stage) (void)hipHostFree(c->h_stage);
   dfree(c->d_ktab); dfree(c->d_ktw); dfree(c->d_om); dfree(c->d_hm); dfree(c->d_nx);
   dfree(c->d_obs); dfree(c->d_res); dfree(c->d_A); dfree(c->d_Aave); dfree(c->d_step);
   tdhf::gs_free(c->gs);
@@ -698,6 +700,42 @@ int ctx_fail(tdhf_ctx* c, int code, const char* msg) { return fail(c, code, "%s"
 // ---------------------------------------------------------------------------
 // C-ABI
 // ---------------------------------------------------------------------------
+namespace {
+
+// The four stages of RT_RK4_ubk on u0 (path's layout) with the fields as kernel
+// arguments: no step counter, field arrays or observables.
+int rk4_stages(tdhf_ctx* c, zd* u0, zd* ksum, zd* sa, zd* sb, double Aave, double A,
+               hipStream_t st, bool kp) {
+  tdhf::ApplyArgs a = base_args(c);
+  a.u0 = u0;
+  a.ksum = ksum;
+  const int rows = c->nb * c->nk;
+  const int modes[4] = {tdhf::M_S1, tdhf::M_S2, tdhf::M_S3, tdhf::M_S4};
+  const double fields[4] = {2.0 * Aave - A, Aave, Aave, A};
+  zd* ins[4] = {u0, sa, sb, sa};
+  zd* nexts[4] = {sa, sb, sa, nullptr};
+  for (int s = 0; s < 4; ++s) {
+    a.mode = modes[s];
+    a.A = a.Aobs = fields[s];
+    a.u = a.w = ins[s];
+    a.unext = nexts[s];
+    if (kp) {
+      CHKRET(launch_kspace(c, a, 1, st));
+      continue;
+    }
+    switch (c->ng) {
+      case 16: launch_apply_t<16>(a, rows, 1, c->nw, c->lds, st); break;
+      case 32: launch_apply_t<32>(a, rows, 1, c->nw, c->lds, st); break;
+      case 64: launch_apply_t<64>(a, rows, 1, c->nw, c->lds, st); break;
+      case 128: launch_apply_t<128>(a, rows, 1, c->nw, c->lds, st); break;
+    }
+    HIPCHK(c, hipGetLastError());
+  }
+  return 0;
+}
+
+}  // namespace
+
 extern "C" {
 
 const char* tdhf_last_error(const tdhf_ctx* c) { return c ? c->err.c_str() : g_err.c_str(); }
@@ -759,6 +797,11 @@ int tdhf_create(const tdhf_params* p, const double* vion, const double* vcg, con
       hipMemcpy(c->d_vion, vion, c->ng * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
     fail(c, TDHF_EDEVICE, "table upload failed");
     return bail(TDHF_EDEVICE);
+  }
+  if (nstate(c) <= kStageState &&
+      hipHostMalloc((void**)&c->h_stage, 3 * nstate(c) * sizeof(zd), 0) != hipSuccess) {
+    c->h_stage = nullptr;  // without it: copies from and to the caller's arrays
+    (void)hipGetLastError();
   }
   if ((rc = build_tables(c, vcg, vcgkk))) return bail(rc);
   if (c->kn && (rc = kspace_tables(c))) return bail(rc);
@@ -826,10 +869,11 @@ int tdhf_get_tables(tdhf_ctx* c, double* vcg, double* vq) {
 int tdhf_hpsi(tdhf_ctx* c, const double* u, const double* w, double A, double* hw) {
   if (!c) return fail(nullptr, TDHF_EINVAL, "ctx is NULL");
   if (!u || !w || !hw) return fail(c, TDHF_EINVAL, "NULL array");
-  CHKRET(upload_state(c, c->d_sa, u));
-  CHKRET(upload_state(c, c->d_w, w));
-  CHKRET(path_hpsi(c, c->d_sa, c->d_w, A, c->d_out));
-  CHKRET(download_state(c, hw, c->d_out));
+  CHKRET(stage_in(c, c->d_sa, u, c->d_w, w));
+  // (row-wise, the result goes straight to the pinned memory)
+  zd* out = c->h_stage && !c->kpath ? c->h_stage + 2 * nstate(c) : c->d_out;
+  CHKRET(path_hpsi(c, c->d_sa, c->d_w, A, out));
+  CHKRET(stage_out(c, hw, out));
   return sync(c);
 }
 
@@ -964,17 +1008,10 @@ int tdhf_rt_run(tdhf_ctx* c, double* u, int nt, const double* A, const double* A
 int tdhf_rk4_step(tdhf_ctx* c, double* u, double Aave, double A) {
   if (!c) return fail(nullptr, TDHF_EINVAL, "ctx is NULL");
   if (!u) return fail(c, TDHF_EINVAL, "NULL array");
-  CHKRET(tdhf_state_upload(c, u));
-  CHKRET(ensure_obs(c, 2));
-  CHKRET(ensure_field(c, 1));
-  HIPCHK(c, hipMemcpyAsync(c->d_A, &A, sizeof A, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipMemcpyAsync(c->d_Aave, &Aave, sizeof Aave, hipMemcpyHostToDevice, c->stream));
-  const int zero = 0;
-  HIPCHK(c, hipMemcpyAsync(c->d_step, &zero, sizeof zero, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  CHKRET(enqueue_steps(c, 0, 1));
-  CHKRET(sync(c));
-  return tdhf_state_download(c, u);
+  CHKRET(stage_in(c, c->d_u0, u));
+  c->u0_padded = c->kpath;
+  CHKRET(rk4_stages(c, c->d_u0, c->d_ksum, c->d_sa, c->d_sb, Aave, A, c->stream, c->kpath));
+  return stage_out(c, u, c->d_u0);
 }
 
 int tdhf_rk4_step_noalloc(tdhf_ctx* c, double* u, double Aave, double A, void* stream) {
@@ -1000,33 +1037,7 @@ int tdhf_rk4_step_noalloc(tdhf_ctx* c, double* u, double Aave, double A, void* s
     u0 = sb + kNoAllocSlot;
     CHKRET(kspace_layout(c, reinterpret_cast<zd*>(u), u0, true, 1, st));
   }
-  // the four stages of RT_RK4_ubk with the fields as kernel arguments
-  // (no step counter, no field arrays, no observables)
-  tdhf::ApplyArgs a = base_args(c);
-  a.u0 = u0;
-  a.ksum = ksum;
-  const int rows = c->nb * c->nk;
-  const int modes[4] = {tdhf::M_S1, tdhf::M_S2, tdhf::M_S3, tdhf::M_S4};
-  const double fields[4] = {2.0 * Aave - A, Aave, Aave, A};
-  zd* ins[4] = {u0, sa, sb, sa};
-  zd* nexts[4] = {sa, sb, sa, nullptr};
-  for (int s = 0; s < 4; ++s) {
-    a.mode = modes[s];
-    a.A = a.Aobs = fields[s];
-    a.u = a.w = ins[s];
-    a.unext = nexts[s];
-    if (kp) {
-      CHKRET(launch_kspace(c, a, 1, st));
-      continue;
-    }
-    switch (c->ng) {
-      case 16: launch_apply_t<16>(a, rows, 1, c->nw, c->lds, st); break;
-      case 32: launch_apply_t<32>(a, rows, 1, c->nw, c->lds, st); break;
-      case 64: launch_apply_t<64>(a, rows, 1, c->nw, c->lds, st); break;
-      case 128: launch_apply_t<128>(a, rows, 1, c->nw, c->lds, st); break;
-    }
-    HIPCHK(c, hipGetLastError());
-  }
+  CHKRET(rk4_stages(c, u0, ksum, sa, sb, Aave, A, st, kp));
   if (kp) CHKRET(kspace_layout(c, u0, reinterpret_cast<zd*>(u), false, 1, st));
   return 0;
 }

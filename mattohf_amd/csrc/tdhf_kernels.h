@@ -781,6 +781,13 @@ __global__ void __launch_bounds__(512, NG == 16 ? 4 : 2) apply_kernel(ApplyArgs 
   }
 }
 
+// d0 = the first n elements of src, d1 = the next m - n.
+__global__ void __launch_bounds__(256) stage_kernel(const zd* src, zd* d0, zd* d1, long n,
+                                                    long m) {
+  const long i = blockIdx.x * 256L + threadIdx.x;
+  if (i < m) gstore(i < n ? d0 + i : d1 + (i - n), gload(src + i));
+}
+
 // Twiddle tables of GroupFFT<NG> (2*NG complex).
 template <int NG>
 __global__ void twiddle_kernel(zd* tw) {

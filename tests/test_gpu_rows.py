@@ -52,3 +52,18 @@ def test_row_adjoint_matches_oracle(case):
         assert np.abs(g[0] - ref[1]).max() < 1e-9 * np.abs(ref[1]).max()
         assert np.abs(gu[0] - ref[2]).max() < 1e-9 * np.abs(ref[2]).max()
     G.close()
+
+
+# 16384 elements, the largest state that goes through pinned memory, row-wise
+# and on the density-matrix path, and one beyond
+@pytest.mark.parametrize("case", [(128, 16, 8, 2) + A128, (64, 32, 8, 8) + A64,
+                                  (128, 17, 8, 2) + A128], ids=lambda c: f"ng{c[0]}_nk{c[1]}")
+def test_staged_calls_match_oracle(case):
+    S, O, G, _ = system(case)
+    with G:
+        for seed in (1, 2):  # (the memory is used again)
+            u, w = orbitals(case, seed), orbitals(case, 10 + seed)
+            assert rel(G.ubkwbk_hwbk(u, w, 0.2), O.ubkwbk_hwbk(u, w, 0.2)) < 1e-12
+            ref = O.RT_RK4_ubk(u, G.dt, 0.05, 0.1)
+            assert rel(G.RT_RK4_ubk(u, 0.05, 0.1), ref) < 1e-12
+            np.testing.assert_array_equal(G.download(), G.RT_RK4_ubk(u, 0.05, 0.1))
