@@ -850,18 +850,27 @@ int tdhf_batch_create(const tdhf_params* p, int ntraj, const int* nk, const doub
     bfail(b, TDHF_EDEVICE, "vion upload failed");
     return bail(TDHF_EDEVICE);
   }
-  // launch shape and row schedule: the cached autotuner choice, else the
-  // fewest waves per workgroup that cover the grid (one at NG <= 64: the
+  // launch shape and row schedule: the cached autotuner choice, else, row-wise,
+  // the fewest waves per workgroup that cover the grid (one at NG <= 64: the
   // groups of a single wave need no workgroup barrier, and eight such
-  // workgroups share a CU) and the XCD-pinned schedule
+  // workgroups share a CU) and the XCD-pinned schedule; two waves for up to four
+  // rows per CU (NG=64, 558 rows: 16.8 -> 14.7 us per stage; NG=16, 800: 8.1 ->
+  // 7.7), and for up to two rows per CU, whose CUs have room, four and the rows
+  // spread over all XCDs (NG=64, 93 rows: 15.7 -> 7.8; 279: 16.3 -> 9.4; NG=32,
+  // 156: 9.1 -> 6.8; 312: 9.5 -> 8.7)
   std::array<int, 3> ct{};
   const bool cached = tune_lookup(tune_key(b), &ct);
   // (density matrices: 8 waves for the product launch, 4 where it has
   // workgroups enough; fewer trajectories than XCDs are not pinned to them,
   // NG=128, NK=128, NB=8: 4 trajectories 166 us per stage pinned, 101 not)
-  b->nw = cached ? ct[0] : !b->kuse ? (p->ng + 63) / 64 : batch_points(b) > 1 ? 4 : 8;
+  const long rows = (long)p->nb * std::accumulate(nk, nk + ntraj, 0L), cus = device_cus();
+  const int fit = choose_nw(p->ng, *std::max_element(nk, nk + ntraj), p->nbocc);
+  const int nwr = std::max((p->ng + 63) / 64,
+                           std::min(fit, rows <= 2 * cus ? 4 : rows <= 4 * cus ? 2 : 1));
+  b->nw = cached ? ct[0] : !b->kuse ? nwr : batch_points(b) > 1 ? 4 : 8;
   b->ngrid = 0;
-  if ((rc = batch_set_schedule(b, cached ? ct[1] : b->kuse && ntraj < 8 ? 2 : 0)))
+  if ((rc = batch_set_schedule(
+           b, cached ? ct[1] : (b->kuse ? ntraj < 8 : rows <= 2 * cus) ? 2 : 0)))
     return bail(rc);
   b->h_td.resize(ntraj);
   if ((rc = batch_update_desc(b))) return bail(rc);

@@ -5,6 +5,7 @@ tolerances of the density-matrix path's tests."""
 import numpy as np
 import pytest
 
+from mattohf_amd import tdhf as T
 from test_gpu_kspace import orbitals, rel, system
 
 pytestmark = pytest.mark.gpu
@@ -67,3 +68,29 @@ def test_staged_calls_match_oracle(case):
             ref = O.RT_RK4_ubk(u, G.dt, 0.05, 0.1)
             assert rel(G.RT_RK4_ubk(u, 0.05, 0.1), ref) < 1e-12
             np.testing.assert_array_equal(G.download(), G.RT_RK4_ubk(u, 0.05, 0.1))
+
+
+# up to two rows per CU (512), up to four, more; one pair in all; NG = 128, which
+# needs two waves
+@pytest.mark.parametrize("ng,nb,nks,ntraj", [(32, 2, [7, 12, 20], 6), (32, 2, [7, 12, 20], 30),
+                                             (16, 3, [5, 9, 4], 80), (64, 1, [1], 3),
+                                             (128, 2, [3, 5], 40)])
+def test_default_batch_shape(ng, nb, nks, ntraj):
+    a, z = {16: A16, 32: A32, 64: A64, 128: A128}[ng]
+    nk = [nks[t % len(nks)] for t in range(ntraj)]
+    vi = {k: T.ion_potential(ng, k, a, [z], [1.0], [0.0]) for k in nks}
+    rng = np.random.default_rng(3)
+    A = 0.1 * rng.standard_normal((ntraj, 3))
+    us = [orbitals((ng, k, nb, nb, a, z), t) for t, k in enumerate(nk)]
+    with T.Batch(ng, nb, nb, a, 0.004, nk, np.array([vi[k] for k in nk])) as B:
+        out = []
+        for shape in (None, (ng + 63) // 64):
+            if shape:
+                B.set_schedule(0)
+                B.set_waves(shape)
+            B.upload(us)
+            e, n, j, _ = B.propagate(A, A)
+            out.append((B.download(), e, j))
+    for u, v in zip(out[0][0], out[1][0]):
+        assert rel(u, v) < 1e-12
+    assert np.abs(out[0][1] - out[1][1]).max() < 1e-10 and rel(out[0][2], out[1][2]) < 1e-8
