@@ -592,8 +592,9 @@ int build_tables(tdhf_ctx* c, const double* vcg, const double* vcgkk) {
     const double dx = c->acell / (double)NG / 20.0;
     const long ns = kvck_nsteps(c->acell, NG, NK);
     if (e == hipSuccess) {
-      hipLaunchKernelGGL(tdhf::kvck_kernel, dim3((unsigned)q.size()), dim3(256), 0, c->stream,
-                         d_q, dx, ns, d_v);
+      constexpr int per = tdhf::kVckArgs;
+      hipLaunchKernelGGL(tdhf::kvck_kernel, dim3((unsigned)((q.size() + per - 1) / per)),
+                         dim3(256), 0, c->stream, d_q, (int)q.size(), dx, ns, d_v);
       e = hipGetLastError();
     }
     if (e == hipSuccess && !vcgkk)

@@ -260,8 +260,8 @@ __host__ __device__ constexpr size_t apply_lds_bytes(int nw) {
 // a graph takes 1.6 us: the arguments, one round trip to memory, the transforms
 // of one pair, two reductions, the stores.  So each link has one wait: scalar
 // loads in one batch, field values and twiddles off the way of the operands,
-// sums whose reads go ahead.  Per RK4 stage, against one
-// batch per use and one read per product:
+// sums whose reads go ahead.  Per RK4 stage, against one batch per use and one
+// read per product:
 //   NG 16, 40 k-points, 8 bands, 1 occupied   5.55 -> 4.93 us
 //   NG 32, 32 k-points, 2 bands               7.51 -> 5.80 us
 //   NG 64, 21 k-points, 3 bands               8.55 -> 7.14 us
@@ -888,25 +888,45 @@ __global__ void step_set_kernel(int* step_base, int value) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *step_base = value;
 }
 
-// k_vCk (src/Functions.f90:33-52) for a list of arguments: one workgroup per
-// argument, the nsteps trapezoid terms split over the threads and summed by
-// a fixed-shape tree (deterministic).
-__global__ void __launch_bounds__(256) kvck_kernel(const double* q, double dx, long nsteps,
+// k_vCk (src/Functions.f90:33-52) for a list of n arguments: four per workgroup,
+// the nsteps trapezoid terms split over the threads and summed by a fixed-shape
+// tree (deterministic).  Bound by FP64 operations (the cosine of every term), so
+// each end of the steps is evaluated once and its 1/sqrt serves four arguments:
+// a context of NG=128, NK=128 is made in 24 ms (59 with both ends of every step
+// for one argument at a time).
+constexpr int kVckArgs = 4;
+__global__ void __launch_bounds__(256) kvck_kernel(const double* q, int n, double dx, long nsteps,
                                                    double* out) {
-  __shared__ double red[256];
-  const double k = q[blockIdx.x];
-  double s = 0.0;
-  for (long ix = threadIdx.x; ix < nsteps; ix += blockDim.x) {
-    const double x0 = (double)ix * dx, x1 = (double)(ix + 1) * dx;
-    s += 0.5 * (cos(k * x0) / sqrt(x0 * x0 + 1.0) + cos(k * x1) / sqrt(x1 * x1 + 1.0));
+  __shared__ double red[kVckArgs][256];
+  const int a0 = blockIdx.x * kVckArgs, t = threadIdx.x;
+  double k[kVckArgs], s[kVckArgs];
+  static_for<0, kVckArgs>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    k[i] = q[a0 + i < n ? a0 + i : n - 1];
+    s[i] = 0.0;
+  });
+  for (long ix = t; ix <= nsteps; ix += 256) {
+    const double x = (double)ix * dx;
+    const double r = (ix == 0 || ix == nsteps ? 0.5 : 1.0) / sqrt(x * x + 1.0);
+    static_for<0, kVckArgs>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      s[i] += cos(k[i] * x) * r;
+    });
   }
-  red[threadIdx.x] = s;
+  static_for<0, kVckArgs>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    red[i][t] = s[i];
+  });
   __syncthreads();
   for (int h = 128; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
+    if (t < h)
+      static_for<0, kVckArgs>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        red[i][t] += red[i][t + h];
+      });
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[blockIdx.x] = 2.0 * red[0] * dx;
+  if (t < kVckArgs && a0 + t < n) out[a0 + t] = nsteps > 0 ? 2.0 * red[t][0] * dx : 0.0;
 }
 
 // Rearranges a raw table t[d*NG + g] into the G layout of GroupFFT<NG>,

@@ -11,7 +11,7 @@ namespace {
 // Row-wise: 5.5 + 0.42 per 10^6 grid points in the pair transforms, weighted by
 // log2 NG.  Density matrices: 13 (two launches, each with its own memory round
 // trips) + 12 per 10^6 matrix elements.  Near the line: NG=64, NK=64, NB=4
-// (one trajectory) 15.5 against 16.0 stays row-wise; NG=128, NK=64, NB=4 32.5
+// (one trajectory) 14.4 against 16.0 stays row-wise; NG=128, NK=64, NB=4 32.5
 // against 27.8 does not.
 struct KspaceCost {
   double rows = 0.0, mat = 0.0;
