@@ -167,7 +167,7 @@ def batch_pulses(ntraj, nt, dt, T, seed):
 def batch_bench(cfg, nks, steps, warmup, seed, gs_iters=60, autotune=True, exchange=None):
     """Batched run of len(nks) trajectories (NG, NB, a, Z of cfg; NK per
     trajectory).  Each trajectory starts from the ground state of its NK.
-    exchange (0 row-wise; 1, 2, 3 pair tiles of 64, 32, 16 rows) fixes the
+    exchange (0 direct; 1, 2, 3 pair tiles of 64, 32, 16 rows) fixes the
     exchange evaluation, with one wave per workgroup and the interleaved row
     schedule, instead of the autotuner's choice (for profiling runs)."""
     from mattohf_amd import tdhf as T
@@ -221,7 +221,8 @@ def batch_bench(cfg, nks, steps, warmup, seed, gs_iters=60, autotune=True, excha
         "frac": f_launch / avg_s / 1e12 / PEAK_FP64_TFLOPS,
         "flop_basis": "the reference algorithm's count (all NK^2 NB NBocc ordered exchange "
                       "pairs per H application); pair tiles run one transform pair per "
-                      "unordered pair, so they execute fewer FP64 operations than this basis",
+                      "unordered pair and the density matrices none, so they execute fewer "
+                      "FP64 operations than this basis",
         "observables_finite": bool(np.isfinite(e).all() and np.isfinite(j).all()),
     }
 
@@ -567,8 +568,8 @@ def batched_full_bench(nt=10000, ntraj=256, seed=20261202, gs_iters=60):
         "observables_finite": bool(np.isfinite(e).all() and np.isfinite(j).all()),
         "N_rel_drift_max": float(np.abs(n - n[:, :1]).max() / np.abs(n[:, :1]).min()),
         "vs_single_runs": checks,
-        "vs_single_note": "one trajectory per NK through tdhf_rt_run on its own context "
-                          "(row-wise exchange), the whole run",
+        "vs_single_note": "one trajectory per NK through tdhf_rt_run on its own context, "
+                          "the whole run",
     }
 
 

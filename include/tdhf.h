@@ -243,11 +243,11 @@ int tdhf_bwd(tdhf_ctx* ctx, double* dLdA, double* dLdu0);
  * initial orbitals and field each; same NK, tables and ion potential), one
  * launch per RK4 stage for all of them (adjoint stages likewise), with either
  * objective.  The memory budget covers the stage states of all trajectories.
- * At NG = 128 the backward call evaluates the reverse stages by pair tiles
- * (one pair of transforms per unordered pair of rows) and allocates their
- * partial sums outside the budget, ntraj * NK*NB * ceil(NK*NB/32) * NG * 16
- * bytes (2.1 GB for 32 trajectories at NK = 128, NB = 8); without that
- * memory it evaluates them row-wise (the same results to rounding).
+ * At NG = 128 a large system whose exchange does not run through the density
+ * matrices below has its reverse stages evaluated by pair tiles (one pair of
+ * transforms per unordered pair of rows), whose partial sums are allocated
+ * outside the budget, ntraj * NK*NB * ceil(NK*NB/32) * NG * 16 bytes; without
+ * that memory row-wise (the same results to rounding).
  * Where the exchange runs through the density matrices of the k-points (large
  * cells or many trajectories; NK <= 128), their matrices are allocated outside
  * the budget too, 32 * NG * (NG+1) * N bytes per trajectory with N = NK rounded
