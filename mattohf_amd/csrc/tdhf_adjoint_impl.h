@@ -416,8 +416,8 @@ int launch_jgrad(tdhf_ctx* c, const AdjState& s, int step, const zd* y, zd* ua, 
     j.blk = (size_t)s.ntraj * nstate(c);
   }
   if (s.kp) {  // the start; the steps' terms are part of launch_kadj's stage 1
-    hipLaunchKernelGGL(tdhf::kadj_jinit_kernel, dim3(c->ng, s.ntraj), dim3(256), 0, c->stream, j,
-                       c->ng, c->kn);
+    hipLaunchKernelGGL(tdhf::kadj_jinit_kernel, dim3(c->ng, s.ntraj, (c->nb * c->kn + 255) / 256),
+                       dim3(256), 0, c->stream, j, c->ng, c->kn);
     HIPCHK(c, hipGetLastError());
     return 0;
   }

@@ -412,25 +412,31 @@ __global__ void __launch_bounds__(512, 2) kadj_apply_kernel(KAdjArgs ka) {
 
 // Start of the reverse sweep of the current-squared objective, at the final
 // state y: ua = c, gb = i (dt/6) c with c = 2 dt J (-2 occ dv/vcell) P_A y,
-// P_A y = K_1 * y + (k + A) y; one thread per (band, k) at x (once per call).
+// P_A y = K_1 * y + (k + A) y; one thread per (band, k) at x (once per call),
+// blocks of them in grid z.  Bound by the latency of the reads of y, sixteen in
+// flight: three states of NG=128, NK=128, NB=8 128 -> 36 us against one block
+// of threads per x and one read at a time.
 __global__ void __launch_bounds__(256) kadj_jinit_kernel(JgradArgs j, int ng, int n) {
-  const int x = blockIdx.x, tr = blockIdx.y;
+  __shared__ zd sK1[128];
+  const int x = blockIdx.x, tr = blockIdx.y, q = blockIdx.z * 256 + threadIdx.x;
   const size_t so = (size_t)tr * j.tstride;
+  const int m = j.nb * n;
+  for (int i = threadIdx.x; i < ng; i += 256)
+    sK1[i] = gload(reinterpret_cast<const zd*>(j.kc + 2 * ng) + i);
   const double A = j.Aarr[(size_t)tr * j.fstride + j.step];
   const double J = j.J[(size_t)tr * j.fstride + j.step];
   const double f = 2.0 * j.dt * J * (-2.0 * j.occ * j.dv / j.vcell);
-  const int m = j.nb * n;
-  for (int q = threadIdx.x; q < m; q += blockDim.x) {
-    const size_t o = so + (size_t)x * m + q;
-    zd p = zscal(gload(j.y + o), gload(j.kx + q % n) + A);
-    for (int xp = 0; xp < ng; ++xp)
-      zfma(p, gload(reinterpret_cast<const zd*>(j.kc + 2 * ng) + ((x - xp) & (ng - 1))),
-           gload(j.y + so + (size_t)xp * m + q));
-    const zd c = zscal(p, f);
-    const double w = j.dt / 6.0;
-    gstore(j.ua + o, c);
-    gstore(j.gb + o, mk(-w * c.y, w * c.x));
-  }
+  lds_barrier();
+  if (q >= m) return;
+  const size_t o = so + (size_t)x * m + q;
+  zd p = zscal(gload(j.y + o), gload(j.kx + q % n) + A);
+#pragma unroll 16
+  for (int xp = 0; xp < ng; ++xp)
+    zfma(p, sK1[(x - xp) & (ng - 1)], gload(j.y + so + (size_t)xp * m + q));
+  const zd c = zscal(p, f);
+  const double w = j.dt / 6.0;
+  gstore(j.ua + o, c);
+  gstore(j.gb + o, mk(-w * c.y, w * c.x));
 }
 
 }  // namespace tdhf
