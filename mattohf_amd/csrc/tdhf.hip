@@ -242,7 +242,7 @@ void launch_apply_t(const tdhf::ApplyArgs& a, int rows, int ntraj, int nw, size_
   tdhf::ApplyArgs b = a;
   // wave-priority balancing pays only when the grid is one workgroup per CU
   b.balance = (long)rows * ntraj <= device_cus() ? 1 : 0;
-  if constexpr (NG >= 64) {
+  if constexpr (NG == 128) {
     if (tdhf::apply_by_transforms<NG>(nw)) {
       hipLaunchKernelGGL((tdhf::apply_kernel<NG, true>), dim3(rows, ntraj), dim3(64 * nw), lds, s,
                          b);
@@ -264,10 +264,7 @@ hipError_t set_apply_lds_limit(int ng) {
   switch (ng) {
     case 16: return set((const void*)tdhf::apply_kernel<16, false>);
     case 32: return set((const void*)tdhf::apply_kernel<32, false>);
-    case 64: {
-      const hipError_t e = set((const void*)tdhf::apply_kernel<64, false>);
-      return e != hipSuccess ? e : set((const void*)tdhf::apply_kernel<64, true>);
-    }
+    case 64: return set((const void*)tdhf::apply_kernel<64, false>);
     case 128: {
       const hipError_t e = set((const void*)tdhf::apply_kernel<128, false>);
       return e != hipSuccess ? e : set((const void*)tdhf::apply_kernel<128, true>);

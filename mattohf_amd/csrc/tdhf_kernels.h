@@ -17,8 +17,7 @@
 //     K_2(d) = 1/NG sum_G G^2/2 cos(2 pi g d/NG),
 //     K_1(d) = 1/NG sum_G G exp(2 pi i g d/NG)
 // (G in FFT order, Nyquist at -NG/2 b), by all threads of the workgroup, or,
-// when that would leave each thread 32 terms or more (workgroups of one or
-// two waves, NG = 128), as one transform round trip each,
+// at NG = 128 with fewer than four waves, as one transform round trip each,
 //     vH = occ IFFT[vCG/NG . FFT[rho]],   T w = IFFT[(G+k+A)^2/(2 NG) . FFT[w]],
 // on two groups of the first wave.  The epilogue forms
 // H w = T w + (vH + vion) w + V_F w (ubkwbk_hwbk, :187-209) and applies the
@@ -269,10 +268,13 @@ __host__ __device__ constexpr size_t apply_lds_bytes(int nw) {
 //   NG 128, 16 k-points, 4 bands              13.75 -> 12.8 us
 //
 // TE: the Hartree and kinetic round trips as transforms (else circulant
-// products); the launcher chooses (apply_by_transforms).
+// products); the launcher chooses: transforms where the 1024 blocks of the
+// products at NG = 128 meet few waves.  Per stage, transforms against products: NG = 128
+// with two waves 7.3 against 8.2 us, four 8.0 against 7.8, eight 12.8 against
+// 12.5; NG = 64 with one wave 6.3 against 6.0, two 6.45 against 5.6.
 template <int NG>
 __host__ __device__ constexpr bool apply_by_transforms(int nw) {
-  return NG >= 64 && NG >= 32 * (64 * nw / NG);
+  return NG == 128 && nw < 4;
 }
 
 template <int NG, bool TE>
