@@ -107,8 +107,9 @@ int tdhf_rk4_step(tdhf_ctx* ctx, double* u, double Aave, double A);
  * library (16 MiB per GPU, held until the process ends): NG*NB*NK must not
  * exceed 131072 (TDHF_EINVAL otherwise).  The call allocates nothing; the
  * context (tables) must have been created before.  All calls on one GPU share
- * that array, so calls whose launches overlap on one GPU (other streams,
- * other host threads) race. */
+ * that array, so calls of this function whose launches overlap on one GPU
+ * (other streams, other host threads) race.  Other calls on the context may
+ * overlap with them: they share nothing that either writes. */
 int tdhf_rk4_step_noalloc(tdhf_ctx* ctx, double* u, double Aave, double A, void* stream);
 
 /* nt RK4 steps with the observables after every step.  Replaces the loop of

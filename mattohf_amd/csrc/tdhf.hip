@@ -76,6 +76,10 @@ struct tdhf_ctx {
   zd *d_ktab = nullptr, *d_ktw = nullptr, *d_om = nullptr;
   zd* d_hm = nullptr;      // matrices of a stage
   double* d_nx = nullptr;  // density and partial observables of a stage
+  // the same of tdhf_rk4_step_noalloc, whose launches run on the caller's stream
+  // beside those of this context's
+  zd* d_hm_step = nullptr;
+  double* d_nx_step = nullptr;
   // orbital buffers (NG*NB*NK complex each, NK padded to kn with kpath)
   zd *d_u0 = nullptr, *d_ksum = nullptr, *d_sa = nullptr, *d_sb = nullptr;
   zd *d_w = nullptr, *d_out = nullptr;
@@ -674,6 +678,7 @@ void release(tdhf_ctx* c) {
   dfree(c->d_w); dfree(c->d_out);
   if (c->h_stage) (void)hipHostFree(c->h_stage);
   dfree(c->d_ktab); dfree(c->d_ktw); dfree(c->d_om); dfree(c->d_hm); dfree(c->d_nx);
+  dfree(c->d_hm_step); dfree(c->d_nx_step);
   dfree(c->d_obs); dfree(c->d_res); dfree(c->d_A); dfree(c->d_Aave); dfree(c->d_step);
   tdhf::gs_free(c->gs);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -701,9 +706,10 @@ int ctx_fail(tdhf_ctx* c, int code, const char* msg) { return fail(c, code, "%s"
 namespace {
 
 // The four stages of RT_RK4_ubk on u0 (path's layout) with the fields as kernel
-// arguments: no step counter, field arrays or observables.
+// arguments: no step counter, field arrays or observables.  sc: matrices other
+// than the context's.
 int rk4_stages(tdhf_ctx* c, zd* u0, zd* ksum, zd* sa, zd* sb, double Aave, double A,
-               hipStream_t st, bool kp) {
+               hipStream_t st, bool kp, const KScratch* sc = nullptr) {
   tdhf::ApplyArgs a = base_args(c);
   a.u0 = u0;
   a.ksum = ksum;
@@ -718,7 +724,7 @@ int rk4_stages(tdhf_ctx* c, zd* u0, zd* ksum, zd* sa, zd* sb, double Aave, doubl
     a.u = a.w = ins[s];
     a.unext = nexts[s];
     if (kp) {
-      CHKRET(launch_kspace(c, a, 1, st));
+      CHKRET(launch_kspace(c, a, 1, st, sc));
       continue;
     }
     switch (c->ng) {
@@ -803,6 +809,12 @@ int tdhf_create(const tdhf_params* p, const double* vion, const double* vcg, con
   }
   if ((rc = build_tables(c, vcg, vcgkk))) return bail(rc);
   if (c->kn && (rc = kspace_tables(c))) return bail(rc);
+  if (c->kpath && nstate(c) <= kNoAllocMaxState && kcount(c) <= kNoAllocSlot &&
+      (dalloc(c, &c->d_hm_step, tdhf::kmat_elems(c->ng, c->kn)) ||
+       dalloc(c, &c->d_nx_step, tdhf::kmat_extra(c->ng, kspace_gpw(c->kn))))) {
+    dfree(c->d_hm_step);
+    (void)hipGetLastError();
+  }
   {
     const hipError_t e = set_apply_lds_limit(c->ng);
     if (e != hipSuccess && c->lds > 64 * 1024) {
@@ -1028,14 +1040,16 @@ int tdhf_rk4_step_noalloc(tdhf_ctx* c, double* u, double Aave, double A, void* s
   zd* sb = sa + kNoAllocSlot;
   zd* u0 = reinterpret_cast<zd*>(u);
   hipStream_t st = stream ? static_cast<hipStream_t>(stream) : c->stream;
-  // padded k-points: the step runs on a copy in that layout (row-wise if the
-  // padding does not fit the array)
-  const bool kp = c->kpath && kcount(c) <= kNoAllocSlot;
+  // padded k-points: the step runs on a copy in that layout, with matrices of
+  // its own, since calls on the context's stream may run meanwhile (row-wise if
+  // the padding does not fit the array or there was no memory for the matrices)
+  const bool kp = c->d_hm_step != nullptr;
+  const KScratch own = {c->d_hm_step, c->d_nx_step, 0, 0};
   if (kp) {
     u0 = sb + kNoAllocSlot;
     CHKRET(kspace_layout(c, reinterpret_cast<zd*>(u), u0, true, 1, st));
   }
-  CHKRET(rk4_stages(c, u0, ksum, sa, sb, Aave, A, st, kp));
+  CHKRET(rk4_stages(c, u0, ksum, sa, sb, Aave, A, st, kp, &own));
   if (kp) CHKRET(kspace_layout(c, u0, reinterpret_cast<zd*>(u), false, 1, st));
   return 0;
 }

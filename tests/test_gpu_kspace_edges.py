@@ -1,0 +1,34 @@
+"""Calls at the edges of the density-matrix path (tdhf_kspace.h): launch shapes,
+numbers of columns and trajectories, memory, timing.  The systems are well over
+the line from which the library takes the path (twice the row-wise cost or
+more, except where a test says otherwise).  Tolerances as in
+test_gpu_kspace.py."""
+import numpy as np
+import pytest
+
+from mattohf_amd import tdhf as T
+from test_gpu_kspace import orbitals, rel
+
+pytestmark = pytest.mark.gpu
+
+CELL = {16: (3.6, 1.0), 32: (8.0, 4.0), 64: (10.0, 6.0), 128: (12.0, 6.0)}
+
+
+@pytest.mark.parametrize("ng,nk,nb,ntraj", [(64, 64, 4, 9), (16, 16, 4, 16)])
+def test_waves_that_are_no_power_of_two(ng, nk, nb, ntraj):
+    """3, 5, 6 and 7 waves of the product launch: the points do not divide among
+    them, the results are those of 1, 2, 4 and 8."""
+    a, z = CELL[ng]
+    vion = T.ion_potential(ng, nk, a, [z], [1.0], [0.0])
+    A = 0.1 * np.random.default_rng(1).standard_normal((ntraj, 2))
+    us = [orbitals((ng, nk, nb, nb, a, z), t) for t in range(ntraj)]
+    with T.Batch(ng, nb, nb, a, 0.004, [nk] * ntraj, np.array([vion] * ntraj)) as B:
+        out = {}
+        for nw in (4, 3, 5, 6, 7):
+            B.set_waves(nw)
+            B.upload(us)
+            out[nw] = B.propagate(A, A)[0], B.download()
+    for nw in (3, 5, 6, 7):
+        assert rel(out[nw][0], out[4][0]) < 1e-12
+        for u, v in zip(out[nw][1], out[4][1]):
+            assert rel(u, v) < 1e-12

@@ -1,0 +1,98 @@
+"""tdhf_rk4_step_noalloc on the density-matrix path (the padded copy and the
+matrices of its own) and its row-wise form where the padding does not fit the
+fixed array: against tdhf_rk4_step, and with calls on the context's own stream
+while its steps run on another."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from mattohf_amd import tdhf as T
+from test_gpu_kspace import orbitals, rel
+
+pytestmark = pytest.mark.gpu
+
+H2D, D2H, NON_BLOCKING = 1, 2, 1
+
+
+class Device:
+    """A device copy of u and a stream of the caller's."""
+
+    def __init__(self, u):
+        self.hip = C.CDLL("libamdhip64.so")
+        self.hip.hipMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t]
+        self.hip.hipMemcpy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
+        self.hip.hipFree.argtypes = [C.c_void_p]
+        self.hip.hipStreamCreateWithFlags.argtypes = [C.POINTER(C.c_void_p), C.c_uint]
+        self.hip.hipStreamSynchronize.argtypes = [C.c_void_p]
+        self.hip.hipStreamDestroy.argtypes = [C.c_void_p]
+        self.u = np.asfortranarray(u).copy(order="F")
+        self.ptr, self.stream = C.c_void_p(), C.c_void_p()
+        assert self.hip.hipMalloc(C.byref(self.ptr), u.nbytes) == 0
+        assert self.hip.hipStreamCreateWithFlags(C.byref(self.stream), NON_BLOCKING) == 0
+        assert self.hip.hipMemcpy(self.ptr, self.u.ctypes.data_as(C.c_void_p), u.nbytes, H2D) == 0
+
+    def step(self, G, Aave, A):
+        rc = T.load().tdhf_rk4_step_noalloc(G.h, self.ptr, Aave, A, self.stream)
+        assert rc == 0, T.load().tdhf_last_error(G.h)
+
+    def state(self):
+        assert self.hip.hipStreamSynchronize(self.stream) == 0
+        out = np.empty_like(self.u, order="F")
+        assert self.hip.hipMemcpy(out.ctypes.data_as(C.c_void_p), self.ptr, out.nbytes, D2H) == 0
+        return out
+
+    def close(self):
+        self.hip.hipStreamSynchronize(self.stream)
+        self.hip.hipStreamDestroy(self.stream)
+        self.hip.hipFree(self.ptr)
+
+
+def system(case):
+    ng, nk, nb, nbocc, a, z = case
+    vion = T.ion_potential(ng, nk, a, [z], [1.0], [0.1])
+    return T.TDHF(ng, nk, nb, nbocc, a, 0.004, vion), orbitals(case, 1)
+
+
+# every transform length; the last is the largest state the array holds
+@pytest.mark.parametrize("case", [(64, 33, 13, 12, 10.0, 6.0), (128, 16, 16, 16, 12.0, 6.0),
+                                  (64, 32, 14, 14, 10.0, 6.0), (128, 128, 8, 8, 12.0, 6.0)],
+                         ids=lambda c: f"ng{c[0]}_nk{c[1]}")
+def test_equals_rk4_step_beside_other_calls(case):
+    """Steps on the caller's stream, H and observables of other orbitals on the
+    context's at the same time: each as alone."""
+    G, u = system(case)
+    w = orbitals(case, 2)
+    with G:
+        h, e = G.ubkwbk_hwbk(w, w, 0.3), G.observables(w, 0.2)
+        ref = u
+        for i in range(20):
+            ref = G.RT_RK4_ubk(ref, 0.01 * i, 0.02 * i)
+        D = Device(u)
+        try:
+            for i in range(20):
+                D.step(G, 0.01 * i, 0.02 * i)
+            for _ in range(5):
+                np.testing.assert_array_equal(G.ubkwbk_hwbk(w, w, 0.3), h)
+                assert G.observables(w, 0.2)[0] == e[0]
+            np.testing.assert_array_equal(D.state(), ref)
+        finally:
+            D.close()
+
+
+def test_row_wise_where_the_padding_does_not_fit():
+    """NG NB NK = 130816 fits the array, with NK padded to 16 (299008) it does
+    not: the step is row-wise, tdhf_rk4_step goes through the matrices."""
+    case = (128, 7, 146, 12, 12.0, 6.0)
+    ng, nk, nb = case[:3]
+    vion = T.ion_potential(ng, nk, 12.0, [6.0], [1.0], [0.1])
+    rng = np.random.default_rng(3)
+    u = np.asfortranarray(rng.standard_normal((ng, nb, nk)) + 1j * rng.standard_normal((ng, nb, nk)))
+    with T.TDHF(ng, nk, nb, case[3], 12.0, 0.004, vion) as G:
+        ref = G.RT_RK4_ubk(u, 0.05, 0.1)
+        D = Device(u)
+        try:
+            D.step(G, 0.05, 0.1)
+            assert rel(D.state(), ref) < 1e-12
+        finally:
+            D.close()
