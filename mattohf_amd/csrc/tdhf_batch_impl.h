@@ -391,9 +391,10 @@ int batch_update_desc(tdhf_batch* b) {
 }
 
 // Waves of the product launch: as asked for, as far as the grid has x' for
-// them (every trajectory of the batch).
+// them (every trajectory of the batch).  A power of two: the waves share out
+// the x' evenly.
 int batch_apply_waves(const tdhf_batch* b, int nw) {
-  int w = nw;
+  int w = nw >= 8 ? 8 : nw >= 4 ? 4 : nw >= 2 ? 2 : 1;
   for (size_t i = 0; i < b->tabs.size(); ++i)
     w = std::min(w, kapply_waves(b->tabs[i]->kn, b->p.ng));
   return w;

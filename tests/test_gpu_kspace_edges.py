@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 CELL = {16: (3.6, 1.0), 32: (8.0, 4.0), 64: (10.0, 6.0), 128: (12.0, 6.0)}
 
 
-@pytest.mark.parametrize("ng,nk,nb,ntraj", [(64, 64, 4, 9), (16, 16, 4, 16)])
+@pytest.mark.parametrize("ng,nk,nb,ntraj", [(64, 64, 4, 9), (16, 16, 4, 300)])
 def test_waves_that_are_no_power_of_two(ng, nk, nb, ntraj):
     """3, 5, 6 and 7 waves of the product launch: the points do not divide among
     them, the results are those of 1, 2, 4 and 8."""
