@@ -155,8 +155,10 @@ __global__ void __launch_bounds__(256) dos_kernel(int nb, int nk, int nbocc, con
 // rounding errors.  What is missing to the rounded product omega t, whose phase
 // the transform is made of, is x ~ 1e-13 and enters as 1 + i x, so the phases
 // are those of a sine and cosine of omega t to 1e-15.  4000 frequencies, 20000
-// times: 300 -> 98 us.
+// times: 300 -> 98 us.  Beyond omega t = 2^26 (kFourierPhase) the rounding error
+// reaches 2^-26 and its square counts: S = 1 then, a sine and cosine of each product.
 constexpr int kFourierThreads = 512;
+constexpr double kFourierPhase = 67108864.0;
 
 // e^{i w t} with the rounding error of the product carried.
 __device__ __forceinline__ zd phase_of(double w, double t) {

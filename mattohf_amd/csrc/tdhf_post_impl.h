@@ -25,6 +25,19 @@ int te_series(tdhf_ctx* c, const zd* ua, const zd* ub, const zd* x, double Aave,
   return 0;
 }
 
+// The largest |t|, eight at a time (20000 in 4 us).
+double largest(const double* t, int n) {
+  double m[8] = {};
+  int i = 0;
+  for (; i + 8 <= n; i += 8)
+    for (int j = 0; j < 8; ++j) {
+      const double a = std::fabs(t[i + j]);
+      m[j] = a > m[j] ? a : m[j];
+    }
+  for (; i < n; ++i) m[0] = std::max(m[0], std::fabs(t[i]));
+  return *std::max_element(m, m + 8);
+}
+
 int post_device_check() {
   tdhf_ctx tmp;
   return check_device(&tmp);
@@ -165,10 +178,12 @@ extern "C" int tdhf_fourier(int nt, double dt, const double* time, const double*
     // frequencies per workgroup: the fewest rounds of workgroups over the CUs
     // times the operations of one per time (measured at 20000 times, us: 16
     // frequencies 98, 8 68, 4 54, one 48; 4000 in one round of 16 against two of
-    // 8, 1000 in one of 4 against four of one)
+    // 8, 1000 in one of 4 against four of one); one where a phase is large
     int S = 1;
     double best = 0.0;
+    const bool far = largest(time, nt) * std::fabs(omegam) > tdhf::kFourierPhase;
     for (int q : {1, 4, 8, 16}) {
+      if (far && q > 1) break;
       const long wg = ((long)nomega + q - 1) / q;
       const double cost = (double)((wg + device_cus() - 1) / std::max(1, device_cus())) *
                           (q == 1 ? 48.0 : 40.0 + 3.6 * q);
