@@ -706,8 +706,9 @@ int ctx_fail(tdhf_ctx* c, int code, const char* msg) { return fail(c, code, "%s"
 namespace {
 
 // The four stages of RT_RK4_ubk on u0 (path's layout) with the fields as kernel
-// arguments: no step counter, field arrays or observables.  sc: matrices other
-// than the context's.
+// arguments: no step counter, field arrays or observables.  st: a stream other
+// than the context's (nullptr: that one, on the context's path, and timed as its
+// other launches); sc: matrices other than the context's.
 int rk4_stages(tdhf_ctx* c, zd* u0, zd* ksum, zd* sa, zd* sb, double Aave, double A,
                hipStream_t st, bool kp, const KScratch* sc = nullptr) {
   tdhf::ApplyArgs a = base_args(c);
@@ -723,6 +724,10 @@ int rk4_stages(tdhf_ctx* c, zd* u0, zd* ksum, zd* sa, zd* sb, double Aave, doubl
     a.A = a.Aobs = fields[s];
     a.u = a.w = ins[s];
     a.unext = nexts[s];
+    if (!st) {
+      CHKRET(launch_stage(c, a));
+      continue;
+    }
     if (kp) {
       CHKRET(launch_kspace(c, a, 1, st, sc));
       continue;
@@ -1020,7 +1025,7 @@ int tdhf_rk4_step(tdhf_ctx* c, double* u, double Aave, double A) {
   if (!u) return fail(c, TDHF_EINVAL, "NULL array");
   CHKRET(stage_in(c, c->d_u0, u));
   c->u0_padded = c->kpath;
-  CHKRET(rk4_stages(c, c->d_u0, c->d_ksum, c->d_sa, c->d_sb, Aave, A, c->stream, c->kpath));
+  CHKRET(rk4_stages(c, c->d_u0, c->d_ksum, c->d_sa, c->d_sb, Aave, A, nullptr, c->kpath));
   return stage_out(c, u, c->d_u0);
 }
 

@@ -103,7 +103,7 @@ int gs_hamiltonian(tdhf_ctx* c, const zd* u) {
   a.mode = tdhf::M_HPSI;
   a.u = a.w = c->d_sa;
   tdhf::KArgs k = kspace_args(c, a);
-  return launch_kmat(c, k, 1, c->stream);
+  return timed(c, c->timing, [&] { return launch_kmat(c, k, 1, c->stream); });
 }
 
 // out = H[u] w for nbw columns per k-point, w and out held in ld columns per
@@ -124,7 +124,7 @@ int gs_product(tdhf_ctx* c, const zd* u, const zd* w, int nbw, int ld, zd* out) 
   a.w = c->gs.KW;
   a.out = c->gs.KH;
   tdhf::KArgs k = kspace_args(c, a);
-  CHKRET(launch_kapply(c, k, 1, c->stream));
+  CHKRET(timed(c, c->timing, [&] { return launch_kapply(c, k, 1, c->stream); }));
   return kspace_layout(c, c->gs.KH, out, false, 1, nullptr, nbw, ld);
 }
 

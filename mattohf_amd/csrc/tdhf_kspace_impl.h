@@ -217,6 +217,19 @@ int launch_kapply(tdhf_ctx* c, tdhf::KArgs& k, int ntraj, hipStream_t s) {
   return 0;
 }
 
+// launch() on the context's stream, between two events where on.
+template <typename F>
+int timed(tdhf_ctx* c, bool on, F launch) {
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  if (on) {
+    CHKRET(take_events(c, &e0, &e1));
+    HIPCHK(c, hipEventRecord(e0, c->stream));
+  }
+  CHKRET(launch());
+  if (on) HIPCHK(c, hipEventRecord(e1, c->stream));
+  return 0;
+}
+
 int launch_kspace(tdhf_ctx* c, const tdhf::ApplyArgs& a, int ntraj = 1,
                   hipStream_t st = nullptr, const KScratch* sc = nullptr) {
   tdhf::KArgs k = kspace_args(c, a);
@@ -226,17 +239,11 @@ int launch_kspace(tdhf_ctx* c, const tdhf::ApplyArgs& a, int ntraj = 1,
     k.hstride = sc->hstride;
     k.nstride = sc->nstride;
   }
-  const bool timed = c->timing && !st;
   hipStream_t s = st ? st : c->stream;
-  hipEvent_t e0 = nullptr, e1 = nullptr;
-  if (timed) {
-    CHKRET(take_events(c, &e0, &e1));
-    HIPCHK(c, hipEventRecord(e0, c->stream));
-  }
-  CHKRET(launch_kmat(c, k, ntraj, s));
-  CHKRET(launch_kapply(c, k, ntraj, s));
-  if (timed) HIPCHK(c, hipEventRecord(e1, c->stream));
-  return 0;
+  return timed(c, c->timing && !st, [&] {
+    CHKRET(launch_kmat(c, k, ntraj, s));
+    return launch_kapply(c, k, ntraj, s);
+  });
 }
 
 // One stage launch of the context's path, states in that path's layout.
@@ -310,7 +317,10 @@ int stage_in(tdhf_ctx* c, zd* dst, const double* src, zd* dst2 = nullptr,
 
 // src in the path's layout to the caller's state, after all that is queued.
 int stage_out(tdhf_ctx* c, double* dst, const zd* src) {
-  if (!c->h_stage) return download_state(c, dst, src);
+  if (!c->h_stage) {
+    CHKRET(download_state(c, dst, src));
+    return harvest_timing(c);
+  }
   const size_t n = nstate(c);
   zd* h = c->h_stage + 2 * n;
   if (c->kpath) {

@@ -32,3 +32,23 @@ def test_waves_that_are_no_power_of_two(ng, nk, nb, ntraj):
         assert rel(out[nw][0], out[4][0]) < 1e-12
         for u, v in zip(out[nw][1], out[4][1]):
             assert rel(u, v) < 1e-12
+
+
+# the density-matrix path (pinned memory, and a state too large for it) and the
+# row-wise one
+@pytest.mark.parametrize("case", [(16, 128, 8, 8), (64, 64, 8, 8), (32, 4, 2, 2)],
+                         ids=lambda c: f"ng{c[0]}_nk{c[1]}")
+def test_launches_are_timed(case):
+    """Four launches a step; in the ground state every product with H."""
+    a, z = CELL[case[0]]
+    vion = T.ion_potential(case[0], case[1], a, [z], [1.0], [0.0])
+    u = orbitals(case + (a, z), 1)
+    with T.TDHF(*case, a, 0.004, vion) as G:
+        G.set_kernel_timing(True)
+        for _ in range(2):
+            u = G.RT_RK4_ubk(u, 0.1, 0.1)
+        n, ms = G.kernel_stats()
+        assert n == 8 and ms > 0.0
+        G.set_kernel_timing(True)
+        G.GS_calculation(u, 1, 2)
+        assert G.kernel_stats()[0] >= 6  # energies 2, Krylov products 2, subspace 1, residuals 1
