@@ -188,6 +188,7 @@ int dalloc(tdhf_ctx* c, T** p, size_t n) {
   hipError_t e = hipMalloc((void**)p, n * sizeof(T) + 16);
   if (e != hipSuccess) {
     *p = nullptr;
+    (void)hipGetLastError();
     return fail(c, TDHF_ENOMEM, "hipMalloc of %zu bytes failed: %s", n * sizeof(T),
                 hipGetErrorString(e));
   }
@@ -668,16 +669,20 @@ int build_tables(tdhf_ctx* c, const double* vcg, const double* vcgkk) {
   return 0;
 }
 
+void free_states(tdhf_ctx* c) {
+  dfree(c->d_u0); dfree(c->d_ksum); dfree(c->d_sa); dfree(c->d_sb);
+  dfree(c->d_w); dfree(c->d_out); dfree(c->d_hm); dfree(c->d_nx);
+}
+
 void release(tdhf_ctx* c) {
   destroy_graph(c);
   for (auto e : c->ev_pool) (void)hipEventDestroy(e);
   c->ev_pool.clear();
   dfree(c->d_kx); dfree(c->d_vion); dfree(c->d_vcg);
   dfree(c->d_vq); dfree(c->d_vtl); dfree(c->d_tw); dfree(c->d_kc); dfree(c->d_vhg);
-  dfree(c->d_u0); dfree(c->d_ksum); dfree(c->d_sa); dfree(c->d_sb);
-  dfree(c->d_w); dfree(c->d_out);
+  free_states(c);
   if (c->h_stage) (void)hipHostFree(c->h_stage);
-  dfree(c->d_ktab); dfree(c->d_ktw); dfree(c->d_om); dfree(c->d_hm); dfree(c->d_nx);
+  dfree(c->d_ktab); dfree(c->d_ktw); dfree(c->d_om);
   dfree(c->d_hm_step); dfree(c->d_nx_step);
   dfree(c->d_obs); dfree(c->d_res); dfree(c->d_A); dfree(c->d_Aave); dfree(c->d_step);
   tdhf::gs_free(c->gs);
@@ -791,14 +796,17 @@ int tdhf_create(const tdhf_params* p, const double* vion, const double* vcg, con
   }
   c->kn = tdhf::kspace_len(c->nk);
   c->kpath = kspace_pays(c->ng, c->nk, c->nb, c->nbocc, 1);
-  const size_t n = path_count(c);
+  rc = alloc_states(c);
+  if (rc == TDHF_ENOMEM && c->kpath) {  // no memory for the padded states and matrices
+    free_states(c);
+    c->kpath = false;
+    rc = alloc_states(c);
+  }
+  if (rc) return bail(rc);
   // kx with zeros up to the padded number of k-points
   std::vector<double> kxp(std::max(c->nk, c->kn), 0.0);
   std::copy(c->kx.begin(), c->kx.end(), kxp.begin());
   if ((rc = dalloc(c, &c->d_kx, kxp.size())) || (rc = dalloc(c, &c->d_vion, c->ng)) ||
-      (rc = dalloc(c, &c->d_u0, n)) || (rc = dalloc(c, &c->d_ksum, n)) ||
-      (rc = dalloc(c, &c->d_sa, n)) || (rc = dalloc(c, &c->d_sb, n)) ||
-      (rc = dalloc(c, &c->d_w, n)) || (rc = dalloc(c, &c->d_out, n)) ||
       (rc = dalloc(c, &c->d_step, 1)))
     return bail(rc);
   if (hipMemcpy(c->d_kx, kxp.data(), kxp.size() * sizeof(double), hipMemcpyHostToDevice) !=
@@ -816,10 +824,8 @@ int tdhf_create(const tdhf_params* p, const double* vion, const double* vcg, con
   if (c->kn && (rc = kspace_tables(c))) return bail(rc);
   if (c->kpath && nstate(c) <= kNoAllocMaxState && kcount(c) <= kNoAllocSlot &&
       (dalloc(c, &c->d_hm_step, tdhf::kmat_elems(c->ng, c->kn)) ||
-       dalloc(c, &c->d_nx_step, tdhf::kmat_extra(c->ng, kspace_gpw(c->kn))))) {
+       dalloc(c, &c->d_nx_step, tdhf::kmat_extra(c->ng, kspace_gpw(c->kn)))))
     dfree(c->d_hm_step);
-    (void)hipGetLastError();
-  }
   {
     const hipError_t e = set_apply_lds_limit(c->ng);
     if (e != hipSuccess && c->lds > 64 * 1024) {

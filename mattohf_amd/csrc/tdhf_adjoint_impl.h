@@ -80,7 +80,8 @@ AdjState* adj_find(const tdhf_ctx* c) {
   return it == adj_states().end() ? nullptr : &it->second;
 }
 
-void adj_free(AdjState& s) {
+// The record's device memory.
+void adj_free_buffers(AdjState& s) {
   dfree(s.dA);
   dfree(s.dAave);
   dfree(s.dJ);
@@ -98,6 +99,10 @@ void adj_free(AdjState& s) {
   dfree(s.zrow);
   dfree(s.hm);
   dfree(s.nx);
+}
+
+void adj_free(AdjState& s) {
+  adj_free_buffers(s);
   for (auto& g : s.graphs) (void)hipGraphExecDestroy(g.second);
   s = AdjState();
 }
@@ -567,6 +572,34 @@ int adj_fail_free(AdjState& s, int rc) {
   return rc;
 }
 
+// The record's buffers in the layout of s.kp.  On the density-matrix path also
+// fails where the backward call's would not fit beside them, so that the run
+// is row-wise from the start then.
+int adj_alloc(tdhf_ctx* c, AdjState& s) {
+  const size_t blk = (size_t)s.ntraj * adj_count(c, s);
+  const size_t nsl = (size_t)s.ntraj * (s.nt + 1);
+  if (s.kp) {
+    const KScratch k = adj_scratch(c, s);
+    CHKRET(dalloc(c, &s.hm, (size_t)s.ntraj * k.hstride));
+    CHKRET(dalloc(c, &s.nx, (size_t)s.ntraj * k.nstride));
+  }
+  CHKRET(dalloc(c, &s.dA, s.A.size()));
+  CHKRET(dalloc(c, &s.dAave, s.A.size()));
+  CHKRET(dalloc(c, &s.st, 4 * blk));
+  CHKRET(dalloc(c, &s.tape, (size_t)4 * s.seg * blk));
+  CHKRET(dalloc(c, &s.obs, nsl * adj_obs_stride(c, s)));
+  CHKRET(dalloc(c, &s.res, nsl * 7));
+  if (!s.full) CHKRET(dalloc(c, &s.ckpt, (size_t)((s.nt + s.seg - 1) / s.seg) * blk));
+  if (s.kp) {
+    size_t fr = 0, tot = 0;
+    HIPCHK(c, hipMemGetInfo(&fr, &tot));
+    const double later = (double)sizeof(zd) * 4 * blk +
+                         8.0 * s.ntraj * ((double)s.seg * 4 * adj_nabar(c, s) + s.nt * 4.0);
+    if (later > (double)fr) return fail(c, TDHF_ENOMEM, "no memory for the backward call");
+  }
+  return 0;
+}
+
 }  // namespace
 
 // One progress report (tdhf_set_progress): after the segment has finished.
@@ -633,28 +666,17 @@ extern "C" int tdhf_fwd_batch(tdhf_ctx* c, int ntraj, double* u, int nt, const d
     const double kb = (double)ntraj * kcount(c) * sizeof(zd);
     const double plan = s.full ? 4.0 * nt : (double)((nt + s.seg - 1) / s.seg) + 4.0 * s.seg;
     s.kp = !(mem_budget > 0.0) || plan * kb <= budget;
-    if (s.kp) {
-      const KScratch k = adj_scratch(c, s);
-      if (hipMalloc((void**)&s.hm, (size_t)ntraj * k.hstride * sizeof(zd)) != hipSuccess ||
-          hipMalloc((void**)&s.nx, (size_t)ntraj * k.nstride * sizeof(double)) != hipSuccess) {
-        (void)hipGetLastError();  // without that memory: row-wise
-        dfree(s.hm);
-        dfree(s.nx);
-        s.kp = false;
-      }
-    }
   }
+  int rc = adj_alloc(c, s);
+  if (rc == TDHF_ENOMEM && s.kp) {  // without that memory: row-wise
+    adj_free_buffers(s);
+    s.kp = false;
+    rc = adj_alloc(c, s);
+  }
+  if (rc) return adj_fail_free(s, rc);
   const size_t ns = adj_count(c, s), blk = (size_t)ntraj * ns;
-  int rc = 0;
   const long nsl = (long)nt + 1;
   const int ostride = adj_obs_stride(c, s);
-  if ((rc = dalloc(c, &s.dA, s.A.size())) || (rc = dalloc(c, &s.dAave, s.A.size())) ||
-      (rc = dalloc(c, &s.st, 4 * blk)) || (rc = dalloc(c, &s.tape, (size_t)4 * s.seg * blk)) ||
-      (rc = dalloc(c, &s.obs, (size_t)ntraj * nsl * ostride)) ||
-      (rc = dalloc(c, &s.res, (size_t)ntraj * nsl * 7)))
-    return adj_fail_free(s, rc);
-  if (!s.full && (rc = dalloc(c, &s.ckpt, (size_t)((nt + s.seg - 1) / s.seg) * blk)))
-    return adj_fail_free(s, rc);
   HIPCHK(c, hipMemcpyAsync(s.dA, s.A.data(), s.A.size() * sizeof(double), hipMemcpyHostToDevice,
                            c->stream));
   HIPCHK(c, hipMemcpyAsync(s.dAave, s.Aave.data(), s.Aave.size() * sizeof(double),

@@ -43,7 +43,7 @@ struct tdhf_batch {
   double* d_nx = nullptr;
   std::vector<size_t> hoff, noff;
   int2 *d_amap = nullptr, *d_bmap = nullptr;
-  int na = 0, nbm = 0, map_nw = 0, map_sched = -1;
+  int na = 0, nbm = 0, map_sched = -1;
   double* d_vion = nullptr;
   zd* d_state = nullptr;        // 4 * region: u0 | ksum | sa | sb
   tdhf::TrajDesc* d_td = nullptr;
@@ -112,6 +112,7 @@ int balloc(tdhf_batch* b, T** p, size_t n) {
   hipError_t e = hipMalloc((void**)p, n * sizeof(T) + 16);
   if (e != hipSuccess) {
     *p = nullptr;
+    (void)hipGetLastError();
     return bfail(b, TDHF_ENOMEM, "hipMalloc of %zu bytes failed: %s", n * sizeof(T),
                  hipGetErrorString(e));
   }
@@ -670,27 +671,48 @@ size_t batch_slot(const tdhf_batch* b, int t) {
   return std::max((size_t)3 * b->p.nb * b->nk[t] + 3, (size_t)tdhf::kspace_obs_stride(b->p.ng));
 }
 
+int batch_alloc_fields(tdhf_batch* b, long nt) {
+  if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
+  b->gexec = nullptr;
+  dfree(b->d_A);
+  dfree(b->d_Aave);
+  dfree(b->d_obs);
+  dfree(b->d_res);
+  b->A_cap = b->obs_cap = b->res_cap = 0;
+  const long cap = std::max(nt, 1L);
+  CHKRET(balloc(b, &b->d_A, (size_t)cap * b->ntraj));
+  CHKRET(balloc(b, &b->d_Aave, (size_t)cap * b->ntraj));
+  size_t per_slot = 0;
+  for (int t = 0; t < b->ntraj; ++t) per_slot += batch_slot(b, t);
+  CHKRET(balloc(b, &b->d_obs, per_slot * (size_t)(cap + 1)));
+  CHKRET(balloc(b, &b->d_res, (size_t)7 * b->ntraj * (cap + 1)));
+  b->A_cap = cap;
+  b->obs_cap = cap + 1;
+  b->res_cap = cap + 1;
+  return batch_update_desc(b);
+}
+
+// Gives up the density-matrix path and its memory: mode 0 is row-wise.
+void batch_kspace_drop(tdhf_batch* b) {
+  dfree(b->d_roff);
+  dfree(b->d_koff);
+  dfree(b->d_hm);
+  dfree(b->d_nx);
+  dfree(b->d_amap);
+  dfree(b->d_bmap);
+  b->map_sched = -1;
+  b->kuse = false;
+}
+
 int batch_ensure(tdhf_batch* b, long nt) {
-  if (nt > b->A_cap || nt + 1 > b->obs_cap) {
-    if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
-    b->gexec = nullptr;
-    dfree(b->d_A);
-    dfree(b->d_Aave);
-    dfree(b->d_obs);
-    dfree(b->d_res);
-    const long cap = std::max(nt, 1L);
-    CHKRET(balloc(b, &b->d_A, (size_t)cap * b->ntraj));
-    CHKRET(balloc(b, &b->d_Aave, (size_t)cap * b->ntraj));
-    size_t per_slot = 0;
-    for (int t = 0; t < b->ntraj; ++t) per_slot += batch_slot(b, t);
-    CHKRET(balloc(b, &b->d_obs, per_slot * (size_t)(cap + 1)));
-    CHKRET(balloc(b, &b->d_res, (size_t)7 * b->ntraj * (cap + 1)));
-    b->A_cap = cap;
-    b->obs_cap = cap + 1;
-    b->res_cap = cap + 1;
-    CHKRET(batch_update_desc(b));
-  }
-  return 0;
+  if (nt <= b->A_cap && nt + 1 <= b->obs_cap) return 0;
+  const int rc = batch_alloc_fields(b, nt);
+  if (rc != TDHF_ENOMEM || !b->kuse) return rc;
+  // no memory beside the matrices
+  CHKRET(batch_layout(b, false));
+  BHIP(b, hipStreamSynchronize(b->stream));
+  batch_kspace_drop(b);
+  return batch_alloc_fields(b, nt);
 }
 
 void batch_release(tdhf_batch* b) {
@@ -711,7 +733,7 @@ void batch_release(tdhf_batch* b) {
 
 // Sets the batch up for the density-matrix path where it serves every
 // trajectory and is the faster one (KspaceCost); without memory for the
-// matrices mode 0 stays row-wise.
+// matrices, or beside them, mode 0 stays row-wise.
 int batch_kspace_setup(tdhf_batch* b) {
   for (auto c : b->tabs)
     if (!c->kn) return 0;
@@ -734,14 +756,11 @@ int batch_kspace_setup(tdhf_batch* b) {
     b->kmax = std::max(b->kmax, n);
     b->kn = t == 0 || b->kn == n ? n : 0;
   }
-  if (hipMalloc((void**)&b->d_hm, hs * sizeof(zd)) != hipSuccess) {
-    (void)hipGetLastError();
-    b->d_hm = nullptr;
+  if (balloc(b, &b->d_hm, hs) || balloc(b, &b->d_nx, xs) ||
+      balloc(b, &b->d_roff, (size_t)b->ntraj) || balloc(b, &b->d_koff, (size_t)b->ntraj)) {
+    batch_kspace_drop(b);
     return 0;
   }
-  CHKRET(balloc(b, &b->d_nx, xs));
-  CHKRET(balloc(b, &b->d_roff, (size_t)b->ntraj));
-  CHKRET(balloc(b, &b->d_koff, (size_t)b->ntraj));
   BHIP(b, hipMemcpy(b->d_roff, b->off.data(), b->ntraj * sizeof(size_t), hipMemcpyHostToDevice));
   BHIP(b, hipMemcpy(b->d_koff, b->koff.data(), b->ntraj * sizeof(size_t), hipMemcpyHostToDevice));
   const hipError_t e = kmat_lds_limits(b->kn, b->p.nb);
@@ -843,8 +862,13 @@ int tdhf_batch_create(const tdhf_params* p, int ntraj, const int* nk, const doub
   b->region = acc;
   int rc;
   if ((rc = batch_kspace_setup(b))) return bail(rc);
-  if ((rc = balloc(b, &b->d_vion, (size_t)p->ng * ntraj)) ||
-      (rc = balloc(b, &b->d_state, 4 * b->region)) ||
+  rc = balloc(b, &b->d_state, 4 * b->region);
+  if (rc == TDHF_ENOMEM && b->kuse) {
+    batch_kspace_drop(b);
+    b->region = b->total;
+    rc = balloc(b, &b->d_state, 4 * b->region);
+  }
+  if (rc || (rc = balloc(b, &b->d_vion, (size_t)p->ng * ntraj)) ||
       (rc = balloc(b, &b->d_td, (size_t)ntraj)) || (rc = balloc(b, &b->d_step, 1)))
     return bail(rc);
   if (hipMemcpy(b->d_vion, vion, sizeof(double) * p->ng * ntraj, hipMemcpyHostToDevice) != hipSuccess) {

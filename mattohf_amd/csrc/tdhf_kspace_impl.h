@@ -127,6 +127,17 @@ size_t kcount(const tdhf_ctx* c) { return (size_t)c->ng * c->nb * c->kn; }
 // complex elements of a state in the path's layout
 size_t path_count(const tdhf_ctx* c) { return c->kpath ? kcount(c) : nstate(c); }
 
+// The orbital buffers of a context in its path's layout and, on the
+// density-matrix path, the matrices of a stage.
+int alloc_states(tdhf_ctx* c) {
+  const size_t n = path_count(c);
+  for (zd** p : {&c->d_u0, &c->d_ksum, &c->d_sa, &c->d_sb, &c->d_w, &c->d_out})
+    CHKRET(dalloc(c, p, n));
+  if (!c->kpath) return 0;
+  CHKRET(dalloc(c, &c->d_hm, tdhf::kmat_elems(c->ng, c->kn)));
+  return dalloc(c, &c->d_nx, tdhf::kmat_extra(c->ng, kspace_gpw(c->kn)));
+}
+
 // Spectra, twiddles of the k transforms and the twist factors of a context.
 int kspace_tables(tdhf_ctx* c) {
   const int NG = c->ng, NK = c->nk, ND = 2 * NK - 1, N = c->kn;
@@ -134,10 +145,6 @@ int kspace_tables(tdhf_ctx* c) {
   CHKRET(dalloc(c, &c->d_ktab, (size_t)NG * 2 * N));
   CHKRET(dalloc(c, &c->d_ktw, 2 * N));
   CHKRET(dalloc(c, &c->d_om, N));
-  if (c->kpath) {
-    CHKRET(dalloc(c, &c->d_hm, tdhf::kmat_elems(NG, N)));
-    CHKRET(dalloc(c, &c->d_nx, tdhf::kmat_extra(NG, kspace_gpw(N))));
-  }
   CHKRET(dalloc(c, &tsp, (size_t)ND * NG));
   hipStream_t s = c->stream;
   hipLaunchKernelGGL(tdhf::kspace_space_kernel, dim3((ND * NG + 255) / 256), dim3(256), 0, s,
