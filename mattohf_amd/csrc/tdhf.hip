@@ -355,7 +355,7 @@ tdhf::ApplyArgs base_args(const tdhf_ctx* c) {
 int ensure_obs(tdhf_ctx* c, long slots) {
   if (slots > c->obs_slots) {
     dfree(c->d_obs);
-    const int stride = std::max(c->obs_stride, tdhf::kspace_obs_stride(c->ng));
+    const int stride = c->kpath ? tdhf::kspace_obs_stride(c->ng) : c->obs_stride;
     CHKRET(dalloc(c, &c->d_obs, (size_t)slots * stride));
     c->obs_slots = slots;
   }

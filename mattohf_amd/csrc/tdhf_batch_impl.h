@@ -666,9 +666,11 @@ int batch_run_steps(tdhf_batch* b, int nt) {
   return 0;
 }
 
-// Doubles of trajectory t's observables slot (the larger of the two paths').
+// Doubles of trajectory t's observables slot (where the density-matrix path
+// serves mode 0, the larger of the two paths').
 size_t batch_slot(const tdhf_batch* b, int t) {
-  return std::max((size_t)3 * b->p.nb * b->nk[t] + 3, (size_t)tdhf::kspace_obs_stride(b->p.ng));
+  const size_t rows = (size_t)3 * b->p.nb * b->nk[t] + 3;
+  return b->kuse ? std::max(rows, (size_t)tdhf::kspace_obs_stride(b->p.ng)) : rows;
 }
 
 int batch_alloc_fields(tdhf_batch* b, long nt) {
@@ -683,7 +685,10 @@ int batch_alloc_fields(tdhf_batch* b, long nt) {
   CHKRET(balloc(b, &b->d_A, (size_t)cap * b->ntraj));
   CHKRET(balloc(b, &b->d_Aave, (size_t)cap * b->ntraj));
   size_t per_slot = 0;
-  for (int t = 0; t < b->ntraj; ++t) per_slot += batch_slot(b, t);
+  for (int t = 0; t < b->ntraj; ++t) {
+    b->obs_off[t] = per_slot;
+    per_slot += batch_slot(b, t);
+  }
   CHKRET(balloc(b, &b->d_obs, per_slot * (size_t)(cap + 1)));
   CHKRET(balloc(b, &b->d_res, (size_t)7 * b->ntraj * (cap + 1)));
   b->A_cap = cap;
@@ -851,12 +856,10 @@ int tdhf_batch_create(const tdhf_params* p, int ntraj, const int* nk, const doub
   }
   b->off.resize(ntraj);
   b->obs_off.resize(ntraj);
-  size_t acc = 0, oacc = 0;
+  size_t acc = 0;
   for (int t = 0; t < ntraj; ++t) {
     b->off[t] = acc;
     acc += bstate(b, t);
-    b->obs_off[t] = oacc;
-    oacc += batch_slot(b, t);
   }
   b->total = acc;
   b->region = acc;

@@ -102,3 +102,30 @@ def test_batch_memory(when):
             u, e1 = G.RT_calculation(u, A[t, :nt], A[t, :nt])[:2]
         for k in (t, t + 3 * 2665):
             assert rel(out[k], u) < 1e-11 and rel(e[k], e1) < 1e-11
+
+
+def used(call):
+    """Bytes of device memory that call() leaves allocated."""
+    hip = C.CDLL("libamdhip64.so")
+    free, total = [C.c_size_t(), C.c_size_t()], C.c_size_t()
+    assert hip.hipMemGetInfo(C.byref(free[0]), C.byref(total)) == 0
+    call()
+    assert hip.hipMemGetInfo(C.byref(free[1]), C.byref(total)) == 0
+    return free[0].value - free[1].value
+
+
+def test_observables_slots_of_row_wise_runs():
+    """15 doubles a step at NG=128, NK=4, NB=1 (the other path's slots are of
+    768): 24 MB and 56 MB of observables, with the reduced values and the field
+    under 100 and 200 MB."""
+    ng, nk, a, nt = 128, 4, 12.0, 200000
+    vion = T.ion_potential(ng, nk, a, [6.0], [1.0], [0.0])
+    field = np.zeros(nt)
+    with T.TDHF(ng, nk, 1, 1, a, 0.004, vion) as G:
+        G.upload(orbitals((ng, nk, 1, 1, a, 6.0), 1))
+        assert used(lambda: G.rt_begin(field, field)) < 100e6
+    ntraj, nt = 200, 2000
+    with T.Batch(ng, 1, 1, a, 0.004, [nk] * ntraj, np.array([vion] * ntraj)) as B:
+        B.upload([orbitals((ng, nk, 1, 1, a, 6.0), 1)] * ntraj)
+        field = np.zeros((ntraj, nt))
+        assert used(lambda: B.propagate(field, field)) < 200e6
