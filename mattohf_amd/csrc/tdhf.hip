@@ -821,7 +821,7 @@ int tdhf_create(const tdhf_params* p, const double* vion, const double* vcg, con
     (void)hipGetLastError();
   }
   if ((rc = build_tables(c, vcg, vcgkk))) return bail(rc);
-  if (c->kn && (rc = kspace_tables(c))) return bail(rc);
+  if (c->kpath && (rc = kspace_tables(c))) return bail(rc);
   if (c->kpath && nstate(c) <= kNoAllocMaxState && kcount(c) <= kNoAllocSlot &&
       (dalloc(c, &c->d_hm_step, tdhf::kmat_elems(c->ng, c->kn)) ||
        dalloc(c, &c->d_nx_step, tdhf::kmat_extra(c->ng, kspace_gpw(c->kn)))))

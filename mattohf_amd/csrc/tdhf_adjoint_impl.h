@@ -579,6 +579,7 @@ int adj_alloc(tdhf_ctx* c, AdjState& s) {
   const size_t blk = (size_t)s.ntraj * adj_count(c, s);
   const size_t nsl = (size_t)s.ntraj * (s.nt + 1);
   if (s.kp) {
+    CHKRET(kspace_tables(c));
     const KScratch k = adj_scratch(c, s);
     CHKRET(dalloc(c, &s.hm, (size_t)s.ntraj * k.hstride));
     CHKRET(dalloc(c, &s.nx, (size_t)s.ntraj * k.nstride));

@@ -768,6 +768,14 @@ int batch_kspace_setup(tdhf_batch* b) {
   }
   BHIP(b, hipMemcpy(b->d_roff, b->off.data(), b->ntraj * sizeof(size_t), hipMemcpyHostToDevice));
   BHIP(b, hipMemcpy(b->d_koff, b->koff.data(), b->ntraj * sizeof(size_t), hipMemcpyHostToDevice));
+  for (auto c : b->tabs) {
+    const int rc = kspace_tables(c);
+    if (rc == TDHF_ENOMEM) {
+      batch_kspace_drop(b);
+      return 0;
+    }
+    if (rc) return bfail(b, rc, "%s", c->err.c_str());
+  }
   const hipError_t e = kmat_lds_limits(b->kn, b->p.nb);
   if (e != hipSuccess) return bfail(b, TDHF_EDEVICE, "LDS limit: %s", hipGetErrorString(e));
   b->region = std::max(b->total, ks);

@@ -138,14 +138,26 @@ int alloc_states(tdhf_ctx* c) {
   return dalloc(c, &c->d_nx, tdhf::kmat_extra(c->ng, kspace_gpw(c->kn)));
 }
 
-// Spectra, twiddles of the k transforms and the twist factors of a context.
+// Spectra, twiddles of the k transforms and the twist factors of a context, made
+// when the first run on the path needs them (a context that stays row-wise does
+// without: NG=16, NK=40, NB=8 created in 309 us, 377 with them).
 int kspace_tables(tdhf_ctx* c) {
+  if (c->d_ktab) return 0;
   const int NG = c->ng, NK = c->nk, ND = 2 * NK - 1, N = c->kn;
   zd* tsp = nullptr;
-  CHKRET(dalloc(c, &c->d_ktab, (size_t)NG * 2 * N));
-  CHKRET(dalloc(c, &c->d_ktw, 2 * N));
-  CHKRET(dalloc(c, &c->d_om, N));
-  CHKRET(dalloc(c, &tsp, (size_t)ND * NG));
+  int rc = dalloc(c, &c->d_ktab, (size_t)NG * 2 * N);
+  if (!rc) rc = dalloc(c, &c->d_ktw, 2 * N);
+  if (!rc) rc = dalloc(c, &c->d_om, N);
+  if (!rc) rc = dalloc(c, &tsp, (size_t)ND * NG);
+  auto undo = [&] {
+    dfree(c->d_ktab);
+    dfree(c->d_ktw);
+    dfree(c->d_om);
+  };
+  if (rc) {
+    undo();
+    return rc;
+  }
   hipStream_t s = c->stream;
   hipLaunchKernelGGL(tdhf::kspace_space_kernel, dim3((ND * NG + 255) / 256), dim3(256), 0, s,
                      c->d_vq, ND, NG, -1.0 / ((double)NG * (double)NK), tsp);
@@ -173,7 +185,10 @@ int kspace_tables(tdhf_ctx* c) {
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   dfree(tsp);
   if (e == hipSuccess) e = kmat_lds_limits(N, c->nb);
-  if (e != hipSuccess) return fail(c, TDHF_EDEVICE, "k-space tables: %s", hipGetErrorString(e));
+  if (e != hipSuccess) {
+    undo();
+    return fail(c, TDHF_EDEVICE, "k-space tables: %s", hipGetErrorString(e));
+  }
   return 0;
 }
 

@@ -52,3 +52,22 @@ def test_launches_are_timed(case):
         G.set_kernel_timing(True)
         G.GS_calculation(u, 1, 2)
         assert G.kernel_stats()[0] >= 6  # energies 2, Krylov products 2, subspace 1, residuals 1
+
+
+def test_many_pulses_of_a_row_wise_system():
+    """One trajectory is row-wise, twenty-four go through the matrices, whose tables
+    their first forward call makes: batch against single runs, twice."""
+    ng, nk, nb, nt, ntraj = 64, 32, 4, 3, 24
+    a, z = CELL[ng]
+    vion = T.ion_potential(ng, nk, a, [z], [1.0], [0.0])
+    us = [orbitals((ng, nk, nb, nb, a, z), t) for t in range(ntraj)]
+    A = 0.1 * np.random.default_rng(4).standard_normal((ntraj, nt))
+    with T.TDHF(ng, nk, nb, nb, a, 0.004, vion) as G:
+        for objective in ("energy", "jsq"):
+            L, fin, _, _, _ = G.fwd_batch(us, A, objective=objective)
+            g, gu = G.bwd_batch()
+            for t in (0, 11, 23):
+                L1, f1, _, _, _ = G.fwd_batch([us[t]], A[t:t + 1], objective=objective)
+                g1, gu1 = G.bwd_batch()
+                assert abs(L[t] - L1[0]) < 1e-11 * max(1.0, abs(L1[0])) and rel(fin[t], f1[0]) < 1e-12
+                assert rel(g[t], g1[0]) < 1e-9 and rel(gu[t], gu1[0]) < 1e-9
