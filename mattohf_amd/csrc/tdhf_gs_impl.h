@@ -197,11 +197,13 @@ extern "C" int tdhf_gs_run(tdhf_ctx* c, double* u, int nscf, int ncg, double tol
   CHKRET(gs_flag_clear(c));
   CHKRET(upload(c, c->d_u0, u));
   c->u0_padded = false;
-  // the energies are read one by one where the loop may end on them, else 256 at
-  // a time (a read waits for the iteration: 20 us of an idle device)
+  // the energies are read one by one where the loop may end on them, else sixteen
+  // at a time (a read waits for the iteration: 20 us of an idle device), so that
+  // a run whose energy is no longer a number ends within fifteen iterations of it
   const bool each = tol > 0.0;
-  const int cap = each ? 1 : std::min(nscf, 255) + 1;
-  double e[256], eprev = 0.0;
+  constexpr int kRead = 16;
+  const int cap = each ? 1 : std::min(nscf, kRead - 1) + 1;
+  double e[kRead], eprev = 0.0;
   CHKRET(ensure_obs(c, cap));
   int it = 0;
   for (int n = 0;; ++it) {

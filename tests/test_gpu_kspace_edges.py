@@ -71,3 +71,24 @@ def test_many_pulses_of_a_row_wise_system():
                 g1, gu1 = G.bwd_batch()
                 assert abs(L[t] - L1[0]) < 1e-11 * max(1.0, abs(L1[0])) and rel(fin[t], f1[0]) < 1e-12
                 assert rel(g[t], g1[0]) < 1e-9 and rel(gu[t], gu1[0]) < 1e-9
+
+
+@pytest.mark.parametrize("case", [(16, 3, 2, 1), (64, 64, 8, 8)], ids=lambda c: f"ng{c[0]}_nk{c[1]}")
+def test_ground_state_ends_soon_after_a_bad_energy(case):
+    """Orbitals that are not numbers: the first iteration's energy is none, and the
+    run of 200 ends by it (launches counted on the row-wise and the
+    density-matrix path; at most 7 and 9 an iteration)."""
+    a, z = CELL[case[0]]
+    vion = T.ion_potential(case[0], case[1], a, [z], [1.0], [0.0])
+    u = orbitals(case + (a, z), 1)
+    u[0, 0, 0] = np.nan
+    with T.TDHF(*case, a, 0.004, vion) as G:
+        G.set_kernel_timing(True)
+        with pytest.raises(T.TDHFError, match="iteration 1"):
+            G.GS_calculation(u, 200, 2)
+        assert G.kernel_stats()[0] <= 16 * 9
+        # and one that is: the energies of a run longer than is read at a time
+        u[0, 0, 0] = 0.0
+        long, short = G.GS_calculation(u, 33, 2)[1], G.GS_calculation(u, 33, 2, tol=1e-300)[1]
+        n = np.count_nonzero(short)
+        assert n > 17 and np.array_equal(long[:n], short[:n])
