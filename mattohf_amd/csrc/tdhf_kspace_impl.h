@@ -96,8 +96,10 @@ hipError_t kmat_lds_limits(int n, int nbw) {
   for (int v = 0; v < 4 && e == hipSuccess; ++v)
     e = hipFuncSetAttribute(kmat_fn_for(n, v & 1, v & 2),
                             hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  // (the product kernel in every variant: the ground state multiplies NB NCG columns)
   const int nbt = kspace_nbt(nbw);
-  const void* more[] = {kapply_fn(nbt, 1), kapply_fn(nbt, 2), kadj_mat_fn(n), kadj_apply_fn(nbt, 1),
+  const void* more[] = {kapply_fn(2, 1), kapply_fn(2, 2), kapply_fn(4, 1), kapply_fn(4, 2),
+                        kapply_fn(8, 1), kapply_fn(8, 2), kadj_mat_fn(n), kadj_apply_fn(nbt, 1),
                         kadj_apply_fn(nbt, 2)};
   for (auto f : more)
     if (e == hipSuccess)

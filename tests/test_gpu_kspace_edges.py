@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from mattohf_amd import tdhf as T
-from test_gpu_kspace import orbitals, rel
+from test_gpu_kspace import orbitals, rel, system
 
 pytestmark = pytest.mark.gpu
 
@@ -92,3 +92,16 @@ def test_ground_state_ends_soon_after_a_bad_energy(case):
         long, short = G.GS_calculation(u, 33, 2)[1], G.GS_calculation(u, 33, 2, tol=1e-300)[1]
         n = np.count_nonzero(short)
         assert n > 17 and np.array_equal(long[:n], short[:n])
+
+
+def test_ground_state_of_more_columns_than_bands():
+    """Twelve Krylov columns of four bands: the product kernel's variant of eight
+    columns and two grid points (64 KB of LDS and more), which no other call of
+    the context launches, against the oracle."""
+    case = (128, 96, 4, 4) + CELL[128]
+    S, O, G, _ = system(case)
+    u = orbitals(case, 1)
+    with G:
+        _, eh, eps, _ = G.GS_calculation(u, 1, 3)
+    _, eo, epso, _ = O.GS_calculation(u, 1, 3)
+    assert np.abs(np.asarray(eh) - eo).max() < 1e-10 and np.abs(np.asarray(eps) - epso).max() < 1e-10
