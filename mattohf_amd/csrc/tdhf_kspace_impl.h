@@ -15,13 +15,15 @@ namespace {
 // against 27.8 does not.
 struct KspaceCost {
   double rows = 0.0, mat = 0.0;
+  bool fits = true;  // kapply_kernel's byte offsets into a padded state are 32 bits wide
   void add(int ng, int nk, int nb, int nbocc, int ntraj = 1) {
     int lg = 0;
     while ((1 << lg) < ng) ++lg;
     rows += 1e-6 * ntraj * nk * nk * nb * nbocc * (double)ng * lg;
     mat += 1e-6 * ntraj * (double)ng * ng * tdhf::kspace_len(nk);
+    fits = fits && (size_t)ng * nb * tdhf::kspace_len(nk) * sizeof(zd) <= UINT32_MAX;
   }
-  bool pays() const { return 5.5 + 0.42 * rows > 13.0 + 12.0 * mat; }
+  bool pays() const { return fits && 5.5 + 0.42 * rows > 13.0 + 12.0 * mat; }
 };
 
 bool kspace_pays(int ng, int nk, int nb, int nbocc, int ntraj) {

@@ -105,3 +105,20 @@ def test_ground_state_of_more_columns_than_bands():
         _, eh, eps, _ = G.GS_calculation(u, 1, 3)
     _, eo, epso, _ = O.GS_calculation(u, 1, 3)
     assert np.abs(np.asarray(eh) - eo).max() < 1e-10 and np.abs(np.asarray(eps) - epso).max() < 1e-10
+
+
+def test_states_beyond_32_bit_offsets():
+    """1.2 million bands of two k-points, 4.9 GB with the k-points padded to
+    sixteen: row-wise.  Every band's H w is that of a system of few bands."""
+    ng, nk, nb = 16, 2, 1200000
+    a, z = CELL[ng]
+    vion = T.ion_potential(ng, nk, a, [z], [1.0], [0.0])
+    u = orbitals((ng, nk, 4, 1, a, z), 1)
+    with T.TDHF(ng, nk, 4, 1, a, 0.004, vion) as G:
+        ref = G.ubkwbk_hwbk(u, u, 0.2)
+    many = np.empty((ng, nb, nk), dtype=complex, order="F")
+    many.reshape(ng, 4, nb // 4, nk, order="F")[:] = u[:, :, None, :]
+    with T.TDHF(ng, nk, nb, 1, a, 0.004, vion) as G:
+        h = G.ubkwbk_hwbk(many, many, 0.2)
+    d = np.abs(h.reshape(ng, 4, nb // 4, nk, order="F") - ref[:, :, None, :])
+    assert d.max() < 1e-12 * np.abs(ref).max()
