@@ -178,9 +178,12 @@ __global__ void __launch_bounds__(kFourierThreads)
   constexpr int H = S / 2;  // pairs
   __shared__ double red[NW * NV];
   const int iw0 = blockIdx.x * S, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  auto freq = [&](int iw) { return (double)(iw + 1) / (double)nomega * omegam; };
+  auto freq = [&](int iw) {
+#pragma clang fp contract(off)
+    return (double)(iw + 1) / (double)nomega * omegam;
+  };
   const double tn = time[nt - 1];
-  const double h = 0.5 * (omegam / (double)nomega);
+  const double h = 0.5 * (omegam / (double)nomega);  // (a division: not fused)
   const double wc = S == 1 ? freq(iw0) : ((double)(iw0 + 1) + 0.5 * (S - 1)) / (double)nomega * omegam;
   // freq - wc -+ (2m+1) h, uniform: pair m is the frequencies H - 1 - m and H + m
   double dl[S], wj[S];
@@ -189,14 +192,17 @@ __global__ void __launch_bounds__(kFourierThreads)
                             __builtin_amdgcn_readfirstlane(__double2loint(v)));
   };
   static_for<0, S>([&](auto jc) {
+    // (a product fused into a difference here would not be the rounded frequency
+    // that the phases are of: up to two units of omega t in its last place)
+#pragma clang fp contract(off)
     constexpr int jj = decltype(jc)::value;
     double d = 0.0;
     if constexpr (S > 1) {
       constexpr int m = jj < H ? H - 1 - jj : jj - H;
-      const double w = freq(iw0 + jj), step = (jj < H ? -1.0 : 1.0) * (2 * m + 1) * h;
+      const double w = freq(iw0 + jj);
       const double a = w - wc, z = a - w;  // a + err = w - wc exactly
       const double err = (w - (a - z)) + (-wc - z);
-      d = (a - step) + err;
+      d = fma(jj < H ? 2.0 * m + 1.0 : -(2.0 * m + 1.0), h, a) + err;
     }
     dl[jj] = uniform(d);
     wj[jj] = uniform(freq(iw0 + jj));
