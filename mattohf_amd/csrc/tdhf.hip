@@ -890,11 +890,12 @@ int tdhf_get_tables(tdhf_ctx* c, double* vcg, double* vq) {
 int tdhf_hpsi(tdhf_ctx* c, const double* u, const double* w, double A, double* hw) {
   if (!c) return fail(nullptr, TDHF_EINVAL, "ctx is NULL");
   if (!u || !w || !hw) return fail(c, TDHF_EINVAL, "NULL array");
-  CHKRET(stage_in(c, c->d_sa, u, c->d_w, w));
+  const bool kp = kspace_hpsi_pays(c);
+  CHKRET(stage_in(c, kp, c->d_sa, u, c->d_w, w));
   // (row-wise, the result goes straight to the pinned memory)
-  zd* out = c->h_stage && !c->kpath ? c->h_stage + 2 * nstate(c) : c->d_out;
-  CHKRET(path_hpsi(c, c->d_sa, c->d_w, A, out));
-  CHKRET(stage_out(c, hw, out));
+  zd* out = c->h_stage && !kp ? c->h_stage + 2 * nstate(c) : c->d_out;
+  CHKRET(path_hpsi(c, kp, c->d_sa, c->d_w, A, out));
+  CHKRET(stage_out(c, kp, hw, out));
   return sync(c);
 }
 
@@ -1029,10 +1030,10 @@ int tdhf_rt_run(tdhf_ctx* c, double* u, int nt, const double* A, const double* A
 int tdhf_rk4_step(tdhf_ctx* c, double* u, double Aave, double A) {
   if (!c) return fail(nullptr, TDHF_EINVAL, "ctx is NULL");
   if (!u) return fail(c, TDHF_EINVAL, "NULL array");
-  CHKRET(stage_in(c, c->d_u0, u));
+  CHKRET(stage_in(c, c->kpath, c->d_u0, u));
   c->u0_padded = c->kpath;
   CHKRET(rk4_stages(c, c->d_u0, c->d_ksum, c->d_sa, c->d_sb, Aave, A, nullptr, c->kpath));
-  return stage_out(c, u, c->d_u0);
+  return stage_out(c, c->kpath, u, c->d_u0);
 }
 
 int tdhf_rk4_step_noalloc(tdhf_ctx* c, double* u, double Aave, double A, void* stream) {

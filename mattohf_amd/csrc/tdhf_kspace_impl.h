@@ -23,7 +23,8 @@ struct KspaceCost {
     mat += 1e-6 * ntraj * (double)ng * ng * tdhf::kspace_len(nk);
     fits = fits && (size_t)ng * nb * tdhf::kspace_len(nk) * sizeof(zd) <= UINT32_MAX;
   }
-  bool pays() const { return fits && 5.5 + 0.42 * rows > 13.0 + 12.0 * mat; }
+  double gain() const { return fits ? 5.5 + 0.42 * rows - (13.0 + 12.0 * mat) : 0.0; }
+  bool pays() const { return gain() > 0.0; }
 };
 
 bool kspace_pays(int ng, int nk, int nb, int nbocc, int ntraj) {
@@ -31,6 +32,19 @@ bool kspace_pays(int ng, int nk, int nb, int nbocc, int ntraj) {
   KspaceCost c;
   c.add(ng, nk, nb, nbocc, ntraj);
   return c.pays();
+}
+
+// Whether one H application of host arrays pays on the path.  Its two states and
+// its result change layout: with pinned memory the staging kernels do that on
+// their way, else it is three launches between the copies, 20 to 30 us.  Measured
+// per call, row-wise against matrices, with KspaceCost's gain: NG=64, NK=32, NB=9
+// 92 and 114 us (3), NK=64, NB=8 131 and 140 (32), NK=64, NB=11 184 and 160 (69);
+// NG=128, NK=16, NB=16 119 and 141 (14), NK=32, NB=9 158 and 151 (17); NG=32,
+// NK=128, NB=6 with 4 occupied 117 and 120 (17), NB=8 174 and 136 (61).
+bool kspace_hpsi_pays(const tdhf_ctx* c) {
+  KspaceCost k;
+  k.add(c->ng, c->nk, c->nb, c->nbocc);
+  return c->kpath && (c->h_stage || k.gain() > (c->ng == 64 ? 40.0 : 15.0));
 }
 
 // x' values per wave (transform groups).
@@ -320,17 +334,26 @@ int download_state(tdhf_ctx* c, double* dst, const zd* src) {
 // that the copy engines are as fast as a kernel over the bus.
 constexpr size_t kStageState = 256 * 1024 / sizeof(zd);
 
-// The caller's state (and a second one) to dst (dst2) in the path's layout.
-int stage_in(tdhf_ctx* c, zd* dst, const double* src, zd* dst2 = nullptr,
+// The caller's state (and a second one) to dst (dst2), padded with kp.
+int stage_in(tdhf_ctx* c, bool kp, zd* dst, const double* src, zd* dst2 = nullptr,
              const double* src2 = nullptr) {
   if (!c->h_stage) {
-    CHKRET(upload_state(c, dst, src));
-    return src2 ? upload_state(c, dst2, src2) : 0;
+    if (!kp) {
+      CHKRET(upload(c, dst, src));
+      return src2 ? upload(c, dst2, src2) : 0;
+    }
+    if (!src2) return upload_state(c, dst, src);
+    // both copies, then both kernels: a copy after a kernel waits for it on
+    // another engine (d_out holds nothing before the product)
+    CHKRET(upload(c, c->d_ksum, src));
+    CHKRET(upload(c, c->d_out, src2));
+    CHKRET(kspace_layout(c, c->d_ksum, dst, true));
+    return kspace_layout(c, c->d_out, dst2, true);
   }
   const size_t n = nstate(c);
   std::memcpy(c->h_stage, src, n * sizeof(zd));
   if (src2) std::memcpy(c->h_stage + n, src2, n * sizeof(zd));
-  if (c->kpath) {
+  if (kp) {
     CHKRET(kspace_layout(c, c->h_stage, dst, true));
     return src2 ? kspace_layout(c, c->h_stage + n, dst2, true) : 0;
   }
@@ -341,15 +364,15 @@ int stage_in(tdhf_ctx* c, zd* dst, const double* src, zd* dst2 = nullptr,
   return 0;
 }
 
-// src in the path's layout to the caller's state, after all that is queued.
-int stage_out(tdhf_ctx* c, double* dst, const zd* src) {
+// src, padded with kp, to the caller's state, after all that is queued.
+int stage_out(tdhf_ctx* c, bool kp, double* dst, const zd* src) {
   if (!c->h_stage) {
-    CHKRET(download_state(c, dst, src));
+    CHKRET(kp ? download_state(c, dst, src) : download(c, dst, src));
     return harvest_timing(c);
   }
   const size_t n = nstate(c);
   zd* h = c->h_stage + 2 * n;
-  if (c->kpath) {
+  if (kp) {
     CHKRET(kspace_layout(c, src, h, false));
   } else if (src != h) {
     hipLaunchKernelGGL(tdhf::stage_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
@@ -401,8 +424,8 @@ int path_observables_of(tdhf_ctx* c, const zd* u, double A, double* res7) {
   return sync(c);
 }
 
-// out = H[u] w on the path's layout.
-int path_hpsi(tdhf_ctx* c, const zd* u, const zd* w, double A, zd* out) {
+// out = H[u] w, padded states with kp.
+int path_hpsi(tdhf_ctx* c, bool kp, const zd* u, const zd* w, double A, zd* out) {
   tdhf::ApplyArgs a = base_args(c);
   a.mode = tdhf::M_HPSI;
   a.u = u;
@@ -410,7 +433,7 @@ int path_hpsi(tdhf_ctx* c, const zd* u, const zd* w, double A, zd* out) {
   a.A = A;
   a.Aobs = A;
   a.out = out;
-  return launch_stage(c, a);
+  return kp ? launch_kspace(c, a) : launch_apply(c, a, c->nb * c->nk);
 }
 
 }  // namespace

@@ -18,8 +18,8 @@ int te_series(tdhf_ctx* c, const zd* ua, const zd* ub, const zd* x, double Aave,
   const size_t bytes = path_count(c) * sizeof(zd);
   HIPCHK(c, hipMemcpyAsync(c->d_w, x, bytes, hipMemcpyDeviceToDevice, c->stream));
   for (int k = 1; k <= 4; ++k) {
-    CHKRET(path_hpsi(c, ua, c->d_w, Aave, c->d_out));
-    if (ub) CHKRET(path_hpsi(c, ub, c->d_w, Aave, c->d_ksum));
+    CHKRET(path_hpsi(c, c->kpath, ua, c->d_w, Aave, c->d_out));
+    if (ub) CHKRET(path_hpsi(c, c->kpath, ub, c->d_w, Aave, c->d_ksum));
     CHKRET(te_launch_update(c, c->d_out, ub ? c->d_ksum : nullptr, c->dt / (double)k, c->d_w, y));
   }
   return 0;

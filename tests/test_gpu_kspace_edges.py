@@ -73,6 +73,22 @@ def test_many_pulses_of_a_row_wise_system():
                 assert rel(g[t], g1[0]) < 1e-9 and rel(gu[t], gu1[0]) < 1e-9
 
 
+# either side of where one H application of host arrays takes the path, beside
+# steps of the same context, which do
+@pytest.mark.parametrize("case", [(64, 33, 9, 8), (64, 64, 13, 13), (128, 16, 13, 13), (128, 33, 12, 12),
+                                  (32, 65, 17, 17), (16, 128, 9, 9)],
+                         ids=lambda c: f"ng{c[0]}_nk{c[1]}")
+def test_one_application_between_steps(case):
+    case = case + CELL[case[0]]
+    S, O, G, _ = system(case)
+    u, w = orbitals(case, 1), orbitals(case, 2)
+    h, s = O.ubkwbk_hwbk(u, w, 0.2), O.RT_RK4_ubk(u, G.dt, 0.05, 0.1)
+    with G:
+        for _ in range(2):
+            assert rel(G.ubkwbk_hwbk(u, w, 0.2), h) < 1e-12
+            assert rel(G.RT_RK4_ubk(u, 0.05, 0.1), s) < 1e-12
+
+
 @pytest.mark.parametrize("case", [(16, 3, 2, 1), (64, 64, 8, 8)], ids=lambda c: f"ng{c[0]}_nk{c[1]}")
 def test_ground_state_ends_soon_after_a_bad_energy(case):
     """Orbitals that are not numbers: the first iteration's energy is none, and the
