@@ -464,20 +464,14 @@ __global__ void __launch_bounds__(512, NG == 16 ? 4 : 2) apply_kernel(ApplyArgs 
   const int wave_items =  // of its first group
       __builtin_amdgcn_readfirstlane((nitem - wave * GPW + ngrp - 1) / ngrp);
   lds_barrier();  // sW and sTw visible
-  // NG = 16 reads the twiddles where they are used (in registers they would cost
-  // it its occupancy), NG = 32 one of its two sets (they would spill)
+  // NG = 32 reads one of its two sets of twiddles where they are used (they would
+  // spill); read there at NG = 16, whose 122 registers hold both, they cost many
+  // passes 3 to 12 % (NG = 16, 140 k-points, 8 bands: 46.1 against 43.1 us)
   F fft;
-  if constexpr (NG > 16) fft.init_lds(sTw, l);
-  auto fwd = [&](zd (&v)[R]) {
-    if constexpr (NG == 16)
-      fft.fwd_lds(v, T, l, sTw);
-    else
-      fft.fwd(v, T, l);
-  };
+  fft.init_lds(sTw, l);
+  auto fwd = [&](zd (&v)[R]) { fft.fwd(v, T, l); };
   auto inv = [&](zd (&v)[R]) {
-    if constexpr (NG == 16)
-      fft.inv_lds(v, T, l, sTw);
-    else if constexpr (NG == 32)
+    if constexpr (NG == 32)
       fft.inv_t(v, T, l, [&](int g0) { return fft.fw[g0]; },
                 [&](int i) { return sTw[NG + l * R + i]; });
     else
