@@ -270,8 +270,8 @@ __host__ __device__ constexpr size_t apply_lds_bytes(int nw) {
 // TE: the Hartree and kinetic round trips as transforms (else circulant
 // products); the launcher chooses: transforms where the 1024 blocks of the
 // products at NG = 128 meet few waves.  Per stage, transforms against products: NG = 128
-// with two waves 7.3 against 8.2 us, four 8.0 against 7.8, eight 12.8 against
-// 12.5; NG = 64 with one wave 6.3 against 6.0, two 6.45 against 5.6.
+// with two waves 7.3 against 8.2 us, four 8.0 against 8.05, eight 12.8 against
+// 12.7; NG = 64 with one wave 6.3 against 6.2, two 6.45 against 5.8.
 template <int NG>
 __host__ __device__ constexpr bool apply_by_transforms(int nw) {
   return NG == 128 && nw < 4;
@@ -640,12 +640,27 @@ __global__ void __launch_bounds__(512, NG == 16 ? 4 : 2) apply_kernel(ApplyArgs 
     // B^2 products (one read each per product: the LDS bandwidth, 0.85 us at
     // NG = 64, now 0.4).  The threads of a wave with the same x add theirs in
     // registers; the sums are parked in the slot area (free after the
-    // reduction) as [wave][value][x], and thread x adds those in order ----
+    // reduction) as [wave][value][x], and thread x adds those in order.  From
+    // NG = 64 the products are of the differences to the value at x (each kernel
+    // sums to zero: no term at G = 0): K_2 is hundreds near d = 0 and alternates,
+    // and what cancels in its sum costs digits that the transforms keep (kinetic
+    // energy at NG = 128: 4e-15 of it, 2e-16 with the differences or by Parseval;
+    // H w 3e-14 and 4e-15).  They cost 0.1 us with four waves, 0.3 with one ----
+    constexpr bool DIFF = NG >= 64;
     constexpr int B = CB, XN = NG / B, NV = (5 * B * XN + 63) / 64 * 64 / XN, VF = NV * XN / 64;
     const int xr = tid % XN;
     if (wave < CW) {
       double s5[NV];
       static_for<0, NV>([&](auto kc) { s5[decltype(kc)::value] = 0.0; });
+      zd wx[B];
+      double rx[B];
+      if constexpr (DIFF) {
+        static_for<0, B>([&](auto ic) {
+          constexpr int i = decltype(ic)::value;
+          wx[i] = sW[xr + i * XN];
+          rx[i] = sRho[xr + i * XN];
+        });
+      }
       for (int yr = tid / XN; yr < XN; yr += nthr / XN) {
         double kh[B], k2[B];
         zd k1[B];
@@ -662,13 +677,19 @@ __global__ void __launch_bounds__(512, NG == 16 ? 4 : 2) apply_kernel(ApplyArgs 
           const double ry = sRho[yr + jj * XN];
           static_for<0, B>([&](auto ic) {
             constexpr int i = decltype(ic)::value, m = (i - jj + B) % B;
-            s5[i] = fma(kh[m], ry, s5[i]);
-            s5[B + i] = fma(k2[m], wy.x, s5[B + i]);
-            s5[2 * B + i] = fma(k2[m], wy.y, s5[2 * B + i]);
-            s5[3 * B + i] = fma(k1[m].x, wy.x, s5[3 * B + i]);
-            s5[3 * B + i] = fma(-k1[m].y, wy.y, s5[3 * B + i]);
-            s5[4 * B + i] = fma(k1[m].x, wy.y, s5[4 * B + i]);
-            s5[4 * B + i] = fma(k1[m].y, wy.x, s5[4 * B + i]);
+            zd d = wy;
+            double r = ry;
+            if constexpr (DIFF) {
+              d = zsub(wy, wx[i]);
+              r = ry - rx[i];
+            }
+            s5[i] = fma(kh[m], r, s5[i]);
+            s5[B + i] = fma(k2[m], d.x, s5[B + i]);
+            s5[2 * B + i] = fma(k2[m], d.y, s5[2 * B + i]);
+            s5[3 * B + i] = fma(k1[m].x, d.x, s5[3 * B + i]);
+            s5[3 * B + i] = fma(-k1[m].y, d.y, s5[3 * B + i]);
+            s5[4 * B + i] = fma(k1[m].x, d.y, s5[4 * B + i]);
+            s5[4 * B + i] = fma(k1[m].y, d.x, s5[4 * B + i]);
           });
         });
       }

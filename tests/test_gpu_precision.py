@@ -1,0 +1,72 @@
+"""Rounding errors of H and of the kinetic and Hartree energies against extended
+precision, where sums over the circulant kernels could lose digits that transforms
+keep.  Bounds: a kinetic energy by Parseval or by differences carries the rounding
+of its NG positive terms, below 10 2^-52 of it; H w carries 2^-52 of the largest
+(G + k + A)^2 / 2 times the orbital (250 of it at NG = 128 in the root mean
+square of the transform), of which half is allowed."""
+import numpy as np
+import pytest
+
+from mattohf_amd import tdhf as T
+from test_gpu_kspace import orbitals
+
+pytestmark = pytest.mark.gpu
+
+CELL = {64: (10.0, 6.0), 128: (12.0, 6.0)}
+L = np.longdouble
+EPS = 2.0 ** -52
+
+
+def dft(ng):
+    n = np.arange(ng)
+    t = 2 * L("3.14159265358979323846264338327950288") * (np.outer(n, n) % ng).astype(L) / ng
+    return np.cos(t) + 1j * np.sin(t)
+
+
+def exact(case, u, w, A, vcg, vq, vion):
+    """H[u] w (k, band, x), kinetic and Hartree energy of u."""
+    ng, nk, nb, nbocc, a, _ = case
+    n, F = np.arange(ng), dft(ng)
+    b = 2 * L("3.14159265358979323846264338327950288") / L(a)
+    g = np.array([i if i < ng // 2 else i - ng for i in range(ng)]).astype(L)
+    k = (-L(1) / 2 + (2 * np.arange(nk).astype(L) + 1) / (2 * nk)) * b
+    q = (g * b)[None, None, :] + k[:, None, None] + L(A)
+    U, W = (v.transpose(2, 1, 0).astype(np.clongdouble) for v in (u, w))
+    f = lambda z: np.einsum("xy,kiy->kix", F.conj(), z)  # noqa: E731
+    kin = np.einsum("xy,kiy->kix", F, q * q / 2 * f(W)) / ng
+    occ, dv = L(2) / nk, L(a) / ng
+    rho = occ * (np.abs(U[:, :nbocc]) ** 2).sum((0, 1))
+    vh = (F @ (vcg.astype(L) * (F.conj() @ rho.astype(np.clongdouble))) / ng).real
+    td = np.einsum("xy,dy->dx", F, vq.astype(L)) / ng
+    dm = np.einsum("qjx,qjy->qxy", U[:, :nbocc], U[:, :nbocc].conj())
+    y = (n[:, None] - n[None, :]) % ng
+    out = kin + (vh + vion.astype(L)) * W
+    for i in range(nk):
+        K = sum(td[i - j + nk - 1][y] * dm[j] for j in range(nk))
+        out[i] -= np.einsum("xy,iy->ix", K, W[i]) / nk
+    ek = occ * dv * (q * q / 2 * np.abs(f(U[:, :nbocc])) ** 2 / ng).sum()
+    return out, float(ek), float((vh * rho).sum() * dv / 2)
+
+
+def check(case, herr=0.5):
+    ng, nk, nb, nbocc, a, z = case
+    vion = T.ion_potential(ng, nk, a, [z], [1.0], [0.1])
+    u, w = orbitals(case, 1), orbitals(case, 2)
+    with T.TDHF(ng, nk, nb, nbocc, a, 0.004, vion) as G:
+        vcg, vq = G.tables()
+        h = G.ubkwbk_hwbk(u, w, 0.23)
+        ec = G.observables(u, 0.23)[1]
+    ref, ek, eh = exact(case, u, w, 0.23, vcg, vq, vion)
+    qmax = (np.pi * ng / a) ** 2 / 2
+    assert abs(ec[0] - ek) < 10 * EPS * ek, (ec[0] - ek) / ek
+    assert np.abs(h.transpose(2, 1, 0) - ref).max() < herr * EPS * qmax * np.abs(w).max() / np.sqrt(5)
+    return abs(ec[2] - eh) / eh
+
+
+# one to eight waves: transforms (NG = 128 with two) and products
+@pytest.mark.parametrize("case", [(64, 1, 1, 1), (64, 3, 2, 2), (64, 11, 3, 3), (128, 2, 2, 2),
+                                  (128, 4, 4, 4), (128, 8, 2, 2), (128, 16, 4, 3)],
+                         ids=lambda c: f"ng{c[0]}_nk{c[1]}")
+def test_row_wise(case):
+    case = case + CELL[case[0]]
+    assert check(case, 1.0 if case[:2] == (128, 2) else 0.5) < 1e-14
