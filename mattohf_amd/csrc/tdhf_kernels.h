@@ -311,7 +311,7 @@ __global__ void __launch_bounds__(512, NG == 16 ? 4 : 2) apply_kernel(ApplyArgs 
            "+s"(kc), "+s"(u), "+s"(w), "+s"(u0), "+s"(ksum), "+s"(unext), "+s"(obs));
   int wld = a.wld, balance = a.balance, nthr = blockDim.x;
   zd* tape = a.tape;
-  asm("" : "+s"(row), "+s"(wld), "+s"(balance), "+s"(nthr), "+s"(tape), "+s"(vion));
+  asm("" : "+s"(row), "+s"(wld), "+s"(balance), "+s"(nthr), "+s"(tape), "+s"(vion), "+s"(vhg));
   const int tr = blockIdx.y;  // trajectory of a uniform batch (0 otherwise)
   if (tr > 0) {
     Aarr += (size_t)tr * a.fstride;
@@ -542,9 +542,10 @@ __global__ void __launch_bounds__(512, NG == 16 ? 4 : 2) apply_kernel(ApplyArgs 
   // epilogue operands: loaded now, used after the reduction (whose barriers
   // order LDS only, so these loads stay in flight meanwhile)
   zd u0v = mk(0.0, 0.0), ksv = mk(0.0, 0.0);
-  double vionv = 0.0, khv = 0.0;
+  double vionv = 0.0, khv = 0.0, v0 = 0.0;
   if (tid < NG) {
     if constexpr (!TE) khv = gload(kc + tid);
+    if constexpr (!TE && NG >= 64) v0 = gload(vhg + lane0);  // vCG(0)/NG
     vionv = gload(vion + tid);
     if (mode >= M_S1 && mode <= M_S4) {
       u0v = gload(u0 + o);
@@ -641,11 +642,14 @@ __global__ void __launch_bounds__(512, NG == 16 ? 4 : 2) apply_kernel(ApplyArgs 
     // NG = 64, now 0.4).  The threads of a wave with the same x add theirs in
     // registers; the sums are parked in the slot area (free after the
     // reduction) as [wave][value][x], and thread x adds those in order.  From
-    // NG = 64 the products are of the differences to the value at x (each kernel
-    // sums to zero: no term at G = 0): K_2 is hundreds near d = 0 and alternates,
-    // and what cancels in its sum costs digits that the transforms keep (kinetic
-    // energy at NG = 128: 4e-15 of it, 2e-16 with the differences or by Parseval;
-    // H w 3e-14 and 4e-15).  They cost 0.1 us with four waves, 0.3 with one ----
+    // NG = 64 the products are of the differences to the value at x (the kernels
+    // sum to their terms at G = 0: none in K_2 and K_1; K_H's, zero unless a
+    // caller's table has one, is added in the epilogue): K_2 is hundreds near
+    // d = 0 and alternates, and what cancels in its sum costs digits that the
+    // transforms keep (kinetic energy at NG = 128: 4e-15 of it, 2e-16 with the
+    // differences or by Parseval; H w 3e-14 and 4e-15).  They cost 0.1 us with
+    // four waves, 0.3 with one ----
+    static_assert(F::gindex(0, 0) == 0, "vhg[0] is the term at G = 0");
     constexpr bool DIFF = NG >= 64;
     constexpr int B = CB, XN = NG / B, NV = (5 * B * XN + 63) / 64 * 64 / XN, VF = NV * XN / 64;
     const int xr = tid % XN;
@@ -727,6 +731,7 @@ __global__ void __launch_bounds__(512, NG == 16 ? 4 : 2) apply_kernel(ApplyArgs 
         c1.x += q[3 * NG];
         c1.y += q[4 * NG];
       }
+      if constexpr (NG >= 64) vh = fma(NG * v0, sRho[tid], vh);
       vh *= occ;  // the density sum holds sum |u|^2
       const double kA = kxv + akin();
       // T w = K_2 * w + (k+A) K_1 * w + (k+A)^2/2 w

@@ -48,11 +48,17 @@ def exact(case, u, w, A, vcg, vq, vion):
     return out, float(ek), float((vh * rho).sum() * dv / 2)
 
 
-def check(case, herr=0.5):
+def check(case, herr=0.5, v0=None):
+    """v0: a vCG(0) of the caller's."""
     ng, nk, nb, nbocc, a, z = case
     vion = T.ion_potential(ng, nk, a, [z], [1.0], [0.1])
     u, w = orbitals(case, 1), orbitals(case, 2)
-    with T.TDHF(ng, nk, nb, nbocc, a, 0.004, vion) as G:
+    vcg = None
+    if v0 is not None:
+        with T.TDHF(ng, nk, nb, nbocc, a, 0.004, vion) as G:
+            vcg = G.tables()[0]
+        vcg[0] = v0
+    with T.TDHF(ng, nk, nb, nbocc, a, 0.004, vion, vcg=vcg) as G:
         vcg, vq = G.tables()
         h = G.ubkwbk_hwbk(u, w, 0.23)
         ec = G.observables(u, 0.23)[1]
@@ -70,3 +76,12 @@ def check(case, herr=0.5):
 def test_row_wise(case):
     case = case + CELL[case[0]]
     assert check(case, 1.0 if case[:2] == (128, 2) else 0.5) < 1e-14
+
+
+@pytest.mark.parametrize("case", [(64, 3, 2, 2), (64, 11, 3, 3), (128, 2, 2, 2), (128, 8, 2, 2)],
+                         ids=lambda c: f"ng{c[0]}_nk{c[1]}")
+def test_row_wise_with_a_table_that_does_not_sum_to_zero(case):
+    """A Hartree table with a term at G = 0: a constant potential, kept by the
+    transforms and by the products of differences alike."""
+    case = case + CELL[case[0]]
+    assert check(case, 1.0 if case[:2] == (128, 2) else 0.5, v0=3.0) < 1e-14
