@@ -515,7 +515,7 @@ int batch_layout(tdhf_batch* b, bool padded) {
   l.koff = b->d_koff;
   l.to_k = padded;
   hipLaunchKernelGGL(tdhf::kspace_layout_kernel,
-                     dim3(b->p.ng / 16, b->kmax / 16, b->p.nb * b->ntraj), dim3(256), 0, b->stream,
+                     dim3(b->p.nb * b->ntraj, b->kmax / 16, b->p.ng / 16), dim3(256), 0, b->stream,
                      l);
   BHIP(b, hipGetLastError());
   BHIP(b, hipMemcpyAsync(b->d_state, tmp, b->region * sizeof(zd), hipMemcpyDeviceToDevice,

@@ -786,7 +786,7 @@ struct KLayoutArgs {
   zd* dst;
   int ng, nb, nk, n;
   int ld;                   // columns per k-point of the (NG,.,NK) side (0: nb)
-  size_t sstride, dstride;  // per trajectory (grid z = trajectory * nb + band)
+  size_t sstride, dstride;  // per trajectory
   // batch: offsets and k-meshes of the trajectories instead
   const TrajDesc* td;
   const size_t* roff;       // of the (NG,NB,NK) states
@@ -794,10 +794,12 @@ struct KLayoutArgs {
   int to_k;
 };
 
-// 16 x 16 tiles through LDS, so that both sides move 256-byte runs.
+// 16 x 16 tiles through LDS, so that both sides move 256-byte runs.  The grid's x is
+// trajectory * nb + band, the only count without a small bound (a grid's y and z
+// end at 65535, x at 2^32 threads), y the k and z the x tile.
 __global__ void __launch_bounds__(256) kspace_layout_kernel(KLayoutArgs a) {
   __shared__ zd s[16][17];
-  const int tr = blockIdx.z / a.nb, b = blockIdx.z - tr * a.nb, ld = a.ld ? a.ld : a.nb;
+  const int tr = blockIdx.x / a.nb, b = blockIdx.x - tr * a.nb, ld = a.ld ? a.ld : a.nb;
   int nk = a.nk, n = a.n;
   size_t ro = a.to_k ? tr * a.sstride : tr * a.dstride;
   size_t ko = a.to_k ? tr * a.dstride : tr * a.sstride;
@@ -807,7 +809,7 @@ __global__ void __launch_bounds__(256) kspace_layout_kernel(KLayoutArgs a) {
     ro = a.roff[tr];
     ko = a.koff[tr];
   }
-  const int x0 = blockIdx.x * 16, k0 = blockIdx.y * 16;
+  const int x0 = blockIdx.z * 16, k0 = blockIdx.y * 16;
   if (k0 >= n) return;
   const int p = threadIdx.x & 15, q = threadIdx.x >> 4;
   if (a.to_k) {

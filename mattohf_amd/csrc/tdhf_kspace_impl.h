@@ -307,7 +307,7 @@ int kspace_layout(tdhf_ctx* c, const zd* src, zd* dst, bool to_k, int ntraj = 1,
   l.sstride = to_k ? nstate(c) : kcount(c);
   l.dstride = to_k ? kcount(c) : nstate(c);
   l.to_k = to_k;
-  hipLaunchKernelGGL(tdhf::kspace_layout_kernel, dim3(c->ng / 16, c->kn / 16, nb * ntraj),
+  hipLaunchKernelGGL(tdhf::kspace_layout_kernel, dim3(nb * ntraj, c->kn / 16, c->ng / 16),
                      dim3(256), 0, st ? st : c->stream, l);
   HIPCHK(c, hipGetLastError());
   return 0;
