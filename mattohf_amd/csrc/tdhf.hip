@@ -219,8 +219,9 @@ int choose_nw(int ng, int nk, int nbocc) {
   const int items = nk * nbocc;
   int nw = (items + gpw - 1) / gpw;
   // one pair per lane group; up to 64 pairs at NG = 64 run as two per group on
-  // half the waves, which share the SIMDs with no other (7.1 against 7.3 us per
-  // stage; 128 pairs 9.9 against 9.2)
+  // half the waves, which share the SIMDs with no other (stage of 15 pairs 5.5
+  // against 5.8 us, 21 5.7 and 6.1, 32 5.75 and 6.2, 64 7.2 and 7.5; 128 pairs 9.9
+  // against 9.2)
   if (nw > 8) nw = 8;
   if (ng == 64 && items <= 64 && nw > 4) nw = 4;
   if (nw < 1) nw = 1;
@@ -795,7 +796,7 @@ int tdhf_create(const tdhf_params* p, const double* vion, const double* vcg, con
     return bail(TDHF_EDEVICE);
   }
   c->kn = tdhf::kspace_len(c->nk);
-  c->kpath = kspace_pays(c->ng, c->nk, c->nb, c->nbocc, 1);
+  c->kpath = kspace_run_pays(c);
   rc = alloc_states(c);
   if (rc == TDHF_ENOMEM && c->kpath) {  // no memory for the padded states and matrices
     free_states(c);

@@ -10,9 +10,13 @@ namespace {
 // measured over NG = 16..128, NK = 4..128, NB = 1..8 and 1..64 trajectories.
 // Row-wise: 5.5 + 0.42 per 10^6 grid points in the pair transforms, weighted by
 // log2 NG.  Density matrices: 13 (two launches, each with its own memory round
-// trips) + 12 per 10^6 matrix elements.  Near the line: NG=64, NK=64, NB=4
-// (one trajectory) 14.4 against 16.0 stays row-wise; NG=128, NK=64, NB=4 32.5
-// against 27.8 does not.
+// trips) + 12 per 10^6 matrix elements.  Both are averages: the row-wise time goes
+// up in rounds of 256 workgroups (NG=64, NB=4: 256 rows of NK=64 13.4, 260 of NK=65
+// 25.6), the other with the bands too.  Near the line, measured, row-wise against
+// matrices: NG=128, NK=64, NB=4 31.0 and 27.3, NK=16, NB=11 23.2 and 20.5; NG=64,
+// NK=33, NB=8 25.7 and 20.7; NG=32, NK=65, NB=6 22.8 and 18.0 take the matrices,
+// NG=128, NK=48, NB=4 24.8 and 27.3; NG=64, NK=32, NB=6 11.1 and 16.4; NG=32, NK=24,
+// NB=11 17.8 and 17.9; NG=16, NK=128, NB=4 11.9 and 14.7 do not.
 struct KspaceCost {
   double rows = 0.0, mat = 0.0;
   bool fits = true;  // kapply_kernel's byte offsets into a padded state are 32 bits wide
@@ -23,7 +27,8 @@ struct KspaceCost {
     mat += 1e-6 * ntraj * (double)ng * ng * tdhf::kspace_len(nk);
     fits = fits && (size_t)ng * nb * tdhf::kspace_len(nk) * sizeof(zd) <= UINT32_MAX;
   }
-  double gain() const { return fits ? 5.5 + 0.42 * rows - (13.0 + 12.0 * mat) : 0.0; }
+  double matrices() const { return 13.0 + 12.0 * mat; }
+  double gain() const { return fits ? 5.5 + 0.42 * rows - matrices() : 0.0; }
   bool pays() const { return gain() > 0.0; }
 };
 
@@ -32,6 +37,25 @@ bool kspace_pays(int ng, int nk, int nb, int nbocc, int ntraj) {
   KspaceCost c;
   c.add(ng, nk, nb, nbocc, ntraj);
   return c.pays();
+}
+
+// The same for a context's own runs.  Where all rows have a CU each (one round of
+// the row-wise kernel) the averages above mislead, most at NG = 64: the row-wise
+// stage is then 5.5 us + 0.030 per pair of a row, at NG = 128 7.0 + 0.093, and the
+// matrices' with more than four bands a quarter above their price.  Row-wise
+// against matrices: NG=64, NK=32, NB=8 13.5 and 17.5, NK=16, NB=16 13.5 and 18.6;
+// NG=128, NK=40, NB=6 30.0 and 32.5, NK=16, NB=16 with 8 occupied 18.7 and 20.1 are
+// row-wise, NK=24, NB=8 24.8 and 23.7, NK=64, NB=4 31.0 and 27.3 are not.
+// (Gradients, whose reverse stage gains more, are faster through the matrices
+// there too.)
+bool kspace_run_pays(const tdhf_ctx* c) {
+  if (!kspace_pays(c->ng, c->nk, c->nb, c->nbocc, 1)) return false;
+  if (c->ng < 64 || (long)c->nk * c->nb > device_cus()) return true;
+  const double pairs = (double)c->nk * c->nbocc;
+  const double rows = c->ng == 64 ? 5.5 + 0.030 * pairs : 7.0 + 0.093 * pairs;
+  KspaceCost k;
+  k.add(c->ng, c->nk, c->nb, c->nbocc);
+  return rows > k.matrices() * (c->nb > 4 ? 1.25 : 1.0);
 }
 
 // Whether one H application of host arrays pays on the path.  Its two states and

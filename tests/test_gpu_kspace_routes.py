@@ -56,6 +56,16 @@ def test_more_trajectories_than_a_grid_has_in_z():
         assert rel(g[t], gref[t % 3][0]) < 1e-9 and rel(gu[t], gref[t % 3][1]) < 1e-9
 
 
+def launches(case):
+    """Of a ground-state iteration with one Krylov block."""
+    ng, nk, nb, nbocc, a, z = case
+    vion = T.ion_potential(ng, nk, a, [z], [1.0], [0.0])
+    with T.TDHF(ng, nk, nb, nbocc, a, 0.004, vion) as G:
+        G.set_kernel_timing(True)
+        G.GS_calculation(orbitals(case, 1), 1, 1)
+        return G.kernel_stats()[0]
+
+
 @pytest.mark.parametrize("case", [c for c in SYSTEMS if c[:4] != (128, 17, 11, 10)] + [SECOND_BLOCK],
                          ids=lambda c: f"ng{c[0]}_nk{c[1]}")
 def test_systems_take_the_path(case):
@@ -63,12 +73,27 @@ def test_systems_take_the_path(case):
     one with 13 bands; with 11 it is row-wise): a ground-state iteration makes the
     matrices apart from their products, three launches more than the row-wise
     five."""
-    ng, nk, nb, nbocc, a, z = case
-    vion = T.ion_potential(ng, nk, a, [z], [1.0], [0.0])
-    with T.TDHF(ng, nk, nb, nbocc, a, 0.004, vion) as G:
-        G.set_kernel_timing(True)
-        G.GS_calculation(orbitals(case, 1), 1, 1)
-        assert G.kernel_stats()[0] == 8
+    assert launches(case) == 8
+
+
+@pytest.mark.parametrize("case", [(64, 32, 8, 8), (64, 16, 16, 16), (128, 40, 6, 6), (128, 16, 16, 8)],
+                         ids=lambda c: f"ng{c[0]}_nk{c[1]}")
+def test_one_round_of_rows_is_row_wise(case):
+    """Up to 256 rows, one for each CU: the row-wise kernel is the faster one."""
+    assert launches(case + CELL[case[0]]) == 5
+
+
+def test_largest_pinned_state():
+    """16384 elements, the most that go through pinned memory, on the path."""
+    case = (32, 64, 8, 8) + CELL[32]
+    assert launches(case) == 8
+    S, O, G, _ = system(case)
+    with G:
+        for seed in (1, 2):  # (the memory is used again)
+            u, w = orbitals(case, seed), orbitals(case, 10 + seed)
+            assert rel(G.ubkwbk_hwbk(u, w, 0.2), O.ubkwbk_hwbk(u, w, 0.2)) < 1e-12
+            assert rel(G.RT_RK4_ubk(u, 0.05, 0.1), O.RT_RK4_ubk(u, G.dt, 0.05, 0.1)) < 1e-12
+            np.testing.assert_array_equal(G.download(), G.RT_RK4_ubk(u, 0.05, 0.1))
 
 
 def test_just_past_a_transform_length_with_an_empty_band():
