@@ -893,21 +893,28 @@ int tdhf_batch_create(const tdhf_params* p, int ntraj, const int* nk, const doub
   // rows per CU (NG=64, 558 rows: 16.8 -> 14.7 us per stage; NG=16, 800: 8.1 ->
   // 7.7), and for up to two rows per CU, whose CUs have room, four and the rows
   // spread over all XCDs (NG=64, 93 rows: 15.7 -> 7.8; 279: 16.3 -> 9.4; NG=32,
-  // 156: 9.1 -> 6.8; 312: 9.5 -> 8.7)
+  // 156: 9.1 -> 6.8; 312: 9.5 -> 8.7).  A CU holds eight waves at once (16 at
+  // NG = 16): where the fullest XCD has between five and eight rows per CU, they
+  // fit with one wave each and take a second round with two (NG=32, 6 rows: 31.1
+  // and 34.6 us; NG=64, 5.25: 28.8 and 31.3; but 4.5: 41.2 and 35.4, 5: 45.6 and
+  // 38.9, 8.75: 114 and 101; NG=16, 12: 37.2 and 39.3, 8: 21.1 and 18.7)
   std::array<int, 3> ct{};
   const bool cached = tune_lookup(tune_key(b), &ct);
   // (density matrices: 8 waves for the product launch, 4 where it has
   // workgroups enough; fewer trajectories than XCDs are not pinned to them,
   // NG=128, NK=128, NB=8: 4 trajectories 166 us per stage pinned, 101 not)
   const long rows = (long)p->nb * std::accumulate(nk, nk + ntraj, 0L), cus = device_cus();
-  const int fit = choose_nw(p->ng, *std::max_element(nk, nk + ntraj), p->nbocc);
-  const int nwr = std::max((p->ng + 63) / 64,
-                           std::min(fit, rows <= 2 * cus ? 4 : rows <= 4 * cus ? 2 : 1));
-  b->nw = cached ? ct[0] : !b->kuse ? nwr : batch_points(b) > 1 ? 4 : 8;
   b->ngrid = 0;
   if ((rc = batch_set_schedule(
            b, cached ? ct[1] : (b->kuse ? ntraj < 8 : rows <= 2 * cus) ? 2 : 0)))
     return bail(rc);
+  const int fit = choose_nw(p->ng, *std::max_element(nk, nk + ntraj), p->nbocc);
+  const long full = p->ng == 16 ? 2 * cus : cus;
+  const bool one = b->ngrid > 5 * full && b->ngrid <= 8 * full;
+  const int nwr = std::max((p->ng + 63) / 64, std::min(fit, rows <= 2 * cus         ? 4
+                                                            : rows <= 4 * cus && !one ? 2
+                                                                                      : 1));
+  b->nw = cached ? ct[0] : !b->kuse ? nwr : batch_points(b) > 1 ? 4 : 8;
   b->h_td.resize(ntraj);
   if ((rc = batch_update_desc(b))) return bail(rc);
   if (cached && ct[2] && (rc = batch_set_xmode(b, ct[2]))) return bail(rc);

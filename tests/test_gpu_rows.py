@@ -94,3 +94,22 @@ def test_default_batch_shape(ng, nb, nks, ntraj):
     for u, v in zip(out[0][0], out[1][0]):
         assert rel(u, v) < 1e-12
     assert np.abs(out[0][1] - out[1][1]).max() < 1e-10 and rel(out[0][2], out[1][2]) < 1e-8
+
+
+# waves of a row by the rows of the fullest XCD: 5 per CU, 6, 9 (12 at NG = 16)
+@pytest.mark.parametrize("ng,nk,nb,ntraj,waves", [(64, 40, 4, 5, 2), (32, 48, 4, 4, 1),
+                                                  (32, 140, 2, 2, 2), (16, 96, 4, 2, 1)])
+def test_default_batch_waves(ng, nk, nb, ntraj, waves):
+    a, z = {16: A16, 32: A32, 64: A64, 128: A128}[ng]
+    vion = T.ion_potential(ng, nk, a, [z], [1.0], [0.0])
+    u = orbitals((ng, nk, nb, nb, a, z), 1)
+    A = np.tile([0.05, 0.1], (ntraj, 1))
+    with T.TDHF(ng, nk, nb, nb, a, 0.004, vion) as G:
+        ref = G.RT_calculation(u, A[0], A[0])
+    with T.Batch(ng, nb, nb, a, 0.004, [nk] * ntraj, np.array([vion] * ntraj)) as B:
+        assert B.waves() == waves
+        B.upload([u] * ntraj)
+        e = B.propagate(A, A)[0]
+        out = B.download()
+    for t in (0, ntraj - 1):
+        assert rel(out[t], ref[0]) < 1e-12 and np.abs(e[t] - ref[1]).max() < 1e-10
