@@ -408,12 +408,15 @@ long batch_tasks(const tdhf_batch* b) {
   return tasks;
 }
 
-int batch_points(const tdhf_batch* b) {
+// Workgroups of the product launch at one grid point each.
+long batch_groups(const tdhf_batch* b) {
   long groups = 0;
   for (int t = 0; t < b->ntraj; ++t)
     groups += kapply_groups(b->tabs[b->tab_of[t]]->kn, b->p.ng, b->p.nb, 1);
-  return kapply_points(groups);
+  return groups;
 }
+
+int batch_points(const tdhf_batch* b) { return kapply_points(batch_groups(b)); }
 
 // Work lists of the two launches for the current row schedule: per trajectory
 // its groups of (x, block) tasks and its (x tile, bands, k block) items, the
@@ -901,7 +904,9 @@ int tdhf_batch_create(const tdhf_params* p, int ntraj, const int* nk, const doub
   std::array<int, 3> ct{};
   const bool cached = tune_lookup(tune_key(b), &ct);
   // (density matrices: 8 waves for the product launch, 4 where it has
-  // workgroups enough; fewer trajectories than XCDs are not pinned to them,
+  // workgroups enough, which at NG = 16, where eight waves have an x' or two each,
+  // is one per CU: 30 trajectories of NK=21, NB=6 23.9 -> 16.8 us, of NK=40, NB=4
+  // 22.3 -> 17.4; fewer trajectories than XCDs are not pinned to them,
   // NG=128, NK=128, NB=8: 4 trajectories 166 us per stage pinned, 101 not)
   const long rows = (long)p->nb * std::accumulate(nk, nk + ntraj, 0L), cus = device_cus();
   b->ngrid = 0;
@@ -914,7 +919,8 @@ int tdhf_batch_create(const tdhf_params* p, int ntraj, const int* nk, const doub
   const int nwr = std::max((p->ng + 63) / 64, std::min(fit, rows <= 2 * cus         ? 4
                                                             : rows <= 4 * cus && !one ? 2
                                                                                       : 1));
-  b->nw = cached ? ct[0] : !b->kuse ? nwr : batch_points(b) > 1 ? 4 : 8;
+  const bool enough = b->kuse && (batch_points(b) > 1 || (p->ng == 16 && batch_groups(b) >= cus));
+  b->nw = cached ? ct[0] : !b->kuse ? nwr : enough ? 4 : 8;
   b->h_td.resize(ntraj);
   if ((rc = batch_update_desc(b))) return bail(rc);
   if (cached && ct[2] && (rc = batch_set_xmode(b, ct[2]))) return bail(rc);

@@ -96,9 +96,11 @@ def test_default_batch_shape(ng, nb, nks, ntraj):
     assert np.abs(out[0][1] - out[1][1]).max() < 1e-10 and rel(out[0][2], out[1][2]) < 1e-8
 
 
-# waves of a row by the rows of the fullest XCD: 5 per CU, 6, 9 (12 at NG = 16)
+# waves of the product launch (density matrices) or of a row, by the rows of the
+# fullest XCD: 5 per CU, 6, 9 (12 at NG = 16); 480 workgroups of matrices at NG = 16
 @pytest.mark.parametrize("ng,nk,nb,ntraj,waves", [(64, 40, 4, 5, 2), (32, 48, 4, 4, 1),
-                                                  (32, 140, 2, 2, 2), (16, 96, 4, 2, 1)])
+                                                  (32, 140, 2, 2, 2), (16, 96, 4, 2, 1),
+                                                  (16, 21, 6, 30, 4)])
 def test_default_batch_waves(ng, nk, nb, ntraj, waves):
     a, z = {16: A16, 32: A32, 64: A64, 128: A128}[ng]
     vion = T.ion_potential(ng, nk, a, [z], [1.0], [0.0])
