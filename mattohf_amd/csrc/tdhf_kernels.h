@@ -831,39 +831,43 @@ struct CompSum {
   __device__ __forceinline__ double value() const { return s + c; }
 };
 
-// Adds the sums of the 64 lanes of a wave, compensated and in a fixed order;
-// the same in every lane.
-__device__ __forceinline__ void comp_wave_sum(CompSum& c) {
+// Adds the sums of the first n lanes of a wave (the others' are zero), compensated
+// and in a fixed order; M sums at a time, whose exchanges overlap; in lane 0.
+template <int M>
+__device__ __forceinline__ void comp_wave_sum(CompSum (&c)[M], int n) {
   const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const double os = __shfl_xor(c.s, off), oc = __shfl_xor(c.c, off);
-    // the same pair of operands in both lanes of the exchange
-    const double lo = (lane & off) ? os : c.s, hi = (lane & off) ? c.s : os;
-    CompSum r;
-    r.add(lo);
-    r.add(hi);
-    r.c += c.c + oc;
-    c = r;
+  for (int off = 1; off < 64 && off < n; off <<= 1) {
+    static_for<0, M>([&](auto mc) {
+      constexpr int m = decltype(mc)::value;
+      const double os = __shfl_xor(c[m].s, off), oc = __shfl_xor(c[m].c, off);
+      // the same pair of operands in both lanes of the exchange
+      const double lo = (lane & off) ? os : c[m].s, hi = (lane & off) ? c[m].s : os;
+      CompSum r;
+      r.add(lo);
+      r.add(hi);
+      r.c += c[m].c + oc;
+      c[m] = r;
+    });
   }
 }
 
 // Sums the per-row partials of one observables slot p (rows rows) into
 // (Etot, N, J, Ekin, Eion, EH, Ex), src/Functions.f90:74-91 and :289-318; one
 // wave per slot, rows lane, lane + 64, ... of a lane first (one thread per slot
-// took 78 us for 256 rows, one wave 5 us).
+// took 78 us for 256 rows, one wave 5 us; four rows need two of the six exchanges
+// of the lanes' sums: tdhf_observables 31.8 us, 33.0 with all six one by one, 32.3
+// with one thread).
 __device__ __forceinline__ void obs_reduce_slot(const double* p, int rows, double dv, double vcell,
                                                 double* o) {
   const int lane = threadIdx.x & 63;
-  CompSum ek, jj, ex;
+  CompSum c[3];
   for (int r = lane; r < rows; r += 64) {
-    ek.add(p[3 * r + 0]);
-    jj.add(p[3 * r + 1]);
-    ex.add(p[3 * r + 2]);
+    c[0].add(p[3 * r + 0]);
+    c[1].add(p[3 * r + 1]);
+    c[2].add(p[3 * r + 2]);
   }
-  comp_wave_sum(ek);
-  comp_wave_sum(jj);
-  comp_wave_sum(ex);
+  comp_wave_sum(c, rows);
+  const CompSum &ek = c[0], &jj = c[1], &ex = c[2];
   if (lane != 0) return;
   const double n = p[3 * rows + 0], ei = p[3 * rows + 1], eh = p[3 * rows + 2];
   CompSum et;

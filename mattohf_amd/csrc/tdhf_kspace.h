@@ -845,7 +845,7 @@ __global__ void __launch_bounds__(256) kspace_obs_reduce_kernel(const double* ob
   CompSum c[6];
   for (int x = lane; x < ng; x += 64)
     for (int m = 0; m < 6; ++m) c[m].add(p[6 * x + m]);
-  for (int m = 0; m < 6; ++m) comp_wave_sum(c[m]);
+  comp_wave_sum(c, 64);
   if (lane == 0) {
     CompSum et;
     et.add(c[0].s);
