@@ -425,7 +425,7 @@ def adjoint_full_bench(npulse=8, nt=8000, seed=20261206, gs_iters=40, fd=True):
     segment.  Reports the plain batched forward of the same pulses over the
     same steps, the gradient cost relative to it, and central finite
     differences of every pulse's L along one random direction (two more
-    checkpointed forwards).  Opt-in (--only adjoint-full): ~10 minutes at
+    checkpointed forwards).  Opt-in (--only adjoint-full): about a minute at
     npulse = 8; progress lines go to stderr."""
     from mattohf_amd import tdhf as T
 

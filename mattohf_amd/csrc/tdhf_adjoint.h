@@ -281,8 +281,8 @@ __global__ void __launch_bounds__(512, XP ? 3 : 2) adjoint_kernel(AdjArgs a0) {
     sv[m] = 0.0;
   });
   lds_barrier();
-  // NG = 32 reads the transforms' lane twiddles where they are used: its two
-  // register sets of them would spill
+  // from NG = 32 the transforms' lane twiddles are read where they are used: in
+  // registers they would spill (72, 28 and 42 registers at NG = 32, 64 and 128)
   F fft;
   constexpr bool LTW = NG >= 32;
   if constexpr (!XP && !LTW) fft.init_lds(sTw, l);

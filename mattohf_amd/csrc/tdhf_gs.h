@@ -2,7 +2,7 @@
 // iteration: GS_calculation, KS_ubk2_SVD and Subspace_diag
 // (src/GS_calculation.f90:26-57,124-237).
 //
-// The H applications reuse the context's path (gs_apply).  The small per-k
+// The H applications reuse the context's path (gs_product).  The small per-k
 // dense steps run one workgroup per k-point, on columns held in LDS:
 //   orth_kernel : dvcell-weighted modified Gram-Schmidt, right-looking: once a
 //                 column is normalised, its projection leaves all later ones,
