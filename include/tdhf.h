@@ -312,8 +312,9 @@ int tdhf_batch_run(const tdhf_params* p, int ntraj, const int* nk, const double*
                    double* nele, double* jtot, double* init3);
 /* Launch shape: waves per workgroup of the fused kernel, with pair tiles of
  * the per-row epilogue launch, with density matrices of their product with the
- * orbitals (1, 2, 4 or 8, at least NG/64; default the smallest, with density
- * matrices 4 or 8).
+ * orbitals (1 to 8, at least NG/64; of the last the largest power of two that
+ * is not more; default 1, 2 or 4 by the rows per CU, with density matrices 4 or
+ * 8).
  * tdhf_batch_autotune times nt_trial steps for each candidate on a copy of the
  * state (the batch state is unchanged), keeps the fastest and remembers it for
  * batches of the same shape created later in the process; best_nw receives
@@ -326,7 +327,8 @@ int tdhf_batch_autotune(tdhf_batch* b, int nt_trial, const double* A, const doub
  * row, and so on which XCD): 0 = trajectories bin-packed over the XCDs (a
  * trajectory's rows on one XCD, contiguous; the default), 1 = the same with
  * the rows of an XCD's trajectories interleaved, 2 = no XCD pinning (the
- * default for fewer than 8 trajectories with density matrices).  The
+ * default up to two rows per CU, with density matrices for fewer than 8
+ * trajectories).  The
  * results do not depend on it.  tdhf_batch_autotune times every (exchange
  * evaluation, schedule, waves per workgroup) combination and keeps the
  * fastest. */
