@@ -96,3 +96,36 @@ def test_row_wise_where_the_padding_does_not_fit():
             assert rel(D.state(), ref) < 1e-12
         finally:
             D.close()
+
+
+# density matrices, row-wise
+@pytest.mark.parametrize("case", [(64, 33, 13, 12, 10.0, 6.0), (32, 4, 2, 2, 8.0, 4.0)],
+                         ids=lambda c: f"ng{c[0]}_nk{c[1]}")
+def test_captured_step(case):
+    """One step captured into a graph and replayed, with calls of the context
+    between: every replay is the step of tdhf_rk4_step."""
+    G, u = system(case)
+    with G:
+        D = Device(u)
+        hip = D.hip
+        graph, run = C.c_void_p(), C.c_void_p()
+        hip.hipStreamBeginCapture.argtypes = [C.c_void_p, C.c_int]
+        hip.hipStreamEndCapture.argtypes = [C.c_void_p, C.POINTER(C.c_void_p)]
+        hip.hipGraphInstantiate.argtypes = [C.POINTER(C.c_void_p), C.c_void_p, C.c_void_p, C.c_void_p,
+                                            C.c_size_t]
+        hip.hipGraphLaunch.argtypes = [C.c_void_p, C.c_void_p]
+        hip.hipGraphExecDestroy.argtypes = hip.hipGraphDestroy.argtypes = [C.c_void_p]
+        try:
+            assert hip.hipStreamBeginCapture(D.stream, 1) == 0
+            D.step(G, 0.05, 0.1)
+            assert hip.hipStreamEndCapture(D.stream, C.byref(graph)) == 0
+            assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, 0) == 0
+            np.testing.assert_array_equal(D.state(), u)  # nothing ran yet
+            for _ in range(4):
+                assert hip.hipGraphLaunch(run, D.stream) == 0
+                u = G.RT_RK4_ubk(u, 0.05, 0.1)
+                assert rel(D.state(), u) < 1e-13
+            hip.hipGraphExecDestroy(run)
+            hip.hipGraphDestroy(graph)
+        finally:
+            D.close()
