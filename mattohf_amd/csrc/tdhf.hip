@@ -242,15 +242,23 @@ int device_cus() {
   return n;
 }
 
+// pairs: of a row (a batch's largest), where rows of one wave may have many
 template <int NG>
 void launch_apply_t(const tdhf::ApplyArgs& a, int rows, int ntraj, int nw, size_t lds,
-                    hipStream_t s) {
+                    hipStream_t s, long pairs = 0) {
   tdhf::ApplyArgs b = a;
   // wave-priority balancing pays only when the grid is one workgroup per CU
   b.balance = (long)rows * ntraj <= device_cus() ? 1 : 0;
   if constexpr (NG == 128) {
     if (tdhf::apply_by_transforms<NG>(nw)) {
       hipLaunchKernelGGL((tdhf::apply_kernel<NG, true>), dim3(rows, ntraj), dim3(64 * nw), lds, s,
+                         b);
+      return;
+    }
+  }
+  if constexpr (NG == 32) {
+    if (nw == 1 && pairs >= tdhf::kOnePairs) {
+      hipLaunchKernelGGL((tdhf::apply_kernel<NG, false, true>), dim3(rows, ntraj), dim3(64), lds, s,
                          b);
       return;
     }

@@ -31,6 +31,7 @@ struct tdhf_batch {
   std::vector<int> tab_of;
   std::vector<size_t> off;      // state offset (complex elements) per trajectory
   size_t total = 0;             // complex elements of all trajectories
+  long pairs = 0;               // of a row (occupied bands of all k-points), the most
   // density-matrix path (tdhf_kspace.h): whether mode 0 takes it, the padded
   // state offsets, the layout d_state's first region is in, matrices and
   // density scratch per trajectory, the two launches' work lists
@@ -576,7 +577,7 @@ int batch_launch(tdhf_batch* b, const tdhf::ApplyArgs& a, int nw) {
     const size_t lds = lds_for(b->p.ng, nw);
     switch (b->p.ng) {
       case 16: launch_apply_t<16>(a, b->ngrid, 1, nw, lds, b->stream); break;
-      case 32: launch_apply_t<32>(a, b->ngrid, 1, nw, lds, b->stream); break;
+      case 32: launch_apply_t<32>(a, b->ngrid, 1, nw, lds, b->stream, b->pairs); break;
       case 64: launch_apply_t<64>(a, b->ngrid, 1, nw, lds, b->stream); break;
       case 128: launch_apply_t<128>(a, b->ngrid, 1, nw, lds, b->stream); break;
     }
@@ -889,6 +890,7 @@ int tdhf_batch_create(const tdhf_params* p, int ntraj, const int* nk, const doub
     bfail(b, TDHF_EDEVICE, "vion upload failed");
     return bail(TDHF_EDEVICE);
   }
+  b->pairs = (long)*std::max_element(nk, nk + ntraj) * p->nbocc;
   // launch shape and row schedule: the cached autotuner choice, else, row-wise,
   // the fewest waves per workgroup that cover the grid (one at NG <= 64: the
   // groups of a single wave need no workgroup barrier, and eight such

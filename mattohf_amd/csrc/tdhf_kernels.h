@@ -277,7 +277,13 @@ __host__ __device__ constexpr bool apply_by_transforms(int nw) {
   return NG == 128 && nw < 4;
 }
 
-template <int NG, bool TE>
+// ONE: at NG = 32, rows of one wave with many passes: twiddles in registers,
+// multipliers read at the start of their pass, not ahead of it, and no last pass of
+// its own.  12 trajectories of 140 k-points, 4 bands 319 us per stage against 329
+// (8 bands 1.21 against 1.25 ms); the same form costs 120 pairs a row 24.6 against
+// 23.8 and eight waves (16 k-points, 16 bands) 10.5 against 9.3.
+constexpr int kOnePairs = 192;  // pairs a row from which it pays
+template <int NG, bool TE, bool ONE = false>
 __global__ void __launch_bounds__(512, NG == 16 ? 4 : 2) apply_kernel(ApplyArgs a) {
   using F = GroupFFT<NG>;
   constexpr int R = F::R, L = F::L, GPW = 64 / L;
@@ -464,14 +470,15 @@ __global__ void __launch_bounds__(512, NG == 16 ? 4 : 2) apply_kernel(ApplyArgs 
   const int wave_items =  // of its first group
       __builtin_amdgcn_readfirstlane((nitem - wave * GPW + ngrp - 1) / ngrp);
   lds_barrier();  // sW and sTw visible
-  // NG = 32 reads one of its two sets of twiddles where they are used (they would
-  // spill); read there at NG = 16, whose 122 registers hold both, they cost many
-  // passes 3 to 12 % (NG = 16, 140 k-points, 8 bands: 46.1 against 43.1 us)
+  // NG = 32 reads one of its two sets of twiddles where they are used (both fill the
+  // registers: 9.3 against 10.0 us at 16 k-points, 16 bands); read there at NG = 16,
+  // whose 122 registers hold both, they cost many passes 3 to 12 % (NG = 16, 140
+  // k-points, 8 bands: 46.1 against 43.1 us)
   F fft;
   fft.init_lds(sTw, l);
   auto fwd = [&](zd (&v)[R]) { fft.fwd(v, T, l); };
   auto inv = [&](zd (&v)[R]) {
-    if constexpr (NG == 32)
+    if constexpr (NG == 32 && !ONE)
       fft.inv_t(v, T, l, [&](int g0) { return fft.fw[g0]; },
                 [&](int i) { return sTw[NG + l * R + i]; });
     else
@@ -481,6 +488,9 @@ __global__ void __launch_bounds__(512, NG == 16 ? 4 : 2) apply_kernel(ApplyArgs 
   int it = 0;
   auto pass = [&](auto lastc) {
     constexpr bool last = decltype(lastc)::value;
+    if constexpr (ONE) {
+      if (it > 0) fetch_v(cq);
+    }
     if (balance) set_wave_priority(3 - (4 * it) / wave_items);
     zd uq[R], v[R];
     static_for<0, R>([&](auto mc) {
@@ -509,7 +519,7 @@ __global__ void __launch_bounds__(512, NG == 16 ? 4 : 2) apply_kernel(ApplyArgs 
       constexpr int j = decltype(jc)::value;
       v[j] = zscal(v[j], vtr[j]);
     });
-    if constexpr (!last) fetch_v(cq);
+    if constexpr (!last && !ONE) fetch_v(cq);
     inv(v);
     static_for<0, R>([&](auto mc) {
       constexpr int m = decltype(mc)::value;
@@ -519,8 +529,12 @@ __global__ void __launch_bounds__(512, NG == 16 ? 4 : 2) apply_kernel(ApplyArgs 
       acc[m].y = fma(v[m].y, uq[m].x, acc[m].y);
     });
   };
-  for (; it + 1 < wave_items; ++it) pass(std::false_type{});
-  if (grp + it * ngrp < nitem) pass(std::true_type{});
+  if constexpr (ONE) {
+    for (; grp + it * ngrp < nitem; ++it) pass(std::false_type{});
+  } else {
+    for (; it + 1 < wave_items; ++it) pass(std::false_type{});
+    if (grp + it * ngrp < nitem) pass(std::true_type{});
+  }
   if (balance) set_wave_priority(0);
 
   // field values of this launch: read only now, so that they do not hold back

@@ -115,3 +115,29 @@ def test_default_batch_waves(ng, nk, nb, ntraj, waves):
         out = B.download()
     for t in (0, ntraj - 1):
         assert rel(out[t], ref[0]) < 1e-12 and np.abs(e[t] - ref[1]).max() < 1e-10
+
+
+@pytest.mark.parametrize("nk,nb,nw", [(64, 3, 1), (64, 3, 2), (65, 4, 1), (191, 1, 1), (201, 1, 1)])
+def test_rows_of_one_wave(nk, nb, nw):
+    """NG=32: from 192 pairs a row of one wave runs a variant of its own; even and
+    odd numbers of passes, with groups that have no last pair, against single runs."""
+    ng, ntraj = 32, 3
+    a, z = A32
+    vion = T.ion_potential(ng, nk, a, [z], [1.0], [0.0])
+    us = [orbitals((ng, nk, nb, nb, a, z), t) for t in range(ntraj)]
+    A = 0.1 * np.random.default_rng(5).standard_normal((ntraj, 2))
+    ref = []
+    with T.TDHF(ng, nk, nb, nb, a, 0.004, vion) as G:
+        ref = [G.RT_calculation(u, A[t], A[t]) for t, u in enumerate(us)]
+    # one trajectory of few k-points besides: the largest one decides
+    v2 = T.ion_potential(ng, 2, a, [z], [1.0], [0.0])
+    u2 = orbitals((ng, 2, nb, nb, a, z), 9)
+    with T.Batch(ng, nb, nb, a, 0.004, [nk] * ntraj + [2], np.array([vion] * ntraj + [v2])) as B:
+        B.set_waves(nw)
+        B.upload(us + [u2])
+        F = np.concatenate([A, A[:1]])
+        e, _, j, _ = B.propagate(F, F)
+        out = B.download()
+    for t in range(ntraj):
+        assert rel(out[t], ref[t][0]) < 1e-12
+        assert np.abs(e[t] - ref[t][1]).max() < 1e-10 and rel(j[t], ref[t][3]) < 1e-8
