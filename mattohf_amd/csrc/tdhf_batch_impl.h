@@ -902,7 +902,11 @@ int tdhf_batch_create(const tdhf_params* p, int ntraj, const int* nk, const doub
   // NG = 16): where the fullest XCD has between five and eight rows per CU, they
   // fit with one wave each and take a second round with two (NG=32, 6 rows: 31.1
   // and 34.6 us; NG=64, 5.25: 28.8 and 31.3; but 4.5: 41.2 and 35.4, 5: 45.6 and
-  // 38.9, 8.75: 114 and 101; NG=16, 12: 37.2 and 39.3, 8: 21.1 and 18.7)
+  // 38.9, 8.75: 114 and 101; NG=16, 12: 37.2 and 39.3, 8: 21.1 and 18.7).  At
+  // NG=128 the 13 to 16 pairs of a row, one pass of four waves, are cheaper in two of
+  // two with the transforms of two waves once CUs share rows, pinned: 30
+  // trajectories of NK=7, NB=2 12.6 against 13.6 us (but NK=5, NB=2, three waves,
+  // 11.6 against 10.9; 18 of NK=10, NB=2, 20 pairs, 14.9 either way unpinned)
   std::array<int, 3> ct{};
   const bool cached = tune_lookup(tune_key(b), &ct);
   // (density matrices: 8 waves for the product launch, 4 where it has
@@ -911,14 +915,15 @@ int tdhf_batch_create(const tdhf_params* p, int ntraj, const int* nk, const doub
   // 22.3 -> 17.4; fewer trajectories than XCDs are not pinned to them,
   // NG=128, NK=128, NB=8: 4 trajectories 166 us per stage pinned, 101 not)
   const long rows = (long)p->nb * std::accumulate(nk, nk + ntraj, 0L), cus = device_cus();
+  const int fit = choose_nw(p->ng, *std::max_element(nk, nk + ntraj), p->nbocc);
+  const long two = p->ng == 128 && fit == 4 ? cus : 2 * cus;  // rows of up to four waves
   b->ngrid = 0;
   if ((rc = batch_set_schedule(
-           b, cached ? ct[1] : (b->kuse ? ntraj < 8 : rows <= 2 * cus) ? 2 : 0)))
+           b, cached ? ct[1] : (b->kuse ? ntraj < 8 : rows <= two) ? 2 : 0)))
     return bail(rc);
-  const int fit = choose_nw(p->ng, *std::max_element(nk, nk + ntraj), p->nbocc);
   const long full = p->ng == 16 ? 2 * cus : cus;
   const bool one = b->ngrid > 5 * full && b->ngrid <= 8 * full;
-  const int nwr = std::max((p->ng + 63) / 64, std::min(fit, rows <= 2 * cus         ? 4
+  const int nwr = std::max((p->ng + 63) / 64, std::min(fit, rows <= two             ? 4
                                                             : rows <= 4 * cus && !one ? 2
                                                                                       : 1));
   const bool enough = b->kuse && (batch_points(b) > 1 || (p->ng == 16 && batch_groups(b) >= cus));

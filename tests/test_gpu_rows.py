@@ -97,10 +97,12 @@ def test_default_batch_shape(ng, nb, nks, ntraj):
 
 
 # waves of the product launch (density matrices) or of a row, by the rows of the
-# fullest XCD: 5 per CU, 6, 9 (12 at NG = 16); 480 workgroups of matrices at NG = 16
+# fullest XCD: 5 per CU, 6, 9 (12 at NG = 16); 480 workgroups of matrices at NG = 16;
+# 14 pairs a row at NG = 128, on more rows than CUs and on as many
 @pytest.mark.parametrize("ng,nk,nb,ntraj,waves", [(64, 40, 4, 5, 2), (32, 48, 4, 4, 1),
                                                   (32, 140, 2, 2, 2), (16, 96, 4, 2, 1),
-                                                  (16, 21, 6, 30, 4)])
+                                                  (16, 21, 6, 30, 4), (128, 7, 2, 19, 2),
+                                                  (128, 7, 2, 18, 4)])
 def test_default_batch_waves(ng, nk, nb, ntraj, waves):
     a, z = {16: A16, 32: A32, 64: A64, 128: A128}[ng]
     vion = T.ion_potential(ng, nk, a, [z], [1.0], [0.0])
