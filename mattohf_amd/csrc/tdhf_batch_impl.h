@@ -856,7 +856,7 @@ int tdhf_batch_create(const tdhf_params* p, int ntraj, const int* nk, const doub
     if (it == idx.end()) {
       q.nk = nk[t];
       tdhf_ctx* c = nullptr;
-      int rc = tdhf_create(&q, vion + (size_t)p->ng * t, nullptr, nullptr, &c);
+      int rc = create_ctx(&q, vion + (size_t)p->ng * t, nullptr, nullptr, true, &c);
       if (rc) {
         b->err = g_err;
         return bail(rc);

@@ -129,3 +129,23 @@ def test_observables_slots_of_row_wise_runs():
         B.upload([orbitals((ng, nk, 1, 1, a, 6.0), 1)] * ntraj)
         field = np.zeros((ntraj, nt))
         assert used(lambda: B.propagate(field, field)) < 200e6
+
+
+def test_tables_of_a_batch():
+    """Twelve k-meshes of NG=128: tables of 0.6 MB each beside the trajectories'
+    states (four of 2 MB each) and matrices (34 MB), 510 MB in all; with states and
+    matrices for runs of their own the tables alone would hold 970 MB more."""
+    ng, nb, a, nks = 128, 8, 12.0, list(range(117, 129))
+    vion = np.array([T.ion_potential(ng, k, a, [6.0], [1.0], [0.0]) for k in nks])
+    B = []
+    assert used(lambda: B.append(T.Batch(ng, nb, nb, a, 0.004, nks, vion))) < 700e6
+    us = [orbitals((ng, k, nb, nb, a, 6.0), k) for k in nks]
+    A = np.full((12, 2), 0.05)
+    B[0].upload(us)
+    e = B[0].propagate(A, A)[0]
+    out = B[0].download()
+    B[0].close()
+    for t in (0, 11):
+        with T.TDHF(ng, nks[t], nb, nb, a, 0.004, vion[t]) as G:
+            u, e1 = G.RT_calculation(us[t], A[t], A[t])[:2]
+        assert rel(out[t], u) < 1e-11 and rel(e[t], e1) < 1e-11
